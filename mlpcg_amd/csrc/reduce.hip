@@ -11,6 +11,7 @@
 //               exact hi/lo products for BF16 data, any C), else tiled through LDS with a
 //               3x4 register tile per thread.
 #include <mutex>
+#include <type_traits>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -19,114 +20,236 @@ namespace mlpcg {
 
 // ---------------------------------------------------------------------------
 // Mean patch.  A voxel u contributes to ybar[s,e] iff u - e is inside the grid, i.e.
-// per axis: e=-1 -> u <= n-2, e=0 -> always, e=+1 -> u >= 1.  Each thread sums a
-// z-run of VZ voxels once and spreads it over the 27 offsets with those masks.
+// per axis: e = -1 excludes the last cell, e = 0 none, e = +1 the first.  So the 27 sums
+// follow by inclusion and exclusion from T[a1][a2][a3], a in {all, first, last} per axis:
+// the total and the sums over the faces, edges and corners.  An interior row only adds to
+// T[0][0][.]; the rows of the faces take a branch, so the pass over the image is bound by
+// its loads (adding every run to 27 masked sums was VALU-bound).  All sums are FP64.  Each
+// sum of a workgroup leaves its wave by DPP adds: 27 C butterflies over __shfl_xor, an LDS
+// round trip per step, took 20 us on a grid of any size with C = 3.  Whole call, FP32,
+// before -> now: 256^3 C = 1 56 -> 25 us, C = 3 176 -> 56 us; 128^3 C = 3 151 -> 22 us;
+// below that the launches and their host side remain (C = 3, 16^3: 34 -> 20 us).
 // ---------------------------------------------------------------------------
-template <typename TI, int C, int VZ>
-__global__ __launch_bounds__(kThreads) void mean_patch_partial_kernel(const TI* __restrict__ img,
-                                                                      int n1, int n2, int n3,
-                                                                      double* __restrict__ partials) {
-  typedef typename AccOf<TI>::type A;
-  constexpr int NV = 27 * C;
-  A acc[NV];
-#pragma unroll
-  for (int o = 0; o < NV; ++o) acc[o] = A(0);
-  const long V = (long)n1 * n2 * n3;
-  const int n3c = n3 / VZ;
-  const long nch = (long)n1 * n2 * n3c;
-  for (long cid = (long)blockIdx.x * kThreads + threadIdx.x; cid < nch;
-       cid += (long)gridDim.x * kThreads) {
-    const int kc = (int)(cid % n3c);
-    const long t = cid / n3c;
-    const int j = (int)(t % n2), i = (int)(t / n2);
-    const int k0 = kc * VZ;
-    const long v0 = ((long)i * n2 + j) * n3 + k0;
-    const A m1[3] = {i <= n1 - 2 ? A(1) : A(0), A(1), i >= 1 ? A(1) : A(0)};
-    const A m2[3] = {j <= n2 - 2 ? A(1) : A(0), A(1), j >= 1 ? A(1) : A(0)};
-#pragma unroll
-    for (int s = 0; s < C; ++s) {
-      A v[VZ];
-      load_vec<VZ>(img + s * V + v0, v);
-      A cs = A(0);
-#pragma unroll
-      for (int u = 0; u < VZ; ++u) cs += v[u];
-      const A first = (k0 == 0) ? v[0] : A(0);
-      const A last = (k0 + VZ == n3) ? v[VZ - 1] : A(0);
-      const A s3[3] = {cs - last, cs, cs - first};
-#pragma unroll
-      for (int a1 = 0; a1 < 3; ++a1)
-#pragma unroll
-        for (int a2 = 0; a2 < 3; ++a2)
-#pragma unroll
-          for (int a3 = 0; a3 < 3; ++a3) acc[s * 27 + a1 * 9 + a2 * 3 + a3] += m1[a1] * m2[a2] * s3[a3];
-    }
-  }
-  __shared__ double sh[NV][4];
-  const int w = threadIdx.x >> 6;
-#pragma unroll
-  for (int o = 0; o < NV; ++o) {
-    const double s = wave_sum((double)acc[o]);
-    if ((threadIdx.x & 63) == 0) sh[o][w] = s;
-  }
-  __syncthreads();
-  for (int o = threadIdx.x; o < NV; o += kThreads)
-    partials[(size_t)blockIdx.x * NV + o] = sh[o][0] + sh[o][1] + sh[o][2] + sh[o][3];
+constexpr int kPatchBlocks = 512;       // workgroups of the partial sums at most (two per CU)
+constexpr long kPatchOneRuns = 1 << 12;  // grids of at most this many z-runs take one workgroup
+
+template <int C>
+struct PatchSums {
+  double t[C][27];
+};
+
+// sum over the wave by DPP row shifts and row broadcasts; valid in lane 63
+__device__ __forceinline__ double wave_sum_dpp(double v) {
+  auto step = [](double x, auto ctrl, auto rows) {
+    constexpr int kCtrl = decltype(ctrl)::value, kRows = decltype(rows)::value;
+    const long long u = __builtin_bit_cast(long long, x);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)u, kCtrl, kRows, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), kCtrl, kRows, 0xf, false);
+    return x + __builtin_bit_cast(double, ((long long)(unsigned)hi << 32) | (unsigned)lo);
+  };
+  typedef std::integral_constant<int, 0xf> All;
+  v = step(v, std::integral_constant<int, 0x111>(), All());  // row_shr 1, 2, 4, 8
+  v = step(v, std::integral_constant<int, 0x112>(), All());
+  v = step(v, std::integral_constant<int, 0x114>(), All());
+  v = step(v, std::integral_constant<int, 0x118>(), All());
+  v = step(v, std::integral_constant<int, 0x142>(), std::integral_constant<int, 0xa>());  // row_bcast 15
+  v = step(v, std::integral_constant<int, 0x143>(), std::integral_constant<int, 0xc>());  // row_bcast 31
+  return v;
 }
 
-// ybar = (sum of the block partials) / V, then z0 = w0 . ybar + b0 and, if w1 is given,
-// z1 = w1 . ybar + b1: c0 and c1 of one level share their mean patch (sm_model_3d.py:236-239
-// evaluates both on the same image), so one reduction serves both.  One wave per output
-// (lanes strided over the partials, a wave sum), all outputs in flight at once.
+template <typename TI, int C, int VZ>
+__device__ __forceinline__ void patch_accumulate(const TI* __restrict__ img, int n1, int n2, int n3, unsigned first,
+                                                 unsigned stride, PatchSums<C>& p) {
+#pragma unroll
+  for (int s = 0; s < C; ++s)
+#pragma unroll
+    for (int o = 0; o < 27; ++o) p.t[s][o] = 0.0;
+  const long V = (long)n1 * n2 * n3;
+  const unsigned n3c = (unsigned)(n3 / VZ), nch = (unsigned)n1 * (unsigned)n2 * n3c;
+  for (unsigned cid = first; cid < nch; cid += stride) {
+    const unsigned row = cid / n3c, kc = cid - row * n3c;
+    const unsigned i = row / (unsigned)n2, j = row - i * (unsigned)n2;
+    const bool zf = kc == 0, zl = kc == n3c - 1;
+    const bool edge = i == 0 || (int)i == n1 - 1 || j == 0 || (int)j == n2 - 1;
+#pragma unroll
+    for (int s = 0; s < C; ++s) {
+      typedef typename AccOf<TI>::type A;
+      A v[VZ];
+      load_vec<VZ>(img + s * V + (long)cid * VZ, v);
+      double cs = (double)v[0];
+#pragma unroll
+      for (int u = 1; u < VZ; ++u) cs += (double)v[u];
+      const double t3[3] = {cs, zf ? (double)v[0] : 0.0, zl ? (double)v[VZ - 1] : 0.0};
+      auto add = [&](int a1, int a2) {
+#pragma unroll
+        for (int u = 0; u < 3; ++u) p.t[s][9 * a1 + 3 * a2 + u] += t3[u];
+      };
+      add(0, 0);
+      if (edge) {
+        const bool i0 = i == 0, i1 = (int)i == n1 - 1;
+        if (i0) add(1, 0);
+        if (i1) add(2, 0);
+        if (j == 0) {
+          add(0, 1);
+          if (i0) add(1, 1);
+          if (i1) add(2, 1);
+        }
+        if ((int)j == n2 - 1) {
+          add(0, 2);
+          if (i0) add(1, 2);
+          if (i1) add(2, 2);
+        }
+      }
+    }
+  }
+}
+
+// ybar = (inclusion-exclusion of the 27 C sums in T) / V, then z0 = w0 . ybar + b0 and, if
+// w1 is given, z1 = w1 . ybar + b1: c0 and c1 of one level share their mean patch
+// (sm_model_3d.py:236-239 evaluates both on the same image), so one reduction serves both.
+// Run by threads 0 .. 127 of the workgroup that holds T in LDS; red: 4 doubles of LDS.
 template <typename A>
-__global__ __launch_bounds__(kThreads) void mean_patch_final_kernel(
+__device__ __forceinline__ void patch_finish(const double* T, double* red, int NV, double invV,
+                                             const A* __restrict__ w0, const A* __restrict__ b0, A* __restrict__ z0,
+                                             const A* __restrict__ w1, const A* __restrict__ b1, A* __restrict__ z1,
+                                             A* __restrict__ ybar) {
+  const int o = threadIdx.x;
+  double c0 = 0.0, c1 = 0.0;
+  if (o < NV) {
+    const double* t = T + (o / 27) * 27;
+    const int e = o % 27;
+    // per axis: the sums over all cells, less those over the cell that the offset drops
+    const int d1 = e / 9 == 1 ? 0 : (e / 9 == 0 ? 2 : 1), d2 = (e / 3) % 3 == 1 ? 0 : ((e / 3) % 3 == 0 ? 2 : 1);
+    const int d3 = e % 3 == 1 ? 0 : (e % 3 == 0 ? 2 : 1);
+    double s = 0.0;
+    for (int m = 0; m < 8; ++m) {
+      if (((m & 1) && !d1) || ((m & 2) && !d2) || ((m & 4) && !d3)) continue;
+      const double v = t[9 * ((m & 1) ? d1 : 0) + 3 * ((m & 2) ? d2 : 0) + ((m & 4) ? d3 : 0)];
+      s += (__popc(m) & 1) ? -v : v;
+    }
+    const A yb = (A)(s * invV);
+    ybar[o] = yb;
+    c0 = (double)w0[o] * (double)yb;
+    if (w1) c1 = (double)w1[o] * (double)yb;
+  }
+  c0 = wave_sum_dpp(c0);
+  c1 = wave_sum_dpp(c1);
+  if (o < 128 && (o & 63) == 63) {
+    red[2 * (o >> 6)] = c0;
+    red[2 * (o >> 6) + 1] = c1;
+  }
+  __syncthreads();
+  if (o == 0) {
+    z0[0] = (A)(red[0] + red[2] + (double)b0[0]);
+    if (w1) z1[0] = (A)(red[1] + red[3] + (double)b1[0]);
+  }
+}
+
+// Workgroup sums of the grid's runs; partials [27 C][gridDim.x].
+template <typename TI, int C, int VZ>
+__global__ __launch_bounds__(kThreads) void mean_patch_partial_kernel(const TI* __restrict__ img, int n1, int n2,
+                                                                      int n3, double* __restrict__ partials) {
+  PatchSums<C> p;
+  patch_accumulate<TI, C, VZ>(img, n1, n2, n3, blockIdx.x * kThreads + threadIdx.x, gridDim.x * kThreads, p);
+  __shared__ double sh[27 * C][4];
+  const int w = threadIdx.x >> 6;
+#pragma unroll
+  for (int o = 0; o < 27 * C; ++o) {
+    const double s = wave_sum_dpp(p.t[o / 27][o % 27]);
+    if ((threadIdx.x & 63) == 63) sh[o][w] = s;
+  }
+  __syncthreads();
+  for (int o = threadIdx.x; o < 27 * C; o += kThreads)
+    partials[(size_t)o * gridDim.x + blockIdx.x] = (sh[o][0] + sh[o][1]) + (sh[o][2] + sh[o][3]);
+}
+
+// One wave per sum (coalesced over the workgroups' partials, the loads of a sum in flight
+// together), then the patch and its products.
+constexpr int kPatchFinalThreads = 1024;
+template <typename A>
+__global__ __launch_bounds__(kPatchFinalThreads) void mean_patch_final_kernel(
     const double* __restrict__ partials, int nblk, int NV, double invV, const A* __restrict__ w0,
     const A* __restrict__ b0, A* __restrict__ z0, const A* __restrict__ w1, const A* __restrict__ b1,
     A* __restrict__ z1, A* __restrict__ ybar) {
-  __shared__ A ys[27 * 3];
+  __shared__ double T[27 * 3], red[4];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  for (int o = wv; o < NV; o += kThreads / 64) {
-    double s = 0.0;
-    for (int blk = lane; blk < nblk; blk += 64) s += partials[(size_t)blk * NV + o];
-    s = wave_sum(s);
-    const A yb = (A)(s * invV);
-    if (lane == 0) {
-      ys[o] = yb;
-      ybar[o] = yb;
+  for (int o = wv; o < NV; o += kPatchFinalThreads / 64) {
+    double a[kPatchBlocks / 64];
+#pragma unroll
+    for (int u = 0; u < kPatchBlocks / 64; ++u)
+      a[u] = lane + 64 * u < nblk ? partials[(size_t)o * nblk + lane + 64 * u] : 0.0;
+#pragma unroll
+    for (int u = 1; u < kPatchBlocks / 64; ++u) a[0] += a[u];
+    const double s = wave_sum_dpp(a[0]);
+    if (lane == 63) T[o] = s;
+  }
+  __syncthreads();
+  patch_finish<A>(T, red, NV, invV, w0, b0, z0, w1, b1, z1, ybar);
+}
+
+// Small grids: sums, patch and products in one workgroup (one launch instead of two).
+template <typename TI, int C, int VZ>
+__global__ __launch_bounds__(kPatchFinalThreads) void mean_patch_one_kernel(
+    const TI* __restrict__ img, int n1, int n2, int n3, double invV, const typename AccOf<TI>::type* __restrict__ w0,
+    const typename AccOf<TI>::type* __restrict__ b0, typename AccOf<TI>::type* __restrict__ z0,
+    const typename AccOf<TI>::type* __restrict__ w1, const typename AccOf<TI>::type* __restrict__ b1,
+    typename AccOf<TI>::type* __restrict__ z1, typename AccOf<TI>::type* __restrict__ ybar) {
+  typedef typename AccOf<TI>::type A;
+  constexpr int NW = kPatchFinalThreads / 64;
+  __shared__ double sh[27 * C][NW], T[27 * C], red[4];
+  const int w = threadIdx.x >> 6;
+#pragma unroll 1
+  for (int s = 0; s < C; ++s) {  // a channel at a time: 1024 threads leave 128 registers each
+    PatchSums<1> p;
+    patch_accumulate<TI, 1, VZ>(img + (long)s * n1 * n2 * n3, n1, n2, n3, threadIdx.x, kPatchFinalThreads, p);
+#pragma unroll
+    for (int o = 0; o < 27; ++o) {
+      const double v = wave_sum_dpp(p.t[0][o]);
+      if ((threadIdx.x & 63) == 63) sh[27 * s + o][w] = v;
     }
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    double c0 = 0.0, c1 = 0.0;
-    for (int o = 0; o < NV; ++o) {
-      c0 += (double)w0[o] * (double)ys[o];
-      if (w1) c1 += (double)w1[o] * (double)ys[o];
-    }
-    z0[0] = (A)(c0 + (double)b0[0]);
-    if (w1) z1[0] = (A)(c1 + (double)b1[0]);
+  for (int o = threadIdx.x; o < 27 * C; o += kPatchFinalThreads) {
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < NW; ++k) s += sh[o][k];
+    T[o] = s;
   }
+  __syncthreads();
+  patch_finish<A>(T, red, 27 * C, invV, w0, b0, z0, w1, b1, z1, ybar);
 }
+
+static int mean_patch_vz(int n3) { return (n3 % 4 == 0) ? 4 : (n3 % 2 == 0 ? 2 : 1); }
 
 static int mean_patch_blocks(int n1, int n2, int n3, int vz) {
   const long nch = (long)n1 * n2 * (n3 / vz);
   long nb = (nch + kThreads - 1) / kThreads;
-  if (nb > 1024) nb = 1024;
+  if (nb > kPatchBlocks) nb = kPatchBlocks;
   return (int)(nb < 1 ? 1 : nb);
 }
-
-static int mean_patch_vz(int n3) { return (n3 % 4 == 0) ? 4 : (n3 % 2 == 0 ? 2 : 1); }
 
 size_t mean_patch_workspace(int /*dtype*/, int C, int n1, int n2, int n3) {
   return (size_t)mean_patch_blocks(n1, n2, n3, mean_patch_vz(n3)) * 27 * C * sizeof(double);
 }
 
 template <typename TI>
-static void launch_mp_t(const void* img, double* part, int nblk, int C, int n1, int n2, int n3, int vz,
-                        hipStream_t st) {
-#define MLPCG_MP(CC, VZZ)                                                                         \
-  if (C == CC && vz == VZZ) {                                                                     \
-    mean_patch_partial_kernel<TI, CC, VZZ><<<nblk, kThreads, 0, st>>>((const TI*)img, n1, n2, n3, \
-                                                                      part);                      \
-    return;                                                                                       \
+static void launch_mp_t(const void* img, double* part, int nblk, bool one, double invV, const void* w0,
+                        const void* b0, void* z0, const void* w1, const void* b1, void* z1, void* ybar, int C, int n1,
+                        int n2, int n3, int vz, hipStream_t st) {
+  typedef typename AccOf<TI>::type A;
+#define MLPCG_MP(CC, VZZ)                                                                                        \
+  if (C == CC && vz == VZZ) {                                                                                    \
+    if (one) {                                                                                                   \
+      mean_patch_one_kernel<TI, CC, VZZ><<<1, kPatchFinalThreads, 0, st>>>(                                      \
+          (const TI*)img, n1, n2, n3, invV, (const A*)w0, (const A*)b0, (A*)z0, (const A*)w1, (const A*)b1, (A*)z1, \
+          (A*)ybar);                                                                                             \
+    } else {                                                                                                     \
+      mean_patch_partial_kernel<TI, CC, VZZ><<<nblk, kThreads, 0, st>>>((const TI*)img, n1, n2, n3, part);       \
+      mean_patch_final_kernel<A><<<1, kPatchFinalThreads, 0, st>>>(part, nblk, 27 * C, invV, (const A*)w0,       \
+                                                                   (const A*)b0, (A*)z0, (const A*)w1,           \
+                                                                   (const A*)b1, (A*)z1, (A*)ybar);              \
+    }                                                                                                            \
+    return;                                                                                                      \
   }
   MLPCG_MP(1, 4) MLPCG_MP(1, 2) MLPCG_MP(1, 1)
   MLPCG_MP(2, 4) MLPCG_MP(2, 2) MLPCG_MP(2, 1)
@@ -143,21 +266,16 @@ int launch_sm_linear_pair(int dtype, const void* img, const void* w0, const void
   const int nblk = mean_patch_blocks(n1, n2, n3, vz);
   double* part = (double*)workspace;
   const double invV = 1.0 / ((double)n1 * n2 * n3);
+  const bool one = (long)n1 * n2 * (n3 / vz) <= kPatchOneRuns;
+#define MLPCG_MPT(T) launch_mp_t<T>(img, part, nblk, one, invV, w0, b0, z0, w1, b1, z1, ybar, C, n1, n2, n3, vz, st)
   switch (dtype) {
-    case kF64: launch_mp_t<double>(img, part, nblk, C, n1, n2, n3, vz, st); break;
-    case kF32: launch_mp_t<float>(img, part, nblk, C, n1, n2, n3, vz, st); break;
-    case kF16: launch_mp_t<f16>(img, part, nblk, C, n1, n2, n3, vz, st); break;
-    case kBF16: launch_mp_t<bf16>(img, part, nblk, C, n1, n2, n3, vz, st); break;
+    case kF64: MLPCG_MPT(double); break;
+    case kF32: MLPCG_MPT(float); break;
+    case kF16: MLPCG_MPT(f16); break;
+    case kBF16: MLPCG_MPT(bf16); break;
     default: MLPCG_REQUIRE(false, "sm_linear: bad dtype %d", dtype);
   }
-  if (dtype == kF64)
-    mean_patch_final_kernel<double><<<1, kThreads, 0, st>>>(
-        part, nblk, 27 * C, invV, (const double*)w0, (const double*)b0, (double*)z0, (const double*)w1,
-        (const double*)b1, (double*)z1, (double*)ybar);
-  else
-    mean_patch_final_kernel<float><<<1, kThreads, 0, st>>>(
-        part, nblk, 27 * C, invV, (const float*)w0, (const float*)b0, (float*)z0, (const float*)w1,
-        (const float*)b1, (float*)z1, (float*)ybar);
+#undef MLPCG_MPT
   return check_launch("sm_linear");
 }
 
@@ -170,7 +288,7 @@ int launch_sm_linear(int dtype, const void* img, const void* w, const void* b, v
 // ---------------------------------------------------------------------------
 // SM linear without allocation.  The block partials of the mean patch go to a file-scope
 // device array instead of a caller workspace: at most 1024 blocks x 27 C doubles
-// (648 KiB for C = 3) for ANY grid, since the partial kernel caps its block count.
+// (648 KiB for C = 3) for ANY grid, since the partial kernel caps its block count (at half of that).
 // Each GPU holds its own copy of the array until the process ends; host code never
 // passes the array's name to a kernel (in host code it names a host-side stand-in) but
 // the device address that hipGetSymbolAddress returned, fetched once per device with
