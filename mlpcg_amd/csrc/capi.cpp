@@ -34,6 +34,10 @@ static bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 // apply (as the BF16 plans do); smaller grids stream stored stencils.
 constexpr size_t kFusedForwardMinVoxels = (size_t)1 << 18;
 
+// FP32 block forwards on grids of at least this many voxels recompute K on the matrix cores
+// (split.hpp) instead of storing it.
+constexpr size_t kSplitMinVoxels = (size_t)1 << 14;
+
 }  // namespace mlpcg
 
 using namespace mlpcg;
@@ -104,6 +108,20 @@ static int block_fwd(bool trans, const void* image, const void* x, const void* w
     f.n2 = n2;
     f.n3 = n3;
     return launch_sm_fused(kBF16, kBF16, kBF16, C, f, STREAM(stream));
+  }
+  if (!trans && dtype == kF32 && V >= kSplitMinVoxels && split_eligible(C, n1, n2, n3)) {
+    if (launch_split_pack(weight, bias, C, workspace, STREAM(stream))) return -1;
+    SplitArgs f;
+    memset(&f, 0, sizeof(f));
+    f.img = (const float*)image;
+    f.pack = workspace;
+    f.x = (const float*)x;
+    f.y = (float*)y;
+    f.B = B;
+    f.n1 = n1;
+    f.n2 = n2;
+    f.n3 = n3;
+    return launch_sm_split(C, f, STREAM(stream));
   }
   if (launch_stencil_weights(dtype, image, weight, bias, workspace, C, n1, n2, n3, trans, STREAM(stream)))
     return -1;

@@ -79,6 +79,35 @@ int launch_fused_kwrite(int C, const FusedArgs& a, void* K, hipStream_t st);
 size_t fused_sgrad_bytes(int n1, int n2, int n3);
 int launch_fused_sgrad(int C, const FusedArgs& a, void* work, void* dx, hipStream_t st);
 
+// FP32 blocks on the matrix cores (split.hpp): K recomputed from the FP32 image img [C][V]
+// and the packed weights (launch_split_pack), applied to x [B][V] with the epilogue of
+// ApplyArgs; any grid whose planes are under 2^31 bytes (split_eligible).
+struct SplitArgs {
+  const float* img;
+  const void* pack;
+  const float* x;
+  float* y;
+  const float* prev;
+  const float* c0;
+  const float* c1;
+  const uint8_t* mask_a;
+  const uint8_t* mask_b;
+  const double* in_scale;
+  const int* done;
+  // optional, B = 1: partial sums [2][split_blocks()] of y.dot0 and y.dot1 (dot1 may be null)
+  const float* dot0;
+  const float* dot1;
+  double* partials;
+  // optional (B = 1, even grid, no epilogue operands): the 2x2x2 means of y, as avgpool2's
+  float* pool_out;
+  int B, n1, n2, n3;
+};
+size_t split_pack_bytes(int C);
+bool split_eligible(int C, int n1, int n2, int n3);
+unsigned split_blocks(int C, int n1, int n2, int n3);
+int launch_split_pack(const void* W, const void* b, int C, void* pack, hipStream_t st);
+int launch_sm_split(int C, const SplitArgs& a, hipStream_t st);
+
 // The two coarsest levels of the SmallSM V-cycle in one workgroup (tail.hip): from the
 // output x_in of pre[n-2] (level n-2 grid) to up(c0 x + c1 post[n-1](up(l(pool(x))))) on
 // the level n-2 grid.  f1..f3: level n-1 dims (even; at most kTailMaxFine voxels, and the

@@ -1,6 +1,7 @@
 // Small helper kernels of the native runtime.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "split.hpp"
 
 namespace mlpcg {
 

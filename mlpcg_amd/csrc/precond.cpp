@@ -32,6 +32,10 @@ static size_t dsize(int dt) {
 // per-level kernels it replaces.
 constexpr long kFusedMinVoxels = 1L << 18;
 
+// FP32 blocks recompute K (split.hpp) on grids above this many voxels.  A 64^3 level's
+// stencils (28 MB) stay in the caches and their apply takes 7.4 us; at 96^3 they no longer do.
+constexpr long kSplitMinVoxels = 1L << 18;
+
 // plan generation ids: never reused within a process, unlike plan addresses
 static std::atomic<unsigned long> g_next_gen{1};
 
@@ -103,23 +107,23 @@ int precond_create(Precond** out, int kind, int n, int C, int n1, int n2, int n3
   }
   // stencils: (weight index, level, transposed)
   if (kind == kSmallSM) {
-    for (int i = 0; i < n; ++i) P->blocks.push_back({i, i, 0, 0});       // pre
-    for (int i = 0; i < n; ++i) P->blocks.push_back({n + i, i, 0, 0});   // post
-    P->blocks.push_back({2 * n, n, 0, 0});                               // l
+    for (int i = 0; i < n; ++i) P->blocks.push_back({i, i, 0, 0, 0});       // pre
+    for (int i = 0; i < n; ++i) P->blocks.push_back({n + i, i, 0, 0, 0});   // post
+    P->blocks.push_back({2 * n, n, 0, 0, 0});                               // l
     P->nw = 2 * n + 1;
   } else if (kind == kSPD) {
-    for (int i = 0; i < n; ++i) P->blocks.push_back({i, i, 0, 0});       // l0
-    for (int i = 0; i < n; ++i) P->blocks.push_back({n + i, i, 0, 0});   // l1
-    P->blocks.push_back({2 * n, n, 0, 0});                               // l
-    for (int i = 0; i < n; ++i) P->blocks.push_back({n + i, i, 1, 0});   // l1_t
-    for (int i = 0; i < n; ++i) P->blocks.push_back({i, i, 1, 0});       // l0_t
-    P->blocks.push_back({2 * n, n, 1, 0});                               // l_t
+    for (int i = 0; i < n; ++i) P->blocks.push_back({i, i, 0, 0, 0});       // l0
+    for (int i = 0; i < n; ++i) P->blocks.push_back({n + i, i, 0, 0, 0});   // l1
+    P->blocks.push_back({2 * n, n, 0, 0, 0});                               // l
+    for (int i = 0; i < n; ++i) P->blocks.push_back({n + i, i, 1, 0, 0});   // l1_t
+    for (int i = 0; i < n; ++i) P->blocks.push_back({i, i, 1, 0, 0});       // l0_t
+    P->blocks.push_back({2 * n, n, 1, 0, 0});                               // l_t
     P->nw = 2 * n + 1;
   } else {
-    for (int i = 0; i < n; ++i) P->blocks.push_back({i, i, 0, 0});       // l0
-    P->blocks.push_back({n, n, 0, 0});                                   // l
-    for (int i = 0; i < n; ++i) P->blocks.push_back({i, i, 1, 0});       // l0_t
-    P->blocks.push_back({n, n, 1, 0});                                   // l_t
+    for (int i = 0; i < n; ++i) P->blocks.push_back({i, i, 0, 0, 0});       // l0
+    P->blocks.push_back({n, n, 0, 0, 0});                                   // l
+    for (int i = 0; i < n; ++i) P->blocks.push_back({i, i, 1, 0, 0});       // l0_t
+    P->blocks.push_back({n, n, 1, 0, 0});                                   // l_t
     P->nw = n + 1;
   }
   const bool half = (dtype == kBF16);
@@ -130,7 +134,13 @@ int precond_create(Precond** out, int kind, int n, int C, int n1, int n2, int n3
     void* wp = nullptr;
     const bool big = P->V[b.level] >= kFusedMinVoxels || fused_mode == 2;
     b.fused = (half && !b.trans && fused_mode && big && fused_eligible(P->cf, 1, d[0], d[1], d[2])) ? 1 : 0;
-    if (b.fused) {
+    b.split = (dtype == kF32 && !b.trans && fused_mode && P->V[b.level] > kSplitMinVoxels &&
+               split_eligible(C, d[0], d[1], d[2]))
+                  ? 1
+                  : 0;
+    if (b.split) {
+      TRY(palloc(P, &wp, split_pack_bytes(C)));
+    } else if (b.fused) {
       TRY(palloc(P, &wp, fused_weights_bytes(P->cf)));
       if (!P->imgw[b.level]) TRY(palloc(P, &P->imgw[b.level], (size_t)P->cf * P->V[b.level] * es));
     } else {
@@ -177,7 +187,9 @@ int Precond::update(const void* image, const void* const* weights, const void* c
   for (size_t k = 0; k < blocks.size(); ++k) {
     const Blk& b = blocks[k];
     const int* d = dims[b.level];
-    if (b.fused)
+    if (b.split)
+      TRY(launch_split_pack(weights[b.w], biases[b.w], C, wpack[k], st));
+    else if (b.fused)
       TRY(launch_fused_pack(dtype, weights[b.w], biases[b.w], C, wpack[k], st, cf < C));
     else
       TRY(launch_stencil_weights2(acc, dtype, img[b.level], weights[b.w], biases[b.w], K[k], C, d[0],
@@ -198,7 +210,7 @@ int Precond::update(const void* image, const void* const* weights, const void* c
   return 0;
 }
 
-// One stencil block: the fused matrix-core kernel or the stored-stencil apply, with the
+// One stencil block: a matrix-core kernel or the stored-stencil apply, with the
 // level-combine / mask epilogue of ApplyArgs.
 int Precond::run_block(int k, int level, const void* x, int tx, void* y, int ty, const void* prev,
                        const void* c0, const void* c1, const uint8_t* ma, const uint8_t* mb,
@@ -225,6 +237,29 @@ int Precond::run_block(int k, int level, const void* x, int tx, void* y, int ty,
     f.n2 = dims[level][1];
     f.n3 = dims[level][2];
     return launch_sm_fused(dtype, tx, ty, cf, f, st);
+  }
+  if (blocks[k].split) {
+    SplitArgs f;
+    f.img = (const float*)img[level];
+    f.pack = wpack[k];
+    f.x = (const float*)x;
+    f.y = (float*)y;
+    f.prev = (const float*)prev;
+    f.c0 = (const float*)c0;
+    f.c1 = (const float*)c1;
+    f.mask_a = ma;
+    f.mask_b = mb;
+    f.in_scale = sc;
+    f.done = done;
+    f.dot0 = dot0;
+    f.dot1 = dot1;
+    f.partials = partials;
+    f.pool_out = (float*)pool_out;
+    f.B = 1;
+    f.n1 = dims[level][0];
+    f.n2 = dims[level][1];
+    f.n3 = dims[level][2];
+    return launch_sm_split(C, f, st);
   }
   ApplyArgs a;
   a.K = K[k];
@@ -299,11 +334,11 @@ int Precond::apply(const float* r_in, float* z_out, const double* in_scale, cons
   // ---- downward half (identical for every kind): x_0 = B0(r), x_i = Bi(pool x_{i-1}) ----
   const int ndown = tail ? n - 1 : n;  // with the tail, levels n-1 and n run in one kernel
   // x_i is pooled into tmp[i+1] for the next block (the tail pools its input itself); a
-  // fused block without epilogue operands (not level 0 under the model mask) writes that
+  // matrix-core block without epilogue operands (not level 0 under the model mask) writes that
   // mean in its epilogue, so the pool kernel is left out
   auto pool_into = [&](int i) -> void* {
     const bool pooled = (i + 1 < ndown) || (!tail && i == n - 1);
-    return (pooled && blocks[i].fused && !(i == 0 && mask)) ? tmp[i + 1] : nullptr;
+    return (pooled && (blocks[i].fused || blocks[i].split) && !(i == 0 && mask)) ? tmp[i + 1] : nullptr;
   };
   TRY(run_block(0, 0, r_in, vdt, xd[0], dtype, nullptr, nullptr, nullptr, mask ? maskimg : nullptr, nullptr,
                 in_scale, done, st, nullptr, nullptr, nullptr, pool_into(0)));
@@ -344,12 +379,15 @@ int Precond::apply(const float* r_in, float* z_out, const double* in_scale, cons
       const uint8_t* mb = last ? out_mask : nullptr;
       if (!swap) {
         if (!(tail && i == n - 1)) TRY(up(cur, tmp[lvl], lvl, 1.0, nullptr, nullptr, nullptr));
-        if (last && dot0 && partials && dot_blocks && blocks[n].fused &&
-            2L * fused_blocks(cf, dims[0][0], dims[0][1], dims[0][2]) <= reduction_capacity()) {
+        const unsigned nb = !last ? 0
+                            : blocks[n].fused ? fused_blocks(cf, dims[0][0], dims[0][1], dims[0][2])
+                            : blocks[n].split ? split_blocks(C, dims[0][0], dims[0][1], dims[0][2])
+                                              : 0;
+        if (nb && dot0 && partials && dot_blocks && 2L * nb <= reduction_capacity()) {
           // the solver's dot products on z ride in the epilogue of the last block
           TRY(run_block(n, 0, tmp[0], dtype, y, ty, xd[0], c0p(0, 0), c1p(0, 0), ma, mb, nullptr, done, st,
                         dot0, dot1, partials));
-          *dot_blocks = fused_blocks(cf, dims[0][0], dims[0][1], dims[0][2]);
+          *dot_blocks = nb;
           cur = xo[lvl];
           continue;
         }

@@ -14,9 +14,10 @@ enum ModelKind : int { kSmallSM = 0, kSPD = 1, kSmallSPD = 2 };
 
 // Everything that depends only on the image is computed once at creation: the image
 // pyramid (accumulate precision), the stencil weights K of every block (storage
-// precision, [27][V_level]) and the SMLinear coefficients c0/c1 (device scalars).  For
-// 16-bit plans, blocks on grids the fused kernel tiles keep no K: they hold the weights
-// packed for the matrix cores and a 16-bit copy of their level's image instead.
+// precision, [27][V_level]) and the SMLinear coefficients c0/c1 (device scalars).  BF16
+// blocks on grids the fused kernel tiles keep no K: they hold the weights packed for the
+// matrix cores and a 16-bit copy of their level's image instead; FP32 blocks on large grids
+// keep no K either (packed weights, and the FP32 image as it is).
 // This is the caching that SmallSMModelDn3D.eval_forward does for imgs/c0/c1 through
 // its list arguments (sm_model_3d.py:180-195), extended to K.
 struct Precond {
@@ -36,10 +37,11 @@ struct Precond {
   uint8_t* maskimg = nullptr;       // level-0 model mask: img[1] != 0
   struct Blk {
     int w, level, trans;            // weight index, level, transposed stencil
-    int fused;                      // 1: K recomputed on the matrix cores (no K stored)
+    int fused;                      // 1: K recomputed on the matrix cores (no K stored), BF16
+    int split;                      // 1: the same for FP32, by split FP16 operands
   };
-  std::vector<Blk> blocks;          // one per entry of K (nullptr for fused blocks)
-  std::vector<void*> wpack;         // fused blocks: packed MFMA weights + bias init
+  std::vector<Blk> blocks;          // one per entry of K (nullptr for fused and split blocks)
+  std::vector<void*> wpack;         // fused and split blocks: packed MFMA weights and bias
   void* imgw[kMaxLevels + 1] = {};  // FP16 image of levels with fused blocks (cf channels)
   int cf = 1;                       // image channels of the fused blocks: C, or 2 when the
                                     // third channel is folded into the first two
@@ -70,7 +72,8 @@ struct Precond {
 
 // Per-plan policies.  fused_mode: eligible BF16 blocks recompute their stencils on the
 // matrix cores inside the apply -- 0 never, 1 (default) on grids of at least
-// kFusedMinVoxels voxels, 2 on every eligible grid; plus kFuseFoldThird: for three-channel
+// kFusedMinVoxels voxels, 2 on every eligible grid; FP32 blocks with mode 1 or 2 on grids
+// above kSplitMinVoxels; plus kFuseFoldThird: for three-channel
 // images whose third channel is the sum of the first two (the [air, fluid, non-solid]
 // images), the fused blocks take two channels with the third channel's weights added to
 // the others' (the caller vouches for the relation).  coarse_tail: the two coarsest SmallSM
