@@ -45,7 +45,8 @@ def hipcc() -> str:
 # copies in its inner loop), and its LDS reads stay 16-bit: without unaligned-access-mode
 # the compiler does not merge two neighbouring 16-bit reads at an odd element into one
 # misaligned 32-bit read, which measured 5x slower on gfx950
-# (misc.hip holds the FP32 matrix-core block, split.hpp, with the same needs)
+# (misc.hip holds the FP32 matrix-core block, split.hpp, and the weight gradient, wgrad.hpp,
+# with the same needs)
 MATRIX = ["-mllvm", "-amdgpu-mfma-vgpr-form", "-Xclang", "-target-feature", "-Xclang", "-unaligned-access-mode"]
 EXTRA = {"fused.hip": MATRIX, "misc.hip": MATRIX}
 

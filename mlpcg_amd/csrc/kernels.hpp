@@ -165,6 +165,12 @@ size_t weight_grad_workspace(int dtype, int C, int B, int n1, int n2, int n3);
 int launch_weight_grad(int dtype, const void* a, const void* c, const void* img, void* gW, void* gb,
                        void* workspace, int C, int B, int n1, int n2, int n3, hipStream_t st);
 
+// The partial sums of it on the matrix cores (wgrad.hpp), FP32, BF16 or FP16 values:
+// part[nblk][27][27 C + 1] with nblk = wgrad_blocks(most, ..) <= most.
+int wgrad_blocks(int most, int n1, int n2, int n3);
+int launch_wgrad(int dtype, const void* a, const void* c, const void* img, float* part, int nblk, int C, int B, int n1,
+                 int n2, int n3, hipStream_t st);
+
 int launch_linear_backward(int dtype, const void* g, const void* ybar, void* gw, void* gb, int C,
                            hipStream_t st);
 

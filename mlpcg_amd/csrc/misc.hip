@@ -2,6 +2,7 @@
 #include "common.hpp"
 #include "kernels.hpp"
 #include "split.hpp"
+#include "wgrad.hpp"
 
 namespace mlpcg {
 

@@ -7,9 +7,8 @@
 //   weight grad G_p(v) = sum_b a[b,v] c[b,v+d_p]              sm_block_3d_kernel.cu:121-229
 //               gW[p,s,e] = sum_v G_p(v) img[s,v+e], gb[p] = sum_v G_p(v)
 //               i.e. the [27 x V] . [V x (27C+1)] product of per-voxel outer products:
-//               on the matrix cores (FP32 operands for one channel; BF16 operands with
-//               exact hi/lo products for BF16 data, any C), else tiled through LDS with a
-//               3x4 register tile per thread.
+//               on the matrix cores (wgrad.hpp; BF16 segments of 64 cells by the kernel here),
+//               FP64 tiled through LDS with a 3x4 register tile per thread.
 #include <mutex>
 #include <type_traits>
 
@@ -472,185 +471,6 @@ __global__ __launch_bounds__(kThreads) void weight_grad_partial_kernel(
   }
 }
 
-// One-channel weight gradient on the matrix cores (FP32 MFMA, so FP32 products and sums
-// as in the VALU kernel above): gW[p][q] = sum_v G_p(v) P_q(v) with P_q the 27 image taps
-// and the bias column (P_27 = 1), a 32 x 32 (padded) product over the voxels.  A wave
-// walks one z-row segment of up to 64 voxels, 4 voxels per v_mfma_f32_16x16x4_f32
-// (A[i][k]: lane 16k + i; B[k][j]: lane 16k + j; D[4(l/16)+t][l%16]): lane (k, i) feeds
-// G and P for taps i and 16 + i of voxel k.  Its neighbour offsets are constants and the
-// validity of its two neighbour rows is fixed per segment, so only the z ends need a
-// check.  Waves of a block add their 32 x 32 tiles in LDS in a fixed order; the block's
-// 27 x 28 sums go to partials[block] like the VALU kernel's.
-typedef float wg_f32x4 __attribute__((ext_vector_type(4)));
-
-template <typename TX, typename TI>
-__global__ __launch_bounds__(kThreads) void weight_grad_mfma_kernel(
-    const TX* __restrict__ a, const TX* __restrict__ cv, int B, const TI* __restrict__ img, int n1,
-    int n2, int n3, float* __restrict__ partials) {
-  constexpr int NQ = 28, NO = 27 * NQ;
-  __shared__ float red[4][32 * 32];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int kq = lane >> 4, il = lane & 15;
-  const long V = (long)n1 * n2 * n3;
-  const long s1 = (long)n2 * n3;
-  // voxels per segment: the largest of 64, 32, 16, 8, 4 that divides n3 (n3 % 4 == 0)
-  const int seg = n3 % 64 == 0 ? 64 : (n3 % 32 == 0 ? 32 : (n3 % 16 == 0 ? 16 : (n3 % 8 == 0 ? 8 : 4)));
-  const int nseg3 = n3 / seg;
-  const long nseg = (long)n1 * n2 * nseg3;
-  // this lane's two taps (rows of G, columns of P): t = il and 16 + il
-  int d1[2], d2[2], d3[2];
-  bool gok[2], pimg[2], pone[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int t = 16 * h + il;
-    const int tt = t < 27 ? t : 0;
-    d1[h] = tt / 9 - 1;
-    d2[h] = (tt / 3) % 3 - 1;
-    d3[h] = tt % 3 - 1;
-    gok[h] = t < 27;
-    pimg[h] = t < 27;
-    pone[h] = t == 27;
-  }
-  wg_f32x4 acc[2][2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int g = 0; g < 2; ++g) acc[h][g] = wg_f32x4{0.f, 0.f, 0.f, 0.f};
-  for (long sg = (long)blockIdx.x * 4 + w; sg < nseg; sg += (long)gridDim.x * 4) {
-    const int zs = (int)(sg % nseg3) * seg;
-    const long rowid = sg / nseg3;
-    const int j = (int)(rowid % n2), i = (int)(rowid / n2);
-    const long vrow = rowid * n3;
-    bool rok[2];
-    long roff[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      rok[h] = (unsigned)(i + d1[h]) < (unsigned)n1 && (unsigned)(j + d2[h]) < (unsigned)n2;
-      roff[h] = (long)d1[h] * s1 + (long)d2[h] * n3 + d3[h];
-    }
-#pragma unroll 4
-    for (int z4 = 0; z4 < seg; z4 += 4) {
-      const int z = zs + z4 + kq;
-      const long v = vrow + z;
-      float gv[2] = {0.f, 0.f}, pv[2];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const bool ok = rok[h] && (unsigned)(z + d3[h]) < (unsigned)n3;
-        const long u = ok ? v + roff[h] : v;
-        float sacc = 0.f;
-        for (int b = 0; b < B; ++b) sacc += (float)a[(long)b * V + v] * (float)cv[(long)b * V + u];
-        gv[h] = (gok[h] && ok) ? sacc : 0.f;
-        const float iv = (float)img[u];
-        pv[h] = pone[h] ? 1.f : ((pimg[h] && ok) ? iv : 0.f);
-      }
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int g = 0; g < 2; ++g) acc[h][g] = __builtin_amdgcn_mfma_f32_16x16x4f32(gv[h], pv[g], acc[h][g], 0, 0, 0);
-    }
-  }
-  // D[16h + 4 kq + t][16g + il] of this wave -> LDS, then a fixed-order sum over the waves
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int g = 0; g < 2; ++g)
-#pragma unroll
-      for (int t = 0; t < 4; ++t) red[w][(16 * h + 4 * kq + t) * 32 + 16 * g + il] = acc[h][g][t];
-  __syncthreads();
-  for (int o = threadIdx.x; o < NO; o += kThreads) {
-    const int pp = o / NQ, qq = o % NQ;
-    const int e = pp * 32 + qq;
-    partials[(size_t)blockIdx.x * NO + o] = (red[0][e] + red[1][e]) + (red[2][e] + red[3][e]);
-  }
-}
-
-// B == 1 form of weight_grad_mfma_kernel with the neighbour rows staged in LDS: per
-// z-row segment (one per wave; the block's four waves run the same number of rounds, so
-// the barriers are uniform) the 9 neighbour rows of x and of the image over
-// [z0 - 1, z0 + seg] are loaded with coalesced row reads, zero outside the grid, and the
-// matrix-core loop reads G and P from LDS without bounds checks.
-template <typename TX, typename TI>
-__global__ __launch_bounds__(kThreads) void weight_grad_mfma_lds_kernel(
-    const TX* __restrict__ a, const TX* __restrict__ cv, const TI* __restrict__ img, int n1, int n2,
-    int n3, float* __restrict__ partials) {
-  constexpr int NQ = 28, NO = 27 * NQ, RL = 66;  // staged row length (seg <= 64, + halo)
-  __shared__ float xs[4][9 * RL], is[4][9 * RL], ac[4][64];
-  __shared__ float red[4][32 * 32];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int kq = lane >> 4, il = lane & 15;
-  const long s1 = (long)n2 * n3;
-  const int seg = n3 % 64 == 0 ? 64 : (n3 % 32 == 0 ? 32 : (n3 % 16 == 0 ? 16 : (n3 % 8 == 0 ? 8 : 4)));
-  const int nseg3 = n3 / seg;
-  const long nseg = (long)n1 * n2 * nseg3;
-  int rr[2], cz[2];  // this lane's taps t = il, 16 + il: staged row and z offset (t / 3, t % 3)
-  bool gok[2], pimg[2], pone[2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int t = 16 * h + il;
-    const int tt = t < 27 ? t : 0;
-    rr[h] = tt / 3;
-    cz[h] = tt % 3;
-    gok[h] = t < 27;
-    pimg[h] = t < 27;
-    pone[h] = t == 27;
-  }
-  wg_f32x4 acc[2][2];
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int g = 0; g < 2; ++g) acc[h][g] = wg_f32x4{0.f, 0.f, 0.f, 0.f};
-  for (long sg0 = (long)blockIdx.x * 4; sg0 < nseg; sg0 += (long)gridDim.x * 4) {
-    const long sg = sg0 + w;
-    const bool active = sg < nseg;  // uniform per wave
-    if (active) {
-      const int zs = (int)(sg % nseg3) * seg;
-      const long rowid = sg / nseg3;
-      const int j = (int)(rowid % n2), i = (int)(rowid / n2);
-      for (int e = lane; e < 9 * (seg + 2); e += 64) {
-        const int r = e / (seg + 2), cc = e - r * (seg + 2);
-        const int ii = i + r / 3 - 1, jj = j + r % 3 - 1, z = zs - 1 + cc;
-        const bool ok = (unsigned)ii < (unsigned)n1 && (unsigned)jj < (unsigned)n2 && (unsigned)z < (unsigned)n3;
-        const long u = ok ? (long)ii * s1 + (long)jj * n3 + z : 0;
-        xs[w][r * RL + cc] = ok ? (float)cv[u] : 0.f;
-        is[w][r * RL + cc] = ok ? (float)img[u] : 0.f;
-      }
-      for (int e = lane; e < seg; e += 64) ac[w][e] = (float)a[rowid * n3 + zs + e];
-    }
-    __syncthreads();
-    if (active) {
-      for (int z4 = 0; z4 < seg; z4 += 4) {
-        const int z = z4 + kq;
-        const float av = ac[w][z];
-        float gv[2], pv[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int cidx = rr[h] * RL + z + cz[h];
-          gv[h] = gok[h] ? av * xs[w][cidx] : 0.f;
-          pv[h] = pone[h] ? 1.f : (pimg[h] ? is[w][cidx] : 0.f);
-        }
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int g = 0; g < 2; ++g)
-            acc[h][g] = __builtin_amdgcn_mfma_f32_16x16x4f32(gv[h], pv[g], acc[h][g], 0, 0, 0);
-      }
-    }
-    __syncthreads();
-  }
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int g = 0; g < 2; ++g)
-#pragma unroll
-      for (int t = 0; t < 4; ++t) red[w][(16 * h + 4 * kq + t) * 32 + 16 * g + il] = acc[h][g][t];
-  __syncthreads();
-  for (int o = threadIdx.x; o < NO; o += kThreads) {
-    const int pp = o / NQ, qq = o % NQ;
-    const int e = pp * 32 + qq;
-    partials[(size_t)blockIdx.x * NO + o] = (red[0][e] + red[1][e]) + (red[2][e] + red[3][e]);
-  }
-}
-
 // BF16 weight gradient on the BF16 matrix cores (v_mfma_f32_16x16x32_bf16), B == 1,
 // n3 % 64 == 0, any C <= 3.  G_p(v) = a(v) c(v + d_p) of two BF16 values has at most 16
 // significant bits, so it is exact in FP32 and splits exactly into hi + lo BF16 parts
@@ -963,86 +783,39 @@ size_t weight_grad_workspace(int dtype, int C, int /*B*/, int n1, int n2, int n3
   return (size_t)wg_blocks(dtype, C, n1, n2, n3) * 27 * (27 * C + 1) * acc;
 }
 
-template <typename TX, typename TI>
-static void launch_wg_t(int dtype, const void* a, const void* c, const void* img, void* part, int nblk,
-                        int C, int B, int n1, int n2, int n3, hipStream_t st) {
-  typedef typename AccOf<TX>::type A;
-  const int tv = wg_tv(dtype, C);
-#define MLPCG_WG(CC, TVV)                                                                  \
-  if (C == CC && tv == TVV) {                                                              \
-    weight_grad_partial_kernel<TX, TI, CC, TVV><<<nblk, kThreads, 0, st>>>(                \
-        (const TX*)a, (const TX*)c, B, (const TI*)img, n1, n2, n3, (A*)part);              \
-    return;                                                                                \
-  }
-  if constexpr (sizeof(A) == 8) {
-    MLPCG_WG(1, 256) MLPCG_WG(2, 128) MLPCG_WG(3, 128)
-  } else {
-    MLPCG_WG(1, 256) MLPCG_WG(2, 256) MLPCG_WG(3, 256)
-  }
-#undef MLPCG_WG
-}
-
 int launch_weight_grad(int dtype, const void* a, const void* c, const void* img, void* gW, void* gb,
                        void* workspace, int C, int B, int n1, int n2, int n3, hipStream_t st) {
   MLPCG_REQUIRE(C >= 1 && C <= 3, "weight_grad: C must be 1, 2 or 3 (got %d)", C);
   const int nblk = wg_blocks(dtype, C, n1, n2, n3);
+  const int NO = 27 * (27 * C + 1);
+  if (dtype == kF64) {
+    const double *pa = (const double*)a, *pc = (const double*)c, *pi = (const double*)img;
+    double* part = (double*)workspace;
+    if (C == 1) weight_grad_partial_kernel<double, double, 1, 256><<<nblk, kThreads, 0, st>>>(pa, pc, B, pi, n1, n2, n3, part);
+    else if (C == 2) weight_grad_partial_kernel<double, double, 2, 128><<<nblk, kThreads, 0, st>>>(pa, pc, B, pi, n1, n2, n3, part);
+    else weight_grad_partial_kernel<double, double, 3, 128><<<nblk, kThreads, 0, st>>>(pa, pc, B, pi, n1, n2, n3, part);
+    weight_grad_final_kernel<double><<<NO, kThreads, 0, st>>>(part, nblk, C, (double*)gW, (double*)gb);
+    return check_launch("weight_grad");
+  }
+  float* part = (float*)workspace;
+  int nb = nblk;
   if (dtype == kBF16 && B == 1 && n3 % wgb::kSeg == 0) {
-    // BF16 matrix-core kernel (same partials layout and block count): columns of J row
-    // segments, about one column per wave
+    // whole 64-cell segments of one BF16 right-hand side: columns of J segments, about one
+    // column per wave, with ring staging (256^3 C = 1 142 us against 175 us of the tiles
+    // below, C = 3 242 against 590 us)
     const long segs = (long)n1 * n2 * (n3 / wgb::kSeg);
     const long per_wave = (segs + 4L * nblk - 1) / (4L * nblk);
     const int J = (int)(per_wave < 4 ? 4 : (per_wave > 64 ? 64 : per_wave));
     const bf16 *pa = (const bf16*)a, *pc = (const bf16*)c, *pi = (const bf16*)img;
-    if (C == 1) weight_grad_bf16_kernel<1><<<nblk, kThreads, 0, st>>>(pa, pc, pi, n1, n2, n3, J, (float*)workspace);
-    else if (C == 2) weight_grad_bf16_kernel<2><<<nblk, kThreads, 0, st>>>(pa, pc, pi, n1, n2, n3, J, (float*)workspace);
-    else weight_grad_bf16_kernel<3><<<nblk, kThreads, 0, st>>>(pa, pc, pi, n1, n2, n3, J, (float*)workspace);
-    weight_grad_final_kernel<float><<<27 * (27 * C + 1), kThreads, 0, st>>>((const float*)workspace, nblk, C,
-                                                                           (float*)gW, (float*)gb);
-    return check_launch("weight_grad");
+    if (C == 1) weight_grad_bf16_kernel<1><<<nblk, kThreads, 0, st>>>(pa, pc, pi, n1, n2, n3, J, part);
+    else if (C == 2) weight_grad_bf16_kernel<2><<<nblk, kThreads, 0, st>>>(pa, pc, pi, n1, n2, n3, J, part);
+    else weight_grad_bf16_kernel<3><<<nblk, kThreads, 0, st>>>(pa, pc, pi, n1, n2, n3, J, part);
+  } else {
+    nb = wgrad_blocks(nblk, n1, n2, n3);
+    const int e = launch_wgrad(dtype, a, c, img, part, nb, C, B, n1, n2, n3, st);
+    if (e) return e;
   }
-  if (C == 1 && dtype != kF64 && n3 % 4 == 0) {
-    // matrix-core kernel (same partials layout and block count)
-    switch (dtype) {
-      case kF32:
-        if (B == 1)
-          weight_grad_mfma_lds_kernel<float, float><<<nblk, kThreads, 0, st>>>(
-              (const float*)a, (const float*)c, (const float*)img, n1, n2, n3, (float*)workspace);
-        else
-          weight_grad_mfma_kernel<float, float><<<nblk, kThreads, 0, st>>>(
-              (const float*)a, (const float*)c, B, (const float*)img, n1, n2, n3, (float*)workspace);
-        break;
-      case kF16:
-        weight_grad_mfma_kernel<f16, f16><<<nblk, kThreads, 0, st>>>(
-            (const f16*)a, (const f16*)c, B, (const f16*)img, n1, n2, n3, (float*)workspace);
-        break;
-      default:
-        if (B == 1)
-          weight_grad_mfma_lds_kernel<bf16, bf16><<<nblk, kThreads, 0, st>>>(
-              (const bf16*)a, (const bf16*)c, (const bf16*)img, n1, n2, n3, (float*)workspace);
-        else
-          weight_grad_mfma_kernel<bf16, bf16><<<nblk, kThreads, 0, st>>>(
-              (const bf16*)a, (const bf16*)c, B, (const bf16*)img, n1, n2, n3, (float*)workspace);
-        break;
-    }
-    weight_grad_final_kernel<float><<<27 * 28, kThreads, 0, st>>>((const float*)workspace, nblk, C,
-                                                                  (float*)gW, (float*)gb);
-    return check_launch("weight_grad");
-  }
-  switch (dtype) {
-    case kF64: launch_wg_t<double, double>(dtype, a, c, img, workspace, nblk, C, B, n1, n2, n3, st); break;
-    case kF32: launch_wg_t<float, float>(dtype, a, c, img, workspace, nblk, C, B, n1, n2, n3, st); break;
-    case kF16: launch_wg_t<f16, f16>(dtype, a, c, img, workspace, nblk, C, B, n1, n2, n3, st); break;
-    case kBF16: launch_wg_t<bf16, bf16>(dtype, a, c, img, workspace, nblk, C, B, n1, n2, n3, st); break;
-    default: MLPCG_REQUIRE(false, "weight_grad: bad dtype %d", dtype);
-  }
-  const int NO = 27 * (27 * C + 1);
-  const int fb = NO;
-  if (dtype == kF64)
-    weight_grad_final_kernel<double><<<fb, kThreads, 0, st>>>((const double*)workspace, nblk, C,
-                                                              (double*)gW, (double*)gb);
-  else
-    weight_grad_final_kernel<float><<<fb, kThreads, 0, st>>>((const float*)workspace, nblk, C,
-                                                             (float*)gW, (float*)gb);
+  weight_grad_final_kernel<float><<<NO, kThreads, 0, st>>>(part, nb, C, (float*)gW, (float*)gb);
   return check_launch("weight_grad");
 }
 

@@ -38,10 +38,8 @@
 // tiles of zero x, and chunks that the output mask zeroes, skip their products.
 #pragma once
 
-#include <type_traits>
-
-#include "common.hpp"
 #include "kernels.hpp"
+#include "split_common.hpp"
 
 namespace mlpcg {
 namespace split {
@@ -51,9 +49,6 @@ constexpr int kPitch = 68;      // cells per staged row (66 used; even, for 8-by
 constexpr int kTarget = 4;      // largest |W| and |img| are scaled into [2^4, 2^5)
 constexpr int kBiasTarget = 8;  // and the largest scaled bias stays below 2^9
 
-typedef f16 h8 __attribute__((ext_vector_type(8)));
-typedef float f16x __attribute__((ext_vector_type(16)));
-typedef unsigned u32x4s __attribute__((ext_vector_type(4)));
 
 // column i (0..4) of lane half h; the fifth of the upper half is a dummy (zero weights)
 __host__ __device__ constexpr int col_of(int h, int i) { return h == 0 ? i : (i < 4 ? 5 + i : 8); }
@@ -70,32 +65,6 @@ struct PackHeader {
 constexpr size_t kHeaderBytes = 64;
 constexpr size_t pack_w_bytes(int C) { return (size_t)2 * 2 * 2 * C * 64 * 8 * sizeof(f16); }
 constexpr size_t pack_bytes(int C) { return kHeaderBytes + pack_w_bytes(C) + 32 * sizeof(float); }
-
-__device__ __forceinline__ unsigned finite_bits(float v) {
-  const unsigned u = __float_as_uint(v) & 0x7fffffffu;
-  return u < 0x7f800000u ? u : 0u;
-}
-// 2^e of the largest finite magnitude (its bits); 0 counts as 1
-__device__ __forceinline__ int exponent_of(unsigned bits) {
-  return bits == 0u ? 0 : (int)(bits >> 23) - 127;
-}
-__device__ __forceinline__ float pow2(int e) { return __uint_as_float((unsigned)(e + 127) << 23); }
-
-__device__ __forceinline__ unsigned wave_max(unsigned v) {
-  auto step = [](unsigned x, auto ctrl, auto rows) {
-    const unsigned o = (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, decltype(ctrl)::value, decltype(rows)::value,
-                                                             0xf, false);
-    return x > o ? x : o;
-  };
-  typedef std::integral_constant<int, 0xf> All;
-  v = step(v, std::integral_constant<int, 0x111>(), All());
-  v = step(v, std::integral_constant<int, 0x112>(), All());
-  v = step(v, std::integral_constant<int, 0x114>(), All());
-  v = step(v, std::integral_constant<int, 0x118>(), All());
-  v = step(v, std::integral_constant<int, 0x142>(), std::integral_constant<int, 0xa>());
-  v = step(v, std::integral_constant<int, 0x143>(), std::integral_constant<int, 0xc>());
-  return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
-}
 
 // Tap (of 27) of K slot j of lane half h in k half kc for z parity par; -1: spare.
 __host__ __device__ constexpr int slot_tap(int par, int h, int kc, int j) {
@@ -173,12 +142,6 @@ __global__ __launch_bounds__(kThreads) void split_pack_kernel(const float* __res
   }
 }
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* p, int bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, bytes, 0x00020000);
-}
-__device__ __forceinline__ float ld(__amdgpu_buffer_rsrc_t r, unsigned boff, int soff) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, boff, soff, 0));
-}
 // a + b after lanes 32..63 of a are traded with lanes 0..31 of b: the lower lanes receive
 // the sum of a's halves, the upper lanes that of b's.  (Both results pass through an empty
 // asm: the ROCm 7.2 compiler otherwise reads the second from the first's register.)
@@ -226,7 +189,7 @@ __device__ __forceinline__ void load_raw(Raw<FI>& r, const float* __restrict__ s
     const int row = w + 4 * k;
     const int gi = t.i0 + row / kPJ - 1, gj = t.j0 + row % kPJ - 1;
     const bool ok = row < tile_rows(FI) && (unsigned)gi < (unsigned)n1 && (unsigned)gj < (unsigned)n2;
-    r.m[k] = ld(rsrc(src + (ok ? gi : 0) * plane, ok ? pb : 0), zo, (ok ? gj : 0) * rb);
+    r.m[k] = ld_as(rsrc(src + (ok ? gi : 0) * plane, ok ? pb : 0), zo, (ok ? gj : 0) * rb, src);
   }
   const int hrow = threadIdx.x >> 1, z = (threadIdx.x & 1) ? t.z0 + kZ : t.z0 - 1;
   const int gi = t.i0 + hrow / kPJ - 1, gj = t.j0 + hrow % kPJ - 1;

@@ -1,0 +1,458 @@
+// Weight gradient of the SM block on the matrix cores, for FP32, BF16 and FP16 data:
+//   D[p][q] = sum_v G_p(v) P_q(v),  G_p(v) = sum_b a[b,v] c[b,v+d_p]   (sm_block_3d_kernel.cu:121-229)
+// with P_q the 27 C image taps and a column of ones (the bias gradient), a 27 x (27C + 1)
+// product over all voxels: gW[p][q] = D[p][q], gb[p] = D[p][27C].
+//
+// a, c and the image are scaled by powers of two (from the tiles' largest finite magnitudes) and G, formed in FP32, and P are split into two FP16 values each (see
+// split_common.hpp); D = G_hi P_hi + G_lo P_hi + G_hi P_lo on v_mfma_f32_32x32x16_f16.  For
+// BF16 data G is exact in its two parts and P in one, so every product is exact; tiles whose
+// image has no low part leave the third product out.  The products with a low part have
+// accumulators of their own: fewer roundings of the large sums (and the matrix cores cut,
+// not round, what is far below their largest addend: adding all three to fresh accumulators
+// per row doubled the error).  A workgroup keeps its smallest factors so far; where a tile
+// needs a smaller one, the sums are rescaled (exact).
+//
+// Tile: 4 planes x 8 rows x 64 z; x and the image with a one-cell halo in LDS, any extents.
+// A wave takes rows of 64 voxels, 16 voxels per product: lane (h, m) = (lane / 32, lane % 32)
+// holds G of tap m and P of column m at voxels 16 s + 8 h + j, j < 8.  The x row and plane
+// pitches (67 and 681 words: 3 and 9 mod 32) put the 27 taps of a half-wave's read on 27
+// different banks; the image's (34 and 358 words) do the same for its words.  a reaches the
+// lanes by a DPP row broadcast inside the multiply (8 LDS reads per product less).  An image tap
+// with d3 = +-1 is five words shifted by half a word, so no shifted copies are kept.
+//
+// Bound by VALU (3 instructions per G: product, difference, two conversions of pairs) and
+// LDS reads, about equally, then by the staging of the tiles (a third of the time), all above
+// the matrix products.  Before (FP32 matrix products gathered from global memory or staged
+// rows, C = 3 on the VALU) -> now: 128^3 FP32 C = 1 88 -> 28 us, two right-hand sides 238 ->
+// 37 us, C = 3 576 -> 98 us; 256^3 C = 1 712 -> 178 us.  Errors against 64 bits (norm-wise):
+// 0.8 to 1.4e-7 where the FP32 products had 0.8 to 3.3e-7.
+#pragma once
+
+#include "kernels.hpp"
+#include "split_common.hpp"
+
+namespace mlpcg {
+namespace wgrad {
+
+using namespace split;
+
+constexpr int kI = 4, kJ = 8, kZ = 64, kPJ = kJ + 2, kRows = (kI + 2) * kPJ;
+constexpr int kXRow = 67, kXPlane = 681;      // x pitches (words); cell z0 - 1 + e at e
+constexpr int kIRow = 68, kIPlane = 716;      // image pitches (half words); cell z0 - 1 + e at 1 + e
+constexpr int kXCells = (kI + 2) * kXPlane, kICells = (kI + 2) * kIPlane;
+static_assert(kXRow % 32 == 3 && kXPlane % 32 == 9 && (kIRow / 2) % 32 == 2 && (kIPlane / 2) % 32 == 6, "banks");
+static_assert(kXPlane >= kPJ * kXRow && kIPlane >= kPJ * kIRow, "planes do not overlap");
+constexpr int kTargetG = 6, kTargetP = 4;  // |a|, |c| into [2^6, 2^7), |image| into [2^4, 2^5)
+constexpr int kOnes = 40;                  // words of FP16 ones, and of zeros, for the bias column
+constexpr int kRw = 3;                     // staged rows per wave and plane: j = w, w + 4, w + 8 of 10
+static_assert(2 * kRows <= kThreads, "staging");
+
+// FP32 cells of a tile as loaded: cell z0 + lane of the wave's rows, and one of the cells
+// z0 - 1, z0 + 64 of all rows
+struct Raw {
+  float m[kI + 2][kRw];
+  float halo;
+};
+
+struct Pos {
+  int i0, j0, z0;
+};
+
+template <typename T>
+__device__ __forceinline__ void load_tile(Raw& r, const T* __restrict__ src, const Pos& t, int n1, int n2, int n3,
+                                          int w, int lane) {
+  const long plane = (long)n2 * n3;
+  const int pb = (int)(plane * (long)sizeof(T)), rb = n3 * (int)sizeof(T);
+  const unsigned zo = t.z0 + lane < n3 ? (unsigned)(t.z0 + lane) * (unsigned)sizeof(T) : 0x80000000u;
+  int so[kRw], jb[kRw];  // row offsets; plane bytes, or 0 for rows outside the grid
+#pragma unroll
+  for (int u = 0; u < kRw; ++u) {
+    const int gj = t.j0 + w + 4 * u - 1;
+    const bool ok = (unsigned)gj < (unsigned)n2 && w + 4 * u < kPJ;
+    so[u] = ok ? gj * rb : 0;
+    jb[u] = ok ? pb : 0;
+  }
+  const T* p = src + (t.i0 - 1) * plane;
+#pragma unroll
+  for (int k = 0; k < kI + 2; ++k) {
+    const bool ok = (unsigned)(t.i0 + k - 1) < (unsigned)n1;
+#pragma unroll
+    for (int u = 0; u < kRw; ++u) r.m[k][u] = ld_as(rsrc(ok ? p : src, ok ? jb[u] : 0), zo, so[u], src);
+    p += plane;
+  }
+  const int hrow = threadIdx.x >> 1, z = (threadIdx.x & 1) ? t.z0 + kZ : t.z0 - 1;
+  const int gi = t.i0 + hrow / kPJ - 1, gj = t.j0 + hrow % kPJ - 1;
+  const bool ok = hrow < kRows && (unsigned)gi < (unsigned)n1 && (unsigned)gj < (unsigned)n2 &&
+                  (unsigned)z < (unsigned)n3;
+  r.halo = ok ? (float)src[((long)gi * n2 + gj) * n3 + z] : 0.f;
+}
+// f(plane, row, e, value) for the thread's cells (rows of the third group exist for two waves)
+template <typename F>
+__device__ __forceinline__ void each(const Raw& r, int w, int lane, F&& f) {
+#pragma unroll
+  for (int u = 0; u < kRw; ++u) {
+    if (w + 4 * u >= kPJ) continue;
+#pragma unroll
+    for (int k = 0; k < kI + 2; ++k) f(k, w + 4 * u, 1 + lane, r.m[k][u]);
+  }
+  const int hrow = threadIdx.x >> 1;
+  if (hrow < kRows) f(hrow / kPJ, hrow % kPJ, (int)(threadIdx.x & 1) * (kZ + 1), r.halo);
+}
+// largest magnitude (NaN aside), infinite if one is
+__device__ __forceinline__ float max_of(const Raw& r) {
+  float m = fabsf(r.halo);
+#pragma unroll
+  for (int k = 0; k < kI + 2; ++k)
+#pragma unroll
+    for (int u = 0; u < kRw; ++u) m = fmaxf(m, fabsf(r.m[k][u]));
+  return m;
+}
+// the same of the finite cells alone
+__device__ __forceinline__ unsigned finite_max_of(const Raw& r) {
+  unsigned m = finite_bits(r.halo);
+#pragma unroll
+  for (int k = 0; k < kI + 2; ++k)
+#pragma unroll
+    for (int u = 0; u < kRw; ++u) m = max(m, finite_bits(r.m[k][u]));
+  return m;
+}
+__device__ __forceinline__ int scale_exp(unsigned bits, int target) {
+  return max(-126, min(target - exponent_of(bits), 126));
+}
+// lane I of a row of 16 to the whole row
+template <int I>
+__device__ __forceinline__ float row_bcast(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x150 + I, 0xf, 0xf, true));
+}
+// FP16 parts of two values: hi rounded, lo = v - hi rounded.  The differences are written out
+// (a mixed-precision FMA each): left to the ROCm 7.2 compiler, hi is rounded from the exact
+// product behind v in one use and from its FP32 value in another, and no longer fits its lo.
+typedef f16 h2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void split_pair(float v0, float v1, unsigned& hi, unsigned& lo) {
+  float d0, d1;
+  asm("" : "+v"(v0), "+v"(v1));
+  hi = __builtin_bit_cast(unsigned, h2{(f16)v0, (f16)v1});
+  asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[0,0,1]" : "=v"(d0) : "v"(v0), "v"(hi));
+  asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(d1) : "v"(v1), "v"(hi));
+  lo = __builtin_bit_cast(unsigned, h2{(f16)d0, (f16)d1});
+}
+
+// G[j] = (ACC: G[j] +) g of voxel j times x[j].  (Contracted into the difference v - hi, the
+// product could not take its broadcast as a DPP operand.)
+template <bool ACC>
+__device__ __forceinline__ void products(float g, const float (&x)[8], float (&G)[8]) {
+#pragma clang fp contract(off)
+  const float gb[8] = {row_bcast<0>(g), row_bcast<1>(g), row_bcast<2>(g), row_bcast<3>(g),
+                       row_bcast<4>(g), row_bcast<5>(g), row_bcast<6>(g), row_bcast<7>(g)};
+#pragma unroll
+  for (int j = 0; j < 8; ++j) G[j] = ACC ? __builtin_fmaf(gb[j], x[j], G[j]) : gb[j] * x[j];
+}
+
+// registers for this many waves per SIMD
+__host__ __device__ constexpr int waves(int C, int BB) { return C == 1 ? 4 : 2; }
+
+// BB: right-hand sides staged together
+template <typename T, int C, int BB>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(waves(C, BB), 8)))
+void wgrad_kernel(const T* __restrict__ a, const T* __restrict__ cv, int B, const T* __restrict__ img, int n1, int n2,
+                  int n3, float* __restrict__ partials) {
+  constexpr int NQ = 27 * C + 1, NT = (NQ + 31) / 32, NO = 27 * NQ, kOneTile = 27 * C / 32;
+  constexpr int kXB = BB * kXCells * 4, kIB = C * kICells * 2, kRed = 4 * 32 * 32 * 4;
+  constexpr int kOnesAt = kXB + 2 * kIB, kUsed = kOnesAt + 2 * kOnes * 4;
+  __shared__ __attribute__((aligned(16))) char lds[kUsed > kRed ? kUsed : kRed];
+  __shared__ unsigned sh[4][4];
+  float* xs = (float*)lds;      // [BB][kXCells]
+  f16* ih = (f16*)(lds + kXB);  // [C][kICells], then the low parts
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = lane >> 5, m = lane & 31;
+  const long V = (long)n1 * n2 * n3;
+  const unsigned tz = (unsigned)((n3 + kZ - 1) / kZ), tj = (unsigned)((n2 + kJ - 1) / kJ);
+  const unsigned tiles = tz * tj * (unsigned)((n1 + kI - 1) / kI);
+  for (int e = threadIdx.x; e < 2 * kOnes; e += kThreads)
+    *(unsigned*)(lds + kOnesAt + 4 * e) = e < kOnes ? 0x3c003c00u : 0u;
+
+  // word offsets in LDS of the lane's tap (27 .. 31 repeat tap 26, their rows are dropped)
+  // and columns at row (0, w), and their steps to the row of the other half tile; the column
+  // of ones stays where it is
+  const int p = m < 27 ? m : 26;
+  const int xo = (p / 9) * kXPlane + (p / 3 % 3) * kXRow + w * kXRow + 8 * h + p % 3;
+  int io[NT], lo_o[NT], ish[NT];
+  const bool one = 32 * kOneTile + m == 27 * C;
+  const int on_row = one ? 0 : 1;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int q = 32 * t + m < 27 * C ? 32 * t + m : 27 * C - 1, c = q / 27, s = q % 27;
+    // word of the first of the lane's cells: d3 = 0 starts on a word, d3 = -1 / +1 half a
+    // word later than the word before / at it
+    const int word = (c * kICells + (s / 9) * kIPlane + (s / 3 % 3) * kIRow + w * kIRow) / 2 + 4 * h + (s % 3 == 0 ? 0 : 1);
+    const bool o1 = t == kOneTile && one;
+    io[t] = o1 ? kOnesAt / 4 : kXB / 4 + word;
+    lo_o[t] = o1 ? kOnesAt / 4 + kOnes : (kXB + kIB) / 4 + word;
+    ish[t] = s % 3 == 1 ? 0 : 16;
+  }
+  // the products of the high parts, and those with a low part: both in units of the block's
+  // scales so far (the smallest factors of its tiles)
+  f16x acc[NT], acl[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) acc[t] = acl[t] = f16x{};
+  int ex = 126, eg = 126, ei = 126;
+  auto rescale = [&](int exg, int eimg) {  // by 2^exg, and 2^eimg but for the column of ones
+    if (exg == 0 && eimg == 0) return;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int e = exg + (t == kOneTile && one ? 0 : eimg);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        acc[t][i] = ldexpf(acc[t][i], e);
+        acl[t][i] = ldexpf(acl[t][i], e);
+      }
+    }
+  };
+
+  for (unsigned tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    const unsigned u = tile / tz;
+    const Pos pos{(int)(u / tj) * kI, (int)(u % tj) * kJ, (int)(tile % tz) * kZ};
+    // a row of a (range-checked: rows and cells outside the grid read 0)
+    auto row_of_a = [&](int b, int q) {
+      const int gi = pos.i0 + (q >> 1), gj = pos.j0 + w + 4 * (q & 1);
+      const bool ok = gi < n1 && gj < n2 && b < B;
+      return rsrc(a + (ok ? (long)b * V + ((long)gi * n2 + gj) * n3 : 0L), ok ? n3 * (int)sizeof(T) : 0);
+    };
+    // the lane's a values of a row: voxels 16 s + 8 h + lane % 8
+    const unsigned go = (unsigned)(pos.z0 + 8 * h + (lane & 7)) * (unsigned)sizeof(T);
+    auto load_g = [&](float (&g)[BB][4], int b0, int q) {
+#pragma unroll
+      for (int bb = 0; bb < BB; ++bb) {
+        const auto r = row_of_a(b0 + bb, q);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) g[bb][s] = ld_as(r, go + 16 * s * (unsigned)sizeof(T), 0, a);
+      }
+    };
+    bool has_lo = false;
+    for (int b0 = 0; b0 < B; b0 += BB) {
+      Raw ri[C], rx[BB];
+      float mi = 0.f, mx = 0.f, mg = 0.f;
+      if (b0 == 0) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) load_tile(ri[c], img + c * V, pos, n1, n2, n3, w, lane);
+      }
+      // (an absent right-hand side repeats the last: its a reads as 0)
+#pragma unroll
+      for (int bb = 0; bb < BB; ++bb) load_tile(rx[bb], cv + (long)min(b0 + bb, B - 1) * V, pos, n1, n2, n3, w, lane);
+      // a's rows, for the scale only (the products read them again, from L2)
+      float rg[BB][kI * kJ / 4];
+#pragma unroll
+      for (int bb = 0; bb < BB; ++bb)
+#pragma unroll
+        for (int q = 0; q < kI * kJ / 4; ++q)
+          rg[bb][q] = ld_as(row_of_a(b0 + bb, q), (unsigned)(pos.z0 + lane) * (unsigned)sizeof(T), 0, a);
+      if (b0 == 0) {
+#pragma unroll
+        for (int c = 0; c < C; ++c) mi = fmaxf(mi, max_of(ri[c]));
+      }
+#pragma unroll
+      for (int bb = 0; bb < BB; ++bb) {
+        mx = fmaxf(mx, max_of(rx[bb]));
+#pragma unroll
+        for (int q = 0; q < kI * kJ / 4; ++q) mg = fmaxf(mg, fabsf(rg[bb][q]));
+      }
+      unsigned bi = __float_as_uint(mi), bx = __float_as_uint(mx), bg = __float_as_uint(mg);
+      if (__builtin_amdgcn_ballot_w64(max(bi, max(bx, bg)) >= 0x7f800000u)) {  // infinities set no scale
+        bi = bx = bg = 0;
+        if (b0 == 0)
+          for (int c = 0; c < C; ++c) bi = max(bi, finite_max_of(ri[c]));
+        for (int bb = 0; bb < BB; ++bb) {
+          bx = max(bx, finite_max_of(rx[bb]));
+          for (int q = 0; q < kI * kJ / 4; ++q) bg = max(bg, finite_bits(rg[bb][q]));
+        }
+      }
+      bi = wave_max(bi);
+      bx = wave_max(bx);
+      bg = wave_max(bg);
+      __syncthreads();  // the previous tile's reads are done
+      if (lane == 0) {
+        sh[w][0] = bi;
+        sh[w][1] = bx;
+        sh[w][2] = bg;
+      }
+      __syncthreads();
+      auto over_waves = [&](int k) {
+        return (unsigned)__builtin_amdgcn_readfirstlane((int)max(max(sh[0][k], sh[1][k]), max(sh[2][k], sh[3][k])));
+      };
+      const int ex_n = min(ex, scale_exp(over_waves(1), kTargetG)), eg_n = min(eg, scale_exp(over_waves(2), kTargetG));
+      const int ei_n = b0 == 0 ? min(ei, scale_exp(over_waves(0), kTargetP)) : ei;
+      rescale(ex_n - ex + eg_n - eg, ei_n - ei);
+      ex = ex_n;
+      eg = eg_n;
+      ei = ei_n;
+      const float sx = pow2(ex), sg = pow2(eg);
+#pragma unroll
+      for (int bb = 0; bb < BB; ++bb)
+        each(rx[bb], w, lane, [&](int k, int j, int e, float v) {
+          xs[bb * kXCells + k * kXPlane + j * kXRow + e] = v * sx;
+        });
+      if (b0 == 0) {
+        unsigned any = 0;
+        const float si = pow2(ei);
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+          each(ri[c], w, lane, [&](int k, int j, int e, float v) {
+            const float sv = v * si;
+            const f16 hi = (f16)sv, lo = (f16)(sv - (float)hi);
+            f16* d = ih + c * kICells + k * kIPlane + j * kIRow + 1 + e;
+            d[0] = hi;
+            d[C * kICells] = lo;
+            any |= __builtin_bit_cast(unsigned short, lo);
+          });
+        any = __builtin_amdgcn_ballot_w64((any & 0x7fffu) != 0) != 0;
+        if (lane == 0) sh[w][3] = any;
+      }
+      __syncthreads();
+      if (b0 == 0) has_lo = over_waves(3) != 0;
+
+      auto rows = [&](auto lo_c) {
+        constexpr bool LO = decltype(lo_c)::value;
+        // operands of one product step, read one step ahead of their use
+        struct Step {
+          float x[BB][8];
+          unsigned ph[NT][5];
+        };
+        struct Base {
+          int x, i[NT], l[NT];
+        };
+        auto base = [&](int q) {  // row w + 4 (q % 2) of plane q / 2
+          const int irow = ((q >> 1) * kIPlane + (q & 1) * 4 * kIRow) / 2;
+          Base r;
+          r.x = xo + (q >> 1) * kXPlane + (q & 1) * 4 * kXRow;
+#pragma unroll
+          for (int t = 0; t < NT; ++t) {
+            const int step = t == kOneTile ? on_row * irow : irow;
+            r.i[t] = io[t] + step;
+            r.l[t] = lo_o[t] + step;
+          }
+          return r;
+        };
+        auto load = [&](Step& st, const Base& r, int s) {
+#pragma unroll
+          for (int bb = 0; bb < BB; ++bb)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) st.x[bb][j] = ((const float*)lds)[r.x + bb * kXCells + 16 * s + j];
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int k = 0; k < 5; ++k) st.ph[t][k] = ((const unsigned*)lds)[r.i[t] + 8 * s + k];
+        };
+        float gc[BB][4], gn[BB][4];
+        load_g(gc, b0, 0);
+        Base bc = base(0);
+        Step cur;
+        load(cur, bc, 0);
+#pragma unroll 1
+        for (int q = 0; q < kI * kJ / 4; ++q) {
+          const int qn = q + 1 < kI * kJ / 4 ? q + 1 : q;
+          load_g(gn, b0, qn);
+          const Base bn = base(qn);
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            Step nxt;
+            if (s < 3) load(nxt, bc, s + 1);
+            else load(nxt, bn, 0);
+            float G[8];
+#pragma unroll
+            for (int bb = 0; bb < BB; ++bb) {
+              if (bb == 0) products<false>(gc[bb][s] * sg, cur.x[bb], G);
+              else products<true>(gc[bb][s] * sg, cur.x[bb], G);
+            }
+            u32x4s gh, gl;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              unsigned hi, lo;
+              split_pair(G[2 * k], G[2 * k + 1], hi, lo);
+              gh[k] = hi;
+              gl[k] = lo;
+            }
+            auto cols = [&](const unsigned (&x)[5], int t) {
+              u32x4s r;
+#pragma unroll
+              for (int k = 0; k < 4; ++k) r[k] = __builtin_amdgcn_alignbit(x[k + 1], x[k], (unsigned)ish[t]);
+              return __builtin_bit_cast(h8, r);
+            };
+            const h8 ah = __builtin_bit_cast(h8, gh), al = __builtin_bit_cast(h8, gl);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+              const h8 ph = cols(cur.ph[t], t);
+              acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, ph, acc[t], 0, 0, 0);
+              acl[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, ph, acl[t], 0, 0, 0);
+              if (LO) {
+                unsigned pl[5];
+#pragma unroll
+                for (int k = 0; k < 5; ++k) pl[k] = ((const unsigned*)lds)[bc.l[t] + 8 * s + k];
+                acl[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, cols(pl, t), acl[t], 0, 0, 0);
+              }
+            }
+            cur = nxt;
+          }
+          bc = bn;
+#pragma unroll
+          for (int bb = 0; bb < BB; ++bb)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) gc[bb][s] = gn[bb][s];
+        }
+      };
+      if (has_lo) rows(std::true_type());
+      else rows(std::false_type());
+    }
+  }
+  // D[8 (i / 4) + 4 h + i % 4][32 t + m] of the wave, the waves added in order
+  float* red = (float*)lds;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      red[(w * 32 + 8 * (i >> 2) + 4 * h + (i & 3)) * 32 + m] =
+          ldexpf(acc[t][i] + acl[t][i], -ex - eg - (t == kOneTile && one ? 0 : ei));
+    __syncthreads();
+    for (int e = threadIdx.x; e < 27 * 32; e += kThreads) {
+      const int pp = e >> 5, q = 32 * t + (e & 31);
+      if (q < NQ)
+        partials[(size_t)blockIdx.x * NO + pp * NQ + q] =
+            (red[e] + red[1024 + e]) + (red[2048 + e] + red[3072 + e]);
+    }
+  }
+}
+
+// workgroups: one per tile, at most `most` (the partial sums' workspace)
+inline int blocks(int most, int n1, int n2, int n3) {
+  const long tiles = (long)((n1 + kI - 1) / kI) * ((n2 + kJ - 1) / kJ) * ((n3 + kZ - 1) / kZ);
+  return (int)(tiles < most ? tiles : most);
+}
+
+template <typename T>
+void launch(const void* a, const void* c, const void* img, float* part, int nblk, int C, int B, int n1, int n2, int n3,
+            hipStream_t st) {
+#define MLPCG_WGK(CC)                                                                                               \
+  if (C == CC) {                                                                                                    \
+    if (B == 1)                                                                                                     \
+      wgrad_kernel<T, CC, 1><<<nblk, kThreads, 0, st>>>((const T*)a, (const T*)c, B, (const T*)img, n1, n2, n3, part); \
+    else                                                                                                            \
+      wgrad_kernel<T, CC, 2><<<nblk, kThreads, 0, st>>>((const T*)a, (const T*)c, B, (const T*)img, n1, n2, n3, part); \
+  }
+  MLPCG_WGK(1) MLPCG_WGK(2) MLPCG_WGK(3)
+#undef MLPCG_WGK
+}
+
+}  // namespace wgrad
+
+int wgrad_blocks(int most, int n1, int n2, int n3) { return wgrad::blocks(most, n1, n2, n3); }
+
+int launch_wgrad(int dtype, const void* a, const void* c, const void* img, float* part, int nblk, int C, int B, int n1,
+                 int n2, int n3, hipStream_t st) {
+  if (dtype == kF32) wgrad::launch<float>(a, c, img, part, nblk, C, B, n1, n2, n3, st);
+  else if (dtype == kF16) wgrad::launch<f16>(a, c, img, part, nblk, C, B, n1, n2, n3, st);
+  else if (dtype == kBF16) wgrad::launch<bf16>(a, c, img, part, nblk, C, B, n1, n2, n3, st);
+  else MLPCG_REQUIRE(false, "weight_grad: bad dtype %d", dtype);
+  return check_launch("weight_grad");
+}
+
+}  // namespace mlpcg
