@@ -8,6 +8,7 @@
 //   values outside the grid are zero.
 #pragma once
 
+#include <type_traits>
 #include <hip/hip_runtime.h>
 #include <cstddef>
 #include <cstdint>
@@ -133,6 +134,25 @@ __device__ __forceinline__ A wave_sum(A v) {
   return v;
 }
 
+// sum over the wave by DPP row shifts and row broadcasts; valid in lane 63
+__device__ __forceinline__ double wave_sum_dpp(double v) {
+  auto step = [](double x, auto ctrl, auto rows) {
+    constexpr int kCtrl = decltype(ctrl)::value, kRows = decltype(rows)::value;
+    const long long u = __builtin_bit_cast(long long, x);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)u, kCtrl, kRows, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), kCtrl, kRows, 0xf, false);
+    return x + __builtin_bit_cast(double, ((long long)(unsigned)hi << 32) | (unsigned)lo);
+  };
+  typedef std::integral_constant<int, 0xf> All;
+  v = step(v, std::integral_constant<int, 0x111>(), All());  // row_shr 1, 2, 4, 8
+  v = step(v, std::integral_constant<int, 0x112>(), All());
+  v = step(v, std::integral_constant<int, 0x114>(), All());
+  v = step(v, std::integral_constant<int, 0x118>(), All());
+  v = step(v, std::integral_constant<int, 0x142>(), std::integral_constant<int, 0xa>());  // row_bcast 15
+  v = step(v, std::integral_constant<int, 0x143>(), std::integral_constant<int, 0xc>());  // row_bcast 31
+  return v;
+}
+
 // Sum over a 256-thread block; result valid in every thread.  `sh` holds >= 4 values.
 template <typename A>
 __device__ __forceinline__ A block_sum(A v, A* sh) {
@@ -156,8 +176,8 @@ __device__ __forceinline__ void block_partials(const double (&v)[NR], double* __
   const int w = threadIdx.x >> 6;
 #pragma unroll
   for (int r = 0; r < NR; ++r) {
-    double s = wave_sum(v[r]);
-    if ((threadIdx.x & 63) == 0) sh[r][w] = s;
+    const double s = wave_sum_dpp(v[r]);
+    if ((threadIdx.x & 63) == 63) sh[r][w] = s;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -185,9 +205,9 @@ __device__ __forceinline__ double sum_partials(const double* __restrict__ p, uns
 #pragma unroll
   for (int u = 0; u < 8; ++u)
     if (b + u * kFinThreads < nb) a[u] += p[b + u * kFinThreads];
-  double s = wave_sum(((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7])));
+  const double s = wave_sum_dpp(((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7])));
   __syncthreads();
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+  if ((threadIdx.x & 63) == 63) sh[threadIdx.x >> 6] = s;
   __syncthreads();
   double t = 0.0;
   if (threadIdx.x == 0)
@@ -207,30 +227,34 @@ __device__ __forceinline__ void sum_partials_rows(const double* __restrict__ p, 
   for (int r = 0; r < NR; ++r)
 #pragma unroll
     for (int u = 0; u < 8; ++u) a[r][u] = 0.0;
-  unsigned b = threadIdx.x;
-  for (; b + 7 * kFinThreads < nb; b += 8 * kFinThreads) {
+  // every load is unconditional (clamped index) and issued before the first sum: a branch
+  // around each would wait for each in turn
+  for (unsigned b = threadIdx.x; b - threadIdx.x < nb; b += 8 * kFinThreads) {
+    double v[NR][8];
 #pragma unroll
     for (int r = 0; r < NR; ++r)
-      if (r < nr)
 #pragma unroll
-        for (int u = 0; u < 8; ++u) a[r][u] += p[(size_t)r * nb + b + u * kFinThreads];
+      for (int u = 0; u < 8; ++u) {
+        const unsigned e = b + u * kFinThreads;
+        v[r][u] = p[(size_t)(r < nr ? r : nr - 1) * nb + (e < nb ? e : nb - 1)];
+      }
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+#pragma unroll
+      for (int u = 0; u < 8; ++u) a[r][u] += b + u * kFinThreads < nb ? v[r][u] : 0.0;
   }
 #pragma unroll
-  for (int r = 0; r < NR; ++r)
-    if (r < nr)
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (b + u * kFinThreads < nb) a[r][u] += p[(size_t)r * nb + b + u * kFinThreads];
-#pragma unroll
   for (int r = 0; r < NR; ++r) {
-    const double s = wave_sum(((a[r][0] + a[r][1]) + (a[r][2] + a[r][3])) + ((a[r][4] + a[r][5]) + (a[r][6] + a[r][7])));
-    if ((threadIdx.x & 63) == 0) sh[r][threadIdx.x >> 6] = s;
+    const double s =
+        wave_sum_dpp(((a[r][0] + a[r][1]) + (a[r][2] + a[r][3])) + ((a[r][4] + a[r][5]) + (a[r][6] + a[r][7])));
+    if ((threadIdx.x & 63) == 63) sh[r][threadIdx.x >> 6] = s;
   }
   __syncthreads();
   if (threadIdx.x == 0) {
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
       double v = 0.0;
+#pragma unroll
       for (int w = 0; w < kFinThreads / 64; ++w) v += sh[r][w];
       t[r] = v;
     }

@@ -59,43 +59,55 @@ struct Run {
 
 template <int VZ>
 __device__ __forceinline__ bool run_at(long cid, int n1, int n2, int n3, Run<VZ>& r) {
-  const int n3c = n3 / VZ;
+  const unsigned n3c = (unsigned)n3 / VZ;
   const long nch = (long)n1 * n2 * n3c;
   if (cid >= nch) return false;
-  r.k0 = (int)(cid % n3c) * VZ;
-  const long t = cid / n3c;
-  r.j = (int)(t % n2);
-  r.i = (int)(t / n2);
+  if (nch <= 0xffffffffL) {  // uniform; 64-bit divisions take a hundred instructions more
+    const unsigned u = (unsigned)cid, t = u / n3c;
+    r.k0 = (int)(u - t * n3c) * VZ;
+    r.i = (int)(t / (unsigned)n2);
+    r.j = (int)(t - (unsigned)r.i * (unsigned)n2);
+  } else {
+    r.k0 = (int)(cid % n3c) * VZ;
+    const long t = cid / n3c;
+    r.j = (int)(t % n2);
+    r.i = (int)(t / n2);
+  }
   r.v0 = ((long)r.i * n2 + r.j) * n3 + r.k0;
   return true;
 }
 
-// Loads u = x + a*p (or just x when p == nullptr) on the 7-point neighbourhood of a run:
+// Loads u = x + a*p (or just x when p == nullptr) on the 7-point neighbourhood of a run
+// (near: of the run's own cells, which neighbouring lanes use; own: all of it):
 // c[0..VZ+1] is the centre row with one halo cell each side, s[4][VZ] the four side rows
 // (i-1, i+1, j-1, j+1).  Out-of-grid values are 0.  u is one FP32 fused multiply-add (the
 // storage precision of x, one rounding) so a residual computed from it is the residual of
 // the stored iterate.
-template <typename TA>
-__device__ __forceinline__ TA upd(float x, float p, float a, bool has_p) {
-  return has_p ? (TA)fmaf(a, p, x) : (TA)x;
+__device__ __forceinline__ float upd(float x, float p, float a, bool has_p) {
+  return has_p ? fmaf(a, p, x) : x;
 }
 
-template <int VZ, typename TA>
+template <int VZ>
 __device__ __forceinline__ void load_star(const float* __restrict__ x, const float* __restrict__ p,
                                           float a, const Run<VZ>& r, int n1, int n2, int n3,
-                                          TA (&c)[VZ + 2], TA (&s)[4][VZ]) {
+                                          float (&c)[VZ + 2], float (&s)[4][VZ], bool own = true, bool near = true) {
   const long s1 = (long)n2 * n3;
   const int lane = threadIdx.x & 63;
   float xv[VZ], pv[VZ];
-  load_vec<VZ>(x + r.v0, xv);
-  if (p) load_vec<VZ>(p + r.v0, pv);
 #pragma unroll
-  for (int t = 0; t < VZ; ++t) c[t + 1] = upd<TA>(xv[t], p ? pv[t] : 0.f, a, p != nullptr);
-  TA lft = wave_from_prev(c[VZ]), rgt = wave_from_next(c[1]);
-  if (lane == 0 && r.k0 > 0) lft = upd<TA>(x[r.v0 - 1], p ? p[r.v0 - 1] : 0.f, a, p != nullptr);
-  if (lane == 63 && r.k0 + VZ < n3) rgt = upd<TA>(x[r.v0 + VZ], p ? p[r.v0 + VZ] : 0.f, a, p != nullptr);
-  c[0] = r.k0 > 0 ? lft : TA(0);
-  c[VZ + 1] = r.k0 + VZ < n3 ? rgt : TA(0);
+  for (int t = 0; t < VZ; ++t) c[t + 1] = 0.f;
+  if (near) {
+    load_vec<VZ>(x + r.v0, xv);
+    if (p) load_vec<VZ>(p + r.v0, pv);
+#pragma unroll
+    for (int t = 0; t < VZ; ++t) c[t + 1] = upd(xv[t], p ? pv[t] : 0.f, a, p != nullptr);
+  }
+  float lft = wave_from_prev(c[VZ]), rgt = wave_from_next(c[1]);
+  if (!own) return;
+  if (lane == 0 && r.k0 > 0) lft = upd(x[r.v0 - 1], p ? p[r.v0 - 1] : 0.f, a, p != nullptr);
+  if (lane == 63 && r.k0 + VZ < n3) rgt = upd(x[r.v0 + VZ], p ? p[r.v0 + VZ] : 0.f, a, p != nullptr);
+  c[0] = r.k0 > 0 ? lft : 0.f;
+  c[VZ + 1] = r.k0 + VZ < n3 ? rgt : 0.f;
   const long offs[4] = {-s1, s1, -(long)n3, (long)n3};
   const bool ok[4] = {r.i > 0, r.i < n1 - 1, r.j > 0, r.j < n2 - 1};
 #pragma unroll
@@ -104,54 +116,84 @@ __device__ __forceinline__ void load_star(const float* __restrict__ x, const flo
       load_vec<VZ>(x + r.v0 + offs[q], xv);
       if (p) load_vec<VZ>(p + r.v0 + offs[q], pv);
 #pragma unroll
-      for (int t = 0; t < VZ; ++t) s[q][t] = upd<TA>(xv[t], p ? pv[t] : 0.f, a, p != nullptr);
+      for (int t = 0; t < VZ; ++t) s[q][t] = upd(xv[t], p ? pv[t] : 0.f, a, p != nullptr);
     } else {
 #pragma unroll
-      for (int t = 0; t < VZ; ++t) s[q][t] = TA(0);
+      for (int t = 0; t < VZ; ++t) s[q][t] = 0.f;
     }
   }
 }
 
+// TA: the type of the sums
 template <int VZ, typename TA>
-__device__ __forceinline__ TA lap_at(const TA (&c)[VZ + 2], const TA (&s)[4][VZ], int t, int code) {
-  const TA nb = c[t] + c[t + 2] + s[0][t] + s[1][t] + s[2][t] + s[3][t];
-  return (TA)(code - 1) * c[t + 1] - nb;
+__device__ __forceinline__ TA lap_at(const float (&c)[VZ + 2], const float (&s)[4][VZ], int t, int code) {
+  const TA nb = (TA)c[t] + (TA)c[t + 2] + (TA)s[0][t] + (TA)s[1][t] + (TA)s[2][t] + (TA)s[3][t];
+  return (TA)(code - 1) * (TA)c[t + 1] - nb;
 }
 
-// r = b - A x_new,  x_new = x_old + alpha p (alpha from the state unless init).
-// Reduces [r.r, b.b].
+// Codes of a run, and which of its vectors matter: a run without fluid cells (air above the
+// water, solids) has zeros in every output, stored once when the buffers were made, and is
+// only read for the halo cell of a neighbouring lane's run.  The kernels below therefore
+// fetch the codes first (one byte per voxel against 16 to 28 of the vectors) and skip the
+// loads and stores of the rest: 256^3 filled to 55 %, npsd_dir 111 -> 74 us, resid 83 -> 57 us
+// (3.2 TB/s of what remains: the air leaves every fourth 256 bytes of a row untouched, so the
+// memory channels are not loaded alike).
 template <int VZ>
-__global__ __launch_bounds__(kThreads) void resid_flat_kernel(FlatArgs a, int init) {
+struct Codes {
+  uint8_t c[VZ];
+  bool own;   // a fluid cell in the run
+  bool near;  // ... or in the run of a neighbouring lane
+  __device__ __forceinline__ void load(const uint8_t* __restrict__ code, bool all) {
+    load_vec_nt<VZ>(code, c);
+    unsigned any = all ? 1u : 0u;
+#pragma unroll
+    for (int t = 0; t < VZ; ++t) any |= c[t];
+    own = any != 0;
+    near = (any | (unsigned)dpp_prev((int)any) | (unsigned)dpp_next((int)any)) != 0;
+  }
+};
+
+// r = b - A x_new,  x_new = x_old + alpha p (alpha from the state unless init).
+// Reduces r.r, and b.b at the start (over all cells).
+template <int VZ, bool INIT>
+__global__ __launch_bounds__(kThreads) void resid_flat_kernel(FlatArgs a) {
   SolveState* st = a.st;
-  if (!init && st->done) return;
-  const float alpha = init ? 0.f : (float)st->alpha;
-  const float* pp = init ? nullptr : a.p;
-  double red[2] = {0.0, 0.0};
+  if (!INIT && st->done) return;
+  const float alpha = INIT ? 0.f : (float)st->alpha;
+  const float* pp = INIT ? nullptr : a.p;
+  double red[INIT ? 2 : 1] = {};
   const long nch = (long)a.n1 * a.n2 * (a.n3 / VZ);
   for (long cid = (long)xcd_block(blockIdx.x, gridDim.x) * kThreads + threadIdx.x; cid < nch;
        cid += (long)gridDim.x * kThreads) {
     Run<VZ> r;
     run_at<VZ>(cid, a.n1, a.n2, a.n3, r);
-    double c[VZ + 2], s[4][VZ];
-    load_star<VZ, double>(a.x_old, pp, alpha, r, a.n1, a.n2, a.n3, c, s);
-    float bv[VZ], code[VZ];
+    Codes<VZ> code;
+    code.load(a.code + r.v0, INIT);
+    float bv[VZ];
     // single-use streams and outputs bypass L2 (the x and p rows of the neighbourhood stay)
-    load_vec_nt<VZ>(a.b + r.v0, bv);
-    load_vec_nt<VZ>(a.code + r.v0, code);
+    if (code.own) load_vec_nt<VZ>(a.b + r.v0, bv);
+    float c[VZ + 2], s[4][VZ];
+    load_star<VZ>(a.x_old, pp, alpha, r, a.n1, a.n2, a.n3, c, s, code.own, code.near);
     float rv[VZ], xn[VZ];
+    if (code.own) {
 #pragma unroll
-    for (int t = 0; t < VZ; ++t) {
-      const int cd = (int)code[t];
-      const double res = cd ? (double)bv[t] - lap_at<VZ, double>(c, s, t, cd) : 0.0;
-      rv[t] = (float)res;
-      xn[t] = cd ? (float)c[t + 1] : 0.f;
-      red[0] += res * res;
-      red[1] += (double)bv[t] * (double)bv[t];
+      for (int t = 0; t < VZ; ++t) {
+        const int cd = (int)code.c[t];
+        const double res = cd ? (double)bv[t] - lap_at<VZ, double>(c, s, t, cd) : 0.0;
+        rv[t] = (float)res;
+        xn[t] = cd ? c[t + 1] : 0.f;
+        red[0] += res * res;
+        if (INIT) red[INIT ? 1 : 0] += (double)bv[t] * (double)bv[t];
+      }
+      store_vec_nt<VZ>(a.r + r.v0, rv);
+      if (!INIT) store_vec_nt<VZ>(a.x_new + r.v0, xn);
+    } else if (a.full_x) {
+#pragma unroll
+      for (int t = 0; t < VZ; ++t) xn[t] = 0.f;
+      store_vec_nt<VZ>(a.x_new + r.v0, xn);
     }
-    store_vec_nt<VZ>(a.r + r.v0, rv);
-    if (!init) store_vec_nt<VZ>(a.x_new + r.v0, xn);
   }
-  block_partials<2>(red, a.partials);
+  block_partials<INIT ? 2 : 1>(red, a.partials);
 }
 
 // p_new = z + beta p_old; w = A p_new; reduces p_new . w -> alpha = rho / (p.w).
@@ -166,15 +208,16 @@ __global__ __launch_bounds__(kThreads) void p_spmv_flat_kernel(FlatArgs a) {
        cid += (long)gridDim.x * kThreads) {
     Run<VZ> r;
     run_at<VZ>(cid, a.n1, a.n2, a.n3, r);
+    Codes<VZ> code;
+    code.load(a.code + r.v0, false);
     float c[VZ + 2], s[4][VZ];
     // p_new = z + beta * p_old, evaluated on the neighbourhood
-    load_star<VZ, float>(a.z, a.p_old, beta, r, a.n1, a.n2, a.n3, c, s);
-    float code[VZ];
-    load_vec_nt<VZ>(a.code + r.v0, code);
+    load_star<VZ>(a.z, a.p_old, beta, r, a.n1, a.n2, a.n3, c, s, code.own, code.near);
+    if (!code.own) continue;
     float wv[VZ], pn[VZ];
 #pragma unroll
     for (int t = 0; t < VZ; ++t) {
-      const int cd = (int)code[t];
+      const int cd = (int)code.c[t];
       const float w = cd ? lap_at<VZ, float>(c, s, t, cd) : 0.f;
       pn[t] = cd ? c[t + 1] : 0.f;
       wv[t] = w;
@@ -321,7 +364,7 @@ __global__ __launch_bounds__(kThreads) void spmv_flat_kernel(const uint8_t* __re
   Run<VZ> r;
   if (!run_at<VZ>(cid, n1, n2, n3, r)) return;
   float c[VZ + 2], s[4][VZ];
-  load_star<VZ, float>(x, nullptr, 0.f, r, n1, n2, n3, c, s);
+  load_star<VZ>(x, nullptr, 0.f, r, n1, n2, n3, c, s);
   float cd[VZ], out[VZ];
   load_vec<VZ>(code + r.v0, cd);
 #pragma unroll
@@ -575,14 +618,17 @@ __device__ __forceinline__ void dir_vec(const DirIn& d, long v0, float (&out)[VZ
 template <int VZ>
 __device__ __forceinline__ void load_dir_star(const DirIn& d, const Run<VZ>& r, int n1, int n2,
                                               int n3, float (&c)[VZ + 2], float (&s)[4][VZ],
-                                              float (&ncen)[VZ]) {
+                                              float (&ncen)[VZ], bool own, bool near) {
   const long s1 = (long)n2 * n3;
   const int lane = threadIdx.x & 63;
   float cv[VZ];
-  dir_vec<VZ>(d, r.v0, cv, ncen);
+#pragma unroll
+  for (int t = 0; t < VZ; ++t) cv[t] = 0.f;
+  if (near) dir_vec<VZ>(d, r.v0, cv, ncen);
 #pragma unroll
   for (int t = 0; t < VZ; ++t) c[t + 1] = cv[t];
   float lft = wave_from_prev(c[VZ]), rgt = wave_from_next(c[1]);  // see load_star
+  if (!own) return;
   if (lane == 0 && r.k0 > 0) lft = dir_at(d, r.v0 - 1);
   if (lane == 63 && r.k0 + VZ < n3) rgt = dir_at(d, r.v0 + VZ);
   c[0] = r.k0 > 0 ? lft : 0.f;
@@ -627,15 +673,17 @@ __global__ __launch_bounds__(kThreads) void npsd_dir_flat_kernel(FlatArgs a, con
        cid += (long)gridDim.x * kThreads) {
     Run<VZ> r;
     run_at<VZ>(cid, a.n1, a.n2, a.n3, r);
+    Codes<VZ> code;
+    code.load(a.code + r.v0, false);
     float c[VZ + 2], s[4][VZ], nv[VZ];
-    load_dir_star<VZ>(d, r, a.n1, a.n2, a.n3, c, s, nv);
-    float code[VZ], rv[VZ], wv[VZ], qn[VZ];
+    float rv[VZ], wv[VZ], qn[VZ];
     // single-use streams and outputs bypass L2 (the Q rows of the neighbourhood stay)
-    load_vec_nt<VZ>(a.code + r.v0, code);
-    load_vec_nt<VZ>(a.r + r.v0, rv);
+    if (code.own) load_vec_nt<VZ>(a.r + r.v0, rv);
+    load_dir_star<VZ>(d, r, a.n1, a.n2, a.n3, c, s, nv, code.own, code.near);
+    if (!code.own) continue;
 #pragma unroll
     for (int t = 0; t < VZ; ++t) {
-      const int cd = (int)code[t];
+      const int cd = (int)code.c[t];
       qn[t] = cd ? c[t + 1] : 0.f;
       wv[t] = cd ? lap_at<VZ, float>(c, s, t, cd) : 0.f;
       red[0] += (double)qn[t] * (double)wv[t];
@@ -681,8 +729,9 @@ __global__ __launch_bounds__(kFinThreads) void finalize_kernel(int op, int nr,
                                                                const double* __restrict__ partials,
                                                                unsigned nb, SolveState* st,
                                                                double* aux, const double* aux2) {
-  if (op != kFinResidInit && op != kFinDot && op != kFinDot2 && op != kFinDot2F32 && st->done)
-    return;  // uniform over the block
+  // fetched with the partials and the scalars, tested once they are summed: one memory latency
+  // instead of two (uniform over the block)
+  const bool skip = op != kFinResidInit && op != kFinDot && op != kFinDot2 && op != kFinDot2F32 && st->done;
   // thread 0 fetches the scalars it will read while the block sums the partials
   double rho = 0.0, rho_old = 0.0, norm_b = 0.0, tol = 0.0, atol = 0.0, cross = 0.0, an = 0.0, ao = 0.0;
   int iter = 0, max_it = 0, method = 0;
@@ -705,7 +754,7 @@ __global__ __launch_bounds__(kFinThreads) void finalize_kernel(int op, int nr,
   }
   double t[3] = {0.0, 0.0, 0.0};
   sum_partials_rows<3>(partials, nb, nr, t);
-  if (threadIdx.x != 0) return;
+  if (threadIdx.x != 0 || skip) return;
   switch (op) {
     case kFinResidInit:
     case kFinResid: {
@@ -794,36 +843,47 @@ int launch_flags_code(const int8_t* flags, uint8_t* code, int n1, int n2, int n3
   return check_launch("flags_code");
 }
 
+// The solver's star kernels take runs of at most 4 cells: one 16-byte load per vector and
+// lane, all of a wave's lines whole, and registers for 6 waves per SIMD and more (256^3 with
+// 55 % fluid: npsd_dir 74 us, resid 57 us; runs of 8: 79 and 63 us).
+static int star_vz(int n3) { return n3 % 4 == 0 ? 4 : (n3 % 2 == 0 ? 2 : 1); }
+// Workgroups: at most half of the partials' space.  More cost the finalize kernel 1.2 us and
+// gain nothing at 256^3; fewer (persistent ones, the codes of the next run fetched ahead)
+// measured no better.
 static unsigned flat_blocks(const FlatArgs& a) {
-  const int vz = flat_vz(a.n3);
-  return red_blocks((long)a.n1 * a.n2 * (a.n3 / vz));
+  const unsigned nb = red_blocks((long)a.n1 * a.n2 * (a.n3 / star_vz(a.n3)));
+  return nb < kMaxRedBlocks / 2 ? nb : kMaxRedBlocks / 2;
 }
 
-#define MLPCG_FLAT_DISPATCH(KERN, ITEMS_VZ, ...)                                                \
+#define MLPCG_FLAT_DISPATCH(KERN, ...)                                                          \
   do {                                                                                          \
-    const int vz_ = flat_vz(a.n3);                                                              \
-    const unsigned nb_ = red_blocks((long)a.n1 * a.n2 * (a.n3 / vz_));                          \
-    if (vz_ == 8) KERN<8><<<nb_, kThreads, 0, st>>>(__VA_ARGS__);                               \
-    else if (vz_ == 4) KERN<4><<<nb_, kThreads, 0, st>>>(__VA_ARGS__);                          \
-    else if (vz_ == 2) KERN<2><<<nb_, kThreads, 0, st>>>(__VA_ARGS__);                          \
-    else KERN<1><<<nb_, kThreads, 0, st>>>(__VA_ARGS__);                                        \
+    const int vz_ = star_vz(a.n3);                                                              \
+    const unsigned nb_ = flat_blocks(a);                                                        \
+    if (vz_ == 4) KERN(4)<<<nb_, kThreads, 0, st>>>(__VA_ARGS__);                               \
+    else if (vz_ == 2) KERN(2)<<<nb_, kThreads, 0, st>>>(__VA_ARGS__);                          \
+    else KERN(1)<<<nb_, kThreads, 0, st>>>(__VA_ARGS__);                                        \
   } while (0)
 
 int launch_resid_flat(const FlatArgs& a, int init, hipStream_t st) {
-  MLPCG_FLAT_DISPATCH(resid_flat_kernel, 0, a, init);
-  finalize(init ? kFinResidInit : kFinResid, 2, a.partials, flat_blocks(a), a.st, nullptr, st);
+#define MLPCG_RESID_INIT(VZ) resid_flat_kernel<VZ, true>
+#define MLPCG_RESID(VZ) resid_flat_kernel<VZ, false>
+  if (init) MLPCG_FLAT_DISPATCH(MLPCG_RESID_INIT, a);
+  else MLPCG_FLAT_DISPATCH(MLPCG_RESID, a);
+  finalize(init ? kFinResidInit : kFinResid, init ? 2 : 1, a.partials, flat_blocks(a), a.st, nullptr, st);
   return check_launch("resid_flat");
 }
 
 int launch_p_spmv_flat(const FlatArgs& a, hipStream_t st) {
-  MLPCG_FLAT_DISPATCH(p_spmv_flat_kernel, 0, a);
+#define MLPCG_PSPMV(VZ) p_spmv_flat_kernel<VZ>
+  MLPCG_FLAT_DISPATCH(MLPCG_PSPMV, a);
   finalize(kFinPW, 1, a.partials, flat_blocks(a), a.st, nullptr, st);
   return check_launch("p_spmv_flat");
 }
 
 int launch_npsd_dir_flat(const FlatArgs& a, const float* pN, double* alfa_out,
                          hipStream_t st) {
-  MLPCG_FLAT_DISPATCH(npsd_dir_flat_kernel, 0, a, pN);
+#define MLPCG_NPSD_DIR(VZ) npsd_dir_flat_kernel<VZ>
+  MLPCG_FLAT_DISPATCH(MLPCG_NPSD_DIR, a, pN);
   finalize(kFinNpsd, 3, a.partials, flat_blocks(a), a.st, alfa_out, st);
   return check_launch("npsd_dir_flat");
 }

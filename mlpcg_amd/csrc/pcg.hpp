@@ -36,6 +36,9 @@ struct FlatArgs {
   SolveState* st;
   double* partials;
   int n1, n2, n3;
+  // resid: x_new may hold nonzeros off the fluid (a caller's x0), so it is written everywhere;
+  // the other outputs, and x_new otherwise, are zero there and only written in runs with fluid
+  int full_x;
 };
 
 struct CsrArgs {

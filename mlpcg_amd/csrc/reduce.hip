@@ -37,25 +37,6 @@ struct PatchSums {
   double t[C][27];
 };
 
-// sum over the wave by DPP row shifts and row broadcasts; valid in lane 63
-__device__ __forceinline__ double wave_sum_dpp(double v) {
-  auto step = [](double x, auto ctrl, auto rows) {
-    constexpr int kCtrl = decltype(ctrl)::value, kRows = decltype(rows)::value;
-    const long long u = __builtin_bit_cast(long long, x);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)u, kCtrl, kRows, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), kCtrl, kRows, 0xf, false);
-    return x + __builtin_bit_cast(double, ((long long)(unsigned)hi << 32) | (unsigned)lo);
-  };
-  typedef std::integral_constant<int, 0xf> All;
-  v = step(v, std::integral_constant<int, 0x111>(), All());  // row_shr 1, 2, 4, 8
-  v = step(v, std::integral_constant<int, 0x112>(), All());
-  v = step(v, std::integral_constant<int, 0x114>(), All());
-  v = step(v, std::integral_constant<int, 0x118>(), All());
-  v = step(v, std::integral_constant<int, 0x142>(), std::integral_constant<int, 0xa>());  // row_bcast 15
-  v = step(v, std::integral_constant<int, 0x143>(), std::integral_constant<int, 0xc>());  // row_bcast 31
-  return v;
-}
-
 template <typename TI, int C, int VZ>
 __device__ __forceinline__ void patch_accumulate(const TI* __restrict__ img, int n1, int n2, int n3, unsigned first,
                                                  unsigned stride, PatchSums<C>& p) {

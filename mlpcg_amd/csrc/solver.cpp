@@ -161,6 +161,7 @@ int Solver::solve(Precond* P, const float* b, const float* x0, float* x_out, int
   fa0.n1 = n1;
   fa0.n2 = n2;
   fa0.n3 = n3;
+  fa0.full_x = x0 != nullptr || use_graphs;  // a graph captured without x0 may be replayed with it
   CsrArgs ca0;
   memset(&ca0, 0, sizeof(ca0));
   ca0.rowptr = rowptr;
