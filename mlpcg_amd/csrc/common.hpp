@@ -124,6 +124,23 @@ __device__ __forceinline__ unsigned xcd_block(unsigned bid, unsigned nblk) {
   return base + slot;
 }
 
+// Idle tiles of a solver's grid: idle[i0 / 2][j0 / 8][z0 / 64] = 1 if no cell of the 2 x 8 x 64
+// tile and its one-cell halo is fluid (launch_idle_tiles).  The solver's vectors are zero there,
+// so a tile of FI planes whose entries are all set has a zero input and a cleared output, and
+// zeros are all a block writes.  (Infinite weights or image values, which would make NaN of the
+// zeros, also make the level's coefficients, or every tile with fluid, non-finite.)
+template <int FI>
+__device__ __forceinline__ bool tile_is_idle(const uint8_t* idle, int i0, int j0, int z0, int n1, int n2, int n3) {
+  if (!idle) return false;
+  const int tj = (n2 + 7) / 8, tz = (n3 + 63) / 64, ti = (n1 + 1) / 2;
+  bool all = true;
+#pragma unroll
+  for (int u = 0; u < FI / 2; ++u) {
+    const int t = i0 / 2 + u;
+    if (t < ti) all = all && idle[((long)t * tj + j0 / 8) * tz + z0 / 64] != 0;
+  }
+  return all;
+}
 // ---------------------------------------------------------------------------
 // Wavefront / block reductions (64-lane wavefronts).
 // ---------------------------------------------------------------------------

@@ -61,6 +61,9 @@ struct FusedArgs {
   // optional (BF16 output, no epilogue operands): also write the 2x2x2 means of y, the
   // next level's input, as avgpool2 computes them (same sums in the same order)
   void* pool_out;
+  // optional: idle tiles (launch_idle_tiles) of the grid x and mask_b belong to; x must be zero
+  // where the fluid is not, and mask_b, if given, the fluid
+  const uint8_t* idle;
   int n1, n2, n3;
 };
 

@@ -48,6 +48,25 @@ __global__ __launch_bounds__(kThreads) void flags_code_kernel(const int8_t* __re
   code[v] = (uint8_t)(1 + d);
 }
 
+// One workgroup per tile of 2 x 8 x 64 cells (29 us at 256^3, once per solver).
+__global__ __launch_bounds__(kThreads) void idle_tiles_kernel(const uint8_t* __restrict__ code,
+                                                              uint8_t* __restrict__ idle, int n1, int n2, int n3) {
+  const int tj = (n2 + 7) / 8, tz = (n3 + 63) / 64;
+  const unsigned t = xcd_block(blockIdx.x, gridDim.x);
+  const int z0 = (int)(t % tz) * 64, j0 = (int)(t / tz % tj) * 8, i0 = (int)(t / tz / tj) * 2;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  unsigned any = 0;
+#pragma unroll
+  for (int k = 0; k < 10; ++k) {  // clamped: a cell outside reads its neighbour inside, one of the tile's too
+    const int q = w + 4 * k, i = min(max(i0 - 1 + q / 10, 0), n1 - 1), j = min(max(j0 - 1 + q % 10, 0), n2 - 1);
+    const uint8_t* row = code + ((long)i * n2 + j) * n3;
+    any |= row[min(max(z0 - 1 + lane, 0), n3 - 1)];
+    any |= row[min(z0 + 63 + (lane & 1), n3 - 1)];
+  }
+  const int some = __syncthreads_or((int)any);
+  if (threadIdx.x == 0) idle[t] = some ? 0 : 1;
+}
+
 // ---------------------------------------------------------------------------
 // Flat stencil helpers: a thread owns a z-run of VZ voxels.
 // ---------------------------------------------------------------------------
@@ -841,6 +860,17 @@ int launch_flags_code(const int8_t* flags, uint8_t* code, int n1, int n2, int n3
   flags_code_kernel<<<(unsigned)((V + kThreads - 1) / kThreads), kThreads, 0, st>>>(flags, code, n1,
                                                                                      n2, n3);
   return check_launch("flags_code");
+}
+
+size_t idle_tiles_bytes(int n1, int n2, int n3) {
+  return (size_t)((n1 + 1) / 2) * (size_t)((n2 + 7) / 8) * (size_t)((n3 + 63) / 64);
+}
+
+int launch_idle_tiles(const uint8_t* code, uint8_t* idle, int n1, int n2, int n3, hipStream_t st) {
+  const size_t nb = idle_tiles_bytes(n1, n2, n3);
+  MLPCG_REQUIRE(nb < (1UL << 31), "idle_tiles: grid (%d,%d,%d) too large", n1, n2, n3);
+  idle_tiles_kernel<<<(unsigned)nb, kThreads, 0, st>>>(code, idle, n1, n2, n3);
+  return check_launch("idle_tiles");
 }
 
 // The solver's star kernels take runs of at most 4 cells: one 16-byte load per vector and

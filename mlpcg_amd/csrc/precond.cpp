@@ -215,9 +215,10 @@ int Precond::update(const void* image, const void* const* weights, const void* c
 int Precond::run_block(int k, int level, const void* x, int tx, void* y, int ty, const void* prev,
                        const void* c0, const void* c1, const uint8_t* ma, const uint8_t* mb,
                        const double* sc, const int* done, hipStream_t st, const float* dot0,
-                       const float* dot1, double* partials, void* pool_out) {
+                       const float* dot1, double* partials, void* pool_out, const uint8_t* idle) {
   if (blocks[k].fused) {
     FusedArgs f;
+    f.idle = idle;
     f.pool_out = pool_out;
     f.dot0 = dot0;
     f.dot1 = dot1;
@@ -292,7 +293,7 @@ int Precond::apply_block(int k, const void* x, int tx, void* y, int ty, const do
 
 int Precond::apply(const float* r_in, float* z_out, const double* in_scale, const uint8_t* out_mask,
                    const int* done, hipStream_t st, const float* dot0, const float* dot1,
-                   double* partials, unsigned* dot_blocks) {
+                   double* partials, unsigned* dot_blocks, const uint8_t* idle) {
   if (dot_blocks) *dot_blocks = 0;
   const int vdt = dtype == kF64 ? kF64 : kF32;  // type of the solver-side vectors
   const size_t as = dsize(acc);
@@ -341,7 +342,7 @@ int Precond::apply(const float* r_in, float* z_out, const double* in_scale, cons
     return (pooled && (blocks[i].fused || blocks[i].split) && !(i == 0 && mask)) ? tmp[i + 1] : nullptr;
   };
   TRY(run_block(0, 0, r_in, vdt, xd[0], dtype, nullptr, nullptr, nullptr, mask ? maskimg : nullptr, nullptr,
-                in_scale, done, st, nullptr, nullptr, nullptr, pool_into(0)));
+                in_scale, done, st, nullptr, nullptr, nullptr, pool_into(0), idle));
   for (int i = 1; i < ndown; ++i) {
     if (!pool_into(i - 1)) TRY(pool(xd[i - 1], tmp[i], i - 1));
     TRY(run_block(i, i, tmp[i], dtype, xd[i], dtype, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, done,
@@ -386,7 +387,7 @@ int Precond::apply(const float* r_in, float* z_out, const double* in_scale, cons
         if (nb && dot0 && partials && dot_blocks && 2L * nb <= reduction_capacity()) {
           // the solver's dot products on z ride in the epilogue of the last block
           TRY(run_block(n, 0, tmp[0], dtype, y, ty, xd[0], c0p(0, 0), c1p(0, 0), ma, mb, nullptr, done, st,
-                        dot0, dot1, partials));
+                        dot0, dot1, partials, nullptr, out_mask ? idle : nullptr));
           *dot_blocks = nb;
           cur = xo[lvl];
           continue;

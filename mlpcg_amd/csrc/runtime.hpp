@@ -56,17 +56,19 @@ struct Precond {
              hipStream_t st);
   // z = P(r * in_scale).  With dot0 (and optionally dot1) and partials, a plan whose last
   // block is fused also writes per-block partial sums [2][*dot_blocks] of z.dot0, z.dot1
-  // (flat layout); *dot_blocks = 0 means they were not computed.
+  // (flat layout); *dot_blocks = 0 means they were not computed.  idle: tiles without fluid
+  // (launch_idle_tiles) of the grid whose fluid out_mask marks; r is zero off the fluid.
   int apply(const float* r, float* z, const double* in_scale, const uint8_t* out_mask,
             const int* done, hipStream_t st, const float* dot0 = nullptr,
             const float* dot1 = nullptr, double* partials = nullptr,
-            unsigned* dot_blocks = nullptr);
+            unsigned* dot_blocks = nullptr, const uint8_t* idle = nullptr);
   int apply_block(int k, const void* x, int tx, void* y, int ty, const double* in_scale,
                   hipStream_t st);
   int run_block(int k, int level, const void* x, int tx, void* y, int ty, const void* prev,
                 const void* c0, const void* c1, const uint8_t* ma, const uint8_t* mb,
                 const double* sc, const int* done, hipStream_t st, const float* dot0 = nullptr,
-                const float* dot1 = nullptr, double* partials = nullptr, void* pool_out = nullptr);
+                const float* dot1 = nullptr, double* partials = nullptr, void* pool_out = nullptr,
+                const uint8_t* idle = nullptr);
   ~Precond();
 };
 
@@ -99,6 +101,7 @@ struct Solver {
   int n1 = 0, n2 = 0, n3 = 0;
   long V = 0, n = 0;
   uint8_t* code = nullptr;
+  uint8_t* idle = nullptr;  // tiles without fluid; null on small grids
   const int* rowptr = nullptr;
   const int* col = nullptr;
   const float* val = nullptr;

@@ -80,6 +80,16 @@ int solver_create_flat(Solver** out, const int8_t* flags, int n1, int n2, int n3
     delete S;
     return -1;
   }
+  // grids of the BF16 matrix-core tiles (smaller ones have few tiles to leave out)
+  if (S->V > (1L << 18) && n1 % 8 == 0 && n2 % 8 == 0 && n3 % 64 == 0) {
+    void* idle = nullptr;
+    if (salloc(S, &idle, idle_tiles_bytes(n1, n2, n3), false, st) ||
+        launch_idle_tiles(S->code, (uint8_t*)idle, n1, n2, n3, st)) {
+      delete S;
+      return -1;
+    }
+    S->idle = (uint8_t*)idle;
+  }
   *out = S;
   return 0;
 }
@@ -201,7 +211,7 @@ int Solver::solve(Precond* P, const float* b, const float* x0, float* x_out, int
       return 0;
     }
     const double* scale = &this->st->scale;
-    if (layout == 0) return P->apply(rin, zout, scale, code, done, s, dot0, dot1, partials, nbd);
+    if (layout == 0) return P->apply(rin, zout, scale, code, done, s, dot0, dot1, partials, nbd, idle);
     int rc2 = launch_scatter(fluid_idx, rin, grid_in, n, done, s);
     if (rc2) return rc2;
     rc2 = P->apply(grid_in, grid_out, scale, nullptr, done, s);
