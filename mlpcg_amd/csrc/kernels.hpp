@@ -76,12 +76,6 @@ int launch_sm_fused(int tw, int tx, int ty, int C, const FusedArgs& a, hipStream
 // The stencils K of the fused apply's first product (a.img, a.apack, a.n1..n3), stored as
 // BF16 [27][V] (the stored-stencil layout) instead of applied.
 int launch_fused_kwrite(int C, const FusedArgs& a, void* K, hipStream_t st);
-// Input gradient of a BF16 block (no transpose) through the nine column sums S of
-// P_p(v) = g(v) K_p(v) (g in a.x, BF16; K from the first product): dx(u) = sum_c S_c(u + d_c)
-// on the matrix-core grids of the fused apply.  work: fused_sgrad_bytes() bytes.
-size_t fused_sgrad_bytes(int n1, int n2, int n3);
-int launch_fused_sgrad(int C, const FusedArgs& a, void* work, void* dx, hipStream_t st);
-
 // FP32 blocks on the matrix cores (split.hpp): K recomputed from the FP32 image img [C][V]
 // and the packed weights (launch_split_pack), applied to x [B][V] with the epilogue of
 // ApplyArgs; any grid whose planes are under 2^31 bytes (split_eligible).
@@ -110,6 +104,12 @@ bool split_eligible(int C, int n1, int n2, int n3);
 unsigned split_blocks(int C, int n1, int n2, int n3);
 int launch_split_pack(const void* W, const void* b, int C, void* pack, hipStream_t st);
 int launch_sm_split(int C, const SplitArgs& a, hipStream_t st);
+// Its input gradient (igrad.hpp), FP32 or BF16 vectors and image: dx [B][V] from g [B][V], image
+// and packed weights as above; work: `bytes` bytes, fused_sgrad_bytes() (the FP32 sums of one
+// right-hand side) or more.
+size_t fused_sgrad_bytes(int n1, int n2, int n3);
+int launch_igrad(int dtype, const void* img, const void* pack, const void* g, void* dx, void* work, size_t bytes, int C,
+                 int B, int n1, int n2, int n3, hipStream_t st);
 
 // The two coarsest levels of the SmallSM V-cycle in one workgroup (tail.hip): from the
 // output x_in of pre[n-2] (level n-2 grid) to up(c0 x + c1 post[n-1](up(l(pool(x))))) on

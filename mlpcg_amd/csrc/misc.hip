@@ -3,6 +3,7 @@
 #include "kernels.hpp"
 #include "split.hpp"
 #include "wgrad.hpp"
+#include "igrad.hpp"
 
 namespace mlpcg {
 

@@ -24,7 +24,7 @@
 // grid, so any extents are taken.  A wave takes one row of 64 voxels at a time (a chunk) as
 // two groups of 32 of one z parity: lane (h, n) = (lane / 32, lane % 32) works on voxels
 // z = 2n and 2n + 1.  The 27 taps, as 9 columns (d1, d2) of three, go to the two lane
-// halves, columns 0..4 and 5..8: per column the two aligned words w0 = cells 2n - 1, 2n and
+// halves, columns 0..4 and 6, 7, 8, 5: per column the two aligned words w0 = cells 2n - 1, 2n and
 // w1 = 2n + 1, 2n + 2 hold all three taps of both voxels.
 // Operands (lane l, element j / i): A[l % 32][8 (l / 32) + j], B[8 (l / 32) + j][l % 32],
 // D[8 (i / 4) + 4 (l / 32) + i % 4][l % 32].  A = W, B = image patches; the rows of D are
@@ -50,8 +50,9 @@ constexpr int kTarget = 4;      // largest |W| and |img| are scaled into [2^4, 2
 constexpr int kBiasTarget = 8;  // and the largest scaled bias stays below 2^9
 
 
-// column i (0..4) of lane half h; the fifth of the upper half is a dummy (zero weights)
-__host__ __device__ constexpr int col_of(int h, int i) { return h == 0 ? i : (i < 4 ? 5 + i : 8); }
+// column i (0..4) of lane half h; the fifth of the upper half is a dummy (zero weights).  The
+// first three are a plane's (d1 = -1, +1), which the input gradient (igrad.hpp) relies on.
+__host__ __device__ constexpr int col_of(int h, int i) { return h == 0 ? i : (i < 3 ? 6 + i : i == 3 ? 5 : 8); }
 __host__ __device__ constexpr bool col_real(int h, int i) { return h == 0 || i < 4; }
 
 struct PackHeader {
@@ -82,15 +83,17 @@ __host__ __device__ constexpr int reg_tap(int h, int i) {
   return i < 15 && col_real(h, i / 3) ? 3 * col_of(h, i / 3) + i % 3 : -1;
 }
 
-// One workgroup per 2048 packed values; every workgroup scans the weights for their scale.
+// One workgroup per 512 packed values; every workgroup scans the weights for their scale.
 __global__ __launch_bounds__(kThreads) void split_pack_kernel(const float* __restrict__ W, const float* __restrict__ b,
                                                               int C, char* __restrict__ out) {
   __shared__ unsigned sh[3][4];
   unsigned mw = 0, mb = 0, bad = 0;
-  for (int e = threadIdx.x; e < 27 * 27 * C; e += kThreads) {
-    const unsigned u = finite_bits(W[e]);
+#pragma unroll
+  for (int k = 0; k < 9; ++k) {  // C <= 3; clamped, so that all loads are in flight together
+    const float v = W[min(k * kThreads + (int)threadIdx.x, 27 * 27 * C - 1)];
+    const unsigned u = finite_bits(v);
     mw = mw > u ? mw : u;
-    bad |= (__float_as_uint(W[e]) & 0x7f800000u) == 0x7f800000u;
+    bad |= (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u;
   }
   if (threadIdx.x < 27) {
     mb = finite_bits(b[threadIdx.x]);
@@ -115,7 +118,9 @@ __global__ __launch_bounds__(kThreads) void split_pack_kernel(const float* __res
   const int nw = (int)(pack_w_bytes(C) / sizeof(f16));
   f16* __restrict__ wp = (f16*)(out + kHeaderBytes);
   float* __restrict__ bp = (float*)(out + kHeaderBytes + pack_w_bytes(C));
-  for (int e = blockIdx.x * 2048 + threadIdx.x; e < min(nw, (int)(blockIdx.x + 1) * 2048); e += kThreads) {
+  #pragma unroll
+  for (int k = 0; k < 2; ++k) {
+    const int e = blockIdx.x * 512 + k * kThreads + threadIdx.x;  // nw is a multiple of 512
     const int j = e % 8, lane = (e / 8) % 64, c = (e / 512) % C, kc = (e / (512 * C)) % 2;
     const int part = (e / (1024 * C)) % 2, par = e / (2048 * C);
     const int m = lane & 31;  // row of D: register i of lane half h
@@ -155,8 +160,9 @@ __device__ __forceinline__ float halves_sum(float a, float b) {
 __device__ __forceinline__ unsigned both_lo(unsigned a, unsigned b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }
 __device__ __forceinline__ unsigned both_hi(unsigned a, unsigned b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
 
-__host__ __device__ constexpr int tile_rows(int FI) { return (FI + 2) * kPJ; }
-__host__ __device__ constexpr int tile_cells(int FI) { return tile_rows(FI) * kPitch; }
+// PJ: staged rows per plane, halo included
+__host__ __device__ constexpr int tile_rows(int FI, int PJ = kPJ) { return (FI + 2) * PJ; }
+__host__ __device__ constexpr int tile_cells(int FI, int PJ = kPJ) { return tile_rows(FI, PJ) * kPitch; }
 
 // Position of a tile: the grid's tiles in z, then j, then i order (XCD-contiguous), z rotated
 // from row to row of tiles: workgroups go to the shader engines in turn, and the cheap tiles
@@ -171,57 +177,58 @@ __device__ __forceinline__ Tile tile_at(int n2, int n3) {
   return Tile{(int)(u / tj) * FI, (int)(u % tj) * kJ, (int)((t + u) % tz) * kZ};
 }
 
-// Raw FP32 cells of a staged tile: rows w, w + 4, ... of the wave, cell z0 + lane of each,
+// Raw cells of a staged tile as FP32: rows w, w + 4, ... of the wave, cell z0 + lane of each,
 // and one z-halo cell of the whole tile per thread (rows' cells z0 - 1 and z0 + 64).
-template <int FI>
+template <int FI, int PJ = kPJ>
 struct Raw {
-  static constexpr int kRows = (tile_rows(FI) + 3) / 4;
+  static constexpr int kRows = (tile_rows(FI, PJ) + 3) / 4;
+  static_assert(2 * tile_rows(FI, PJ) <= kThreads, "one halo cell per thread");
   float m[kRows];
   float halo;
 };
 
-template <int FI>
-__device__ __forceinline__ void load_raw(Raw<FI>& r, const float* __restrict__ src, const Tile& t, int n1, int n2,
+template <int FI, int PJ, typename T>
+__device__ __forceinline__ void load_raw(Raw<FI, PJ>& r, const T* __restrict__ src, const Tile& t, int n1, int n2,
                                          int n3, int w, int lane) {
   const long plane = (long)n2 * n3;
-  const int pb = (int)(plane * 4), rb = n3 * 4;
-  const unsigned zo = t.z0 + lane < n3 ? (unsigned)(t.z0 + lane) * 4u : 0x80000000u;
+  const int pb = (int)(plane * (int)sizeof(T)), rb = n3 * (int)sizeof(T);
+  const unsigned zo = t.z0 + lane < n3 ? (unsigned)(t.z0 + lane) * (unsigned)sizeof(T) : 0x80000000u;
 #pragma unroll
-  for (int k = 0; k < Raw<FI>::kRows; ++k) {
+  for (int k = 0; k < Raw<FI, PJ>::kRows; ++k) {
     const int row = w + 4 * k;
-    const int gi = t.i0 + row / kPJ - 1, gj = t.j0 + row % kPJ - 1;
-    const bool ok = row < tile_rows(FI) && (unsigned)gi < (unsigned)n1 && (unsigned)gj < (unsigned)n2;
+    const int gi = t.i0 + row / PJ - 1, gj = t.j0 + row % PJ - 1;
+    const bool ok = row < tile_rows(FI, PJ) && (unsigned)gi < (unsigned)n1 && (unsigned)gj < (unsigned)n2;
     r.m[k] = ld_as(rsrc(src + (ok ? gi : 0) * plane, ok ? pb : 0), zo, (ok ? gj : 0) * rb, src);
   }
   const int hrow = threadIdx.x >> 1, z = (threadIdx.x & 1) ? t.z0 + kZ : t.z0 - 1;
-  const int gi = t.i0 + hrow / kPJ - 1, gj = t.j0 + hrow % kPJ - 1;
-  const bool ok = hrow < tile_rows(FI) && (unsigned)gi < (unsigned)n1 && (unsigned)gj < (unsigned)n2 &&
+  const int gi = t.i0 + hrow / PJ - 1, gj = t.j0 + hrow % PJ - 1;
+  const bool ok = hrow < tile_rows(FI, PJ) && (unsigned)gi < (unsigned)n1 && (unsigned)gj < (unsigned)n2 &&
                   (unsigned)z < (unsigned)n3;
-  r.halo = ok ? src[((long)gi * n2 + gj) * n3 + z] : 0.f;
+  r.halo = ok ? (float)src[((long)gi * n2 + gj) * n3 + z] : 0.f;
 }
 
-template <int FI, typename F>
-__device__ __forceinline__ void each_cell(const Raw<FI>& r, int w, int lane, F&& f) {
+template <int FI, int PJ, typename F>
+__device__ __forceinline__ void each_cell(const Raw<FI, PJ>& r, int w, int lane, F&& f) {
 #pragma unroll
-  for (int k = 0; k < Raw<FI>::kRows; ++k)
-    if (w + 4 * k < tile_rows(FI)) f((w + 4 * k) * kPitch + 1 + lane, r.m[k]);
-  if ((int)(threadIdx.x >> 1) < tile_rows(FI)) f((threadIdx.x >> 1) * kPitch + (threadIdx.x & 1) * (kZ + 1), r.halo);
+  for (int k = 0; k < Raw<FI, PJ>::kRows; ++k)
+    if (w + 4 * k < tile_rows(FI, PJ)) f((w + 4 * k) * kPitch + 1 + lane, r.m[k]);
+  if ((int)(threadIdx.x >> 1) < tile_rows(FI, PJ)) f((threadIdx.x >> 1) * kPitch + (threadIdx.x & 1) * (kZ + 1), r.halo);
 }
 
 // The image tile of C channels as two FP16 arrays hi, lo [C][cells].  Returns (uniform) the
-// exponent of the tile's factor; flags: any non-finite cell, any nonzero lo.  Ends in a
-// barrier; sh: 8 words of LDS.
+// exponent of the tile's factor; flags: any non-finite cell, any nonzero lo (LO = false: the
+// image is of a type that hi holds, lo is left out).  Ends in a barrier; sh: 8 words of LDS.
 struct ImageTile {
   int exp;
   bool nonfinite, has_lo;
 };
-template <int C, int FI>
-__device__ __forceinline__ ImageTile stage_image(const Raw<FI> (&raw)[C], int limit, int w, int lane, f16* hi, f16* lo,
+template <int C, int FI, int PJ = kPJ, bool LO = true>
+__device__ __forceinline__ ImageTile stage_image(const Raw<FI, PJ> (&raw)[C], int limit, int w, int lane, f16* hi, f16* lo,
                                                  unsigned* sh) {
   unsigned m = 0, bad = 0;
 #pragma unroll
   for (int c = 0; c < C; ++c)
-    each_cell<FI>(raw[c], w, lane, [&](int, float v) {
+    each_cell<FI, PJ>(raw[c], w, lane, [&](int, float v) {
       const unsigned u = __float_as_uint(v) & 0x7fffffffu;
       const bool fin = u < 0x7f800000u;
       m = max(m, fin ? u : 0u);
@@ -243,13 +250,21 @@ __device__ __forceinline__ ImageTile stage_image(const Raw<FI> (&raw)[C], int li
   unsigned any = 0;
 #pragma unroll
   for (int c = 0; c < C; ++c)
-    each_cell<FI>(raw[c], w, lane, [&](int e, float v) {
+    each_cell<FI, PJ>(raw[c], w, lane, [&](int e, float v) {
       const float sv = v * s;
-      const f16 h = (f16)sv, l = (f16)(sv - (float)h);
-      hi[c * tile_cells(FI) + e] = h;
-      lo[c * tile_cells(FI) + e] = l;
-      any |= __builtin_bit_cast(unsigned short, l) & 0x7fffu;
+      const f16 h = (f16)sv;
+      hi[c * tile_cells(FI, PJ) + e] = h;
+      if (LO) {
+        const f16 l = (f16)(sv - (float)h);
+        lo[c * tile_cells(FI, PJ) + e] = l;
+        any |= __builtin_bit_cast(unsigned short, l) & 0x7fffu;
+      }
     });
+  if (!LO) {
+    it.has_lo = false;
+    __syncthreads();
+    return it;
+  }
   any = __builtin_amdgcn_ballot_w64(any != 0) != 0;
   __syncthreads();  // the flags above were read by everyone
   if (lane == 0) sh[w] = any;
@@ -259,15 +274,17 @@ __device__ __forceinline__ ImageTile stage_image(const Raw<FI> (&raw)[C], int li
 }
 
 // A lane's packed weights, and the first product of one chunk for one z parity.
-template <int C>
+// WL = false: hi alone (11 bits, for results of 8; the bias keeps 22).
+template <int C, bool WL = true>
 struct Weights {
-  h8 w[2][2][2][C];  // [parity][hi, lo][k half][channel]
+  static constexpr int kParts = WL ? 2 : 1;
+  h8 w[2][kParts][2][C];  // [parity][hi, lo][k half][channel]
   __device__ __forceinline__ void load(const void* pack, int lane) {
     const f16* p = (const f16*)((const char*)pack + kHeaderBytes);
 #pragma unroll
     for (int par = 0; par < 2; ++par)
 #pragma unroll
-      for (int part = 0; part < 2; ++part)
+      for (int part = 0; part < kParts; ++part)
 #pragma unroll
         for (int kc = 0; kc < 2; ++kc)
 #pragma unroll
@@ -280,20 +297,22 @@ struct Weights {
     const f16 hi = (f16)b, lo = (f16)(b - (float)hi), rest = (f16)(b - (float)hi - (float)lo);
 #pragma unroll
     for (int par = 0; par < 2; ++par) {
-      w[par][0][1][0][spare_slot(par)] = h == 0 ? hi : rest;
-      w[par][1][1][0][spare_slot(par)] = h == 0 ? lo : (f16)0.f;
+      w[par][0][1][0][spare_slot(par)] = h == 0 ? hi : WL ? rest : lo;
+      if constexpr (WL) w[par][1][1][0][spare_slot(par)] = h == 0 ? lo : (f16)0.f;
     }
   }
 };
 
-// byte offsets of the lane's columns' words in a tile of 2-byte cells, at chunk (0, wave row)
+// byte offsets of the lane's columns' words in a tile of 2-byte cells, at the wave's first chunk
+// (row: its staged row less the halo)
 struct WordBase {
   unsigned b0[5], b1[5];
-  __device__ __forceinline__ void init(int h, int n, int w) {
+  template <int PJ = kPJ>
+  __device__ __forceinline__ void init(int h, int n, int row) {
 #pragma unroll
     for (int i = 0; i < 5; ++i) {
       const int c = h == 0 ? col_of(0, i) : col_of(1, i);
-      b0[i] = (unsigned)((((c / 3) * kPJ + c % 3 + w) * kPitch + 2 * n) * 2);
+      b0[i] = (unsigned)((((c / 3) * PJ + c % 3 + row) * kPitch + 2 * n) * 2);
       b1[i] = b0[i] + 4;
       // opaque, so that no two reads are merged into one that needs an address of its own
       asm volatile("" : "+v"(b0[i]), "+v"(b1[i]));
@@ -316,8 +335,8 @@ __device__ __forceinline__ void operands(const f16* arr, const WordBase& wb, int
   b[1][1] = __builtin_bit_cast(h8, u32x4s{o4, both_hi(e[0], e[1]), both_hi(e[2], e[3]), (e4 & 0xffff0000u) | one_lo});
 }
 // scaled K of the lane's columns for both parities, from the tile at `cell`
-template <int C, bool LO>
-__device__ __forceinline__ void stencils(const Weights<C>& W, const f16* hi, const f16* lo, int cells,
+template <int C, bool LO, bool WL>
+__device__ __forceinline__ void stencils(const Weights<C, WL>& W, const f16* hi, const f16* lo, int cells,
                                          const WordBase& wb, int cell, f16x (&K)[2]) {
 #pragma unroll
   for (int c = 0; c < C; ++c) {
@@ -330,7 +349,8 @@ __device__ __forceinline__ void stencils(const Weights<C>& W, const f16* hi, con
 #pragma unroll
       for (int kc = 0; kc < 2; ++kc) {
         const f16x in = c == 0 && kc == 0 ? f16x{} : K[par];
-        K[par] = __builtin_amdgcn_mfma_f32_32x32x16_f16(W.w[par][1][kc][c], bh[par][kc], in, 0, 0, 0);
+        if constexpr (WL) K[par] = __builtin_amdgcn_mfma_f32_32x32x16_f16(W.w[par][1][kc][c], bh[par][kc], in, 0, 0, 0);
+        else K[par] = in;
         if (LO) K[par] = __builtin_amdgcn_mfma_f32_32x32x16_f16(W.w[par][0][kc][c], bl[par][kc], K[par], 0, 0, 0);
         K[par] = __builtin_amdgcn_mfma_f32_32x32x16_f16(W.w[par][0][kc][c], bh[par][kc], K[par], 0, 0, 0);
       }
@@ -361,10 +381,10 @@ void sm_split_kernel(SplitArgs a) {
 
   Raw<FI> rx[BB], ri[C];
 #pragma unroll
-  for (int c = 0; c < C; ++c) load_raw<FI>(ri[c], a.img + c * V, t, a.n1, a.n2, a.n3, w, lane);
+  for (int c = 0; c < C; ++c) load_raw<FI, kPJ>(ri[c], a.img + c * V, t, a.n1, a.n2, a.n3, w, lane);
 #pragma unroll
   for (int bb = 0; bb < BB; ++bb)
-    if (BB == 1 || b0 + bb < a.B) load_raw<FI>(rx[bb], a.x + (long)(b0 + bb) * V, t, a.n1, a.n2, a.n3, w, lane);
+    if (BB == 1 || b0 + bb < a.B) load_raw<FI, kPJ>(rx[bb], a.x + (long)(b0 + bb) * V, t, a.n1, a.n2, a.n3, w, lane);
   const PackHeader* hd = (const PackHeader*)a.pack;
   const float scale = a.in_scale ? (float)(*a.in_scale) : 1.f;
   const float c0 = a.prev ? *a.c0 : 0.f, c1 = a.prev ? *a.c1 : 0.f;
@@ -373,7 +393,7 @@ void sm_split_kernel(SplitArgs a) {
 #pragma unroll
   for (int bb = 0; bb < BB; ++bb) {
     if (BB > 1 && b0 + bb >= a.B) break;
-    each_cell<FI>(rx[bb], w, lane, [&](int e, float v) {
+    each_cell<FI, kPJ>(rx[bb], w, lane, [&](int e, float v) {
       xs[bb][e] = v;
       xany |= __float_as_uint(v) & 0x7fffffffu;
     });
@@ -436,7 +456,7 @@ void sm_split_kernel(SplitArgs a) {
       const bool skip = zero || (LB && has_b && __builtin_amdgcn_ballot_w64(zok && kb != 0) == 0);
       if (!skip) {
         f16x K[2];
-        stencils<C, LO>(W, ih, il, kCells, wb, cell, K);
+        stencils<C, LO, true>(W, ih, il, kCells, wb, cell, K);
 #pragma unroll
         for (int bb = 0; bb < BB; ++bb) {
           float pe = 0.f, po = 0.f;
@@ -550,7 +570,7 @@ unsigned split_blocks(int C, int n1, int n2, int n3) {
 
 int launch_split_pack(const void* W, const void* b, int C, void* pack, hipStream_t st) {
   MLPCG_REQUIRE(C >= 1 && C <= 3, "split_pack: C must be 1, 2 or 3 (got %d)", C);
-  split::split_pack_kernel<<<2 * C, kThreads, 0, st>>>((const float*)W, (const float*)b, C, (char*)pack);
+  split::split_pack_kernel<<<8 * C, kThreads, 0, st>>>((const float*)W, (const float*)b, C, (char*)pack);
   return check_launch("split_pack");
 }
 
