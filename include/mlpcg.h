@@ -247,7 +247,8 @@ void mlpcg_precond_destroy(mlpcg_precond* P);
  *     transposed) recompute K on the matrix cores inside the apply instead of storing it.
  *     0: never (K stored like every other block); 1: on such grids of at least 2^18
  *     voxels (smaller ones are faster with stored K); 2: on every such grid.  With 1 and 2
- *     FP32 blocks (not transposed) above 2^18 voxels recompute K too, any extents.  Plus 4
+ *     FP32 blocks (not transposed) above 2^18 voxels recompute K too, any extents (with 1 and
+ *     C > 1 from 2^21 on).  Plus 4
  *     (C = 3 only): the image's third channel is the sum of the first two (the
  *     [air, fluid, non-solid] images), so the fused blocks take two channels with the third
  *     channel's weights added to the others' -- the caller vouches for the relation.

@@ -743,48 +743,42 @@ enum FinOp : int {
 };
 
 // aux/aux2: the output of kFinDot; alfa of N and O for kFinProj; alfa of the new
-// direction for kFinNpsd.
-__global__ __launch_bounds__(kFinThreads) void finalize_kernel(int op, int nr,
-                                                               const double* __restrict__ partials,
-                                                               unsigned nb, SolveState* st,
-                                                               double* aux, const double* aux2) {
-  // fetched with the partials and the scalars, tested once they are summed: one memory latency
-  // instead of two (uniform over the block)
-  const bool skip = op != kFinResidInit && op != kFinDot && op != kFinDot2 && op != kFinDot2F32 && st->done;
-  // thread 0 fetches the scalars it will read while the block sums the partials
-  double rho = 0.0, rho_old = 0.0, norm_b = 0.0, tol = 0.0, atol = 0.0, cross = 0.0, an = 0.0, ao = 0.0;
-  int iter = 0, max_it = 0, method = 0;
-  double* hist = nullptr;
-  if (threadIdx.x == 0 && st) {
-    rho = st->rho;
-    rho_old = st->rho_old;
-    norm_b = st->norm_b;
-    tol = st->tol;
-    atol = st->atol;
-    cross = st->cross;
-    iter = st->iter;
-    max_it = st->max_it;
-    method = st->method;
-    hist = st->history;
-    if (op == kFinProj) {
-      an = aux[0];
-      ao = aux2 ? aux2[0] : 1.0;
-    }
+// direction for kFinNpsd.  A chain of latencies: the state and the alfas are fetched by lanes of
+// one wave while the block fetches the partials, so that memory is waited for once (scalar loads
+// where they are used, and one kernel for all operations, took 5.3 us at 64^3 and 6.4 us at
+// 256^3; now 3.2 to 4.3 and 4.2 to 6.2 us).
+template <int OP, int NR>
+__global__ __launch_bounds__(kFinThreads) void finalize_kernel(const double* __restrict__ partials, unsigned nb,
+                                                               SolveState* st, double* aux, const double* aux2) {
+  constexpr bool kDots = OP == kFinDot || OP == kFinDot2 || OP == kFinDot2F32;
+  constexpr int op = OP, kWords = (int)(sizeof(SolveState) / sizeof(double));
+  static_assert(sizeof(SolveState) % sizeof(double) == 0 && kWords <= 62, "state and alfas are fetched by one wave");
+  __shared__ double shs[64];
+  if (threadIdx.x < 64) {
+    const double* src = nullptr;
+    if (!kDots && (int)threadIdx.x < kWords) src = (const double*)st + threadIdx.x;
+    if (OP == kFinProj && threadIdx.x == 62) src = aux;
+    if (OP == kFinProj && threadIdx.x == 63) src = aux2;
+    if (src) shs[threadIdx.x] = *src;
   }
-  double t[3] = {0.0, 0.0, 0.0};
-  sum_partials_rows<3>(partials, nb, nr, t);
-  if (threadIdx.x != 0 || skip) return;
+  double t[NR] = {};
+  sum_partials_rows<NR>(partials, nb, NR, t);
+  if (threadIdx.x != 0) return;
+  const SolveState& in = *(const SolveState*)shs;
+  if (!kDots && OP != kFinResidInit && in.done) return;
+  double norm_b = kDots ? 0.0 : in.norm_b;
+  int iter = kDots ? 0 : in.iter;
   switch (op) {
     case kFinResidInit:
     case kFinResid: {
       if (op == kFinResidInit) {
-        norm_b = sqrt(t[1]);
+        norm_b = sqrt(t[NR > 1 ? 1 : 0]);
         st->norm_b = norm_b;
         iter = 0;
         st->done = (t[0] == 0.0) ? 1 : 0;
       } else {
         iter += 1;
-        st->rho_old = rho;
+        st->rho_old = in.rho;
       }
       st->iter = iter;
       st->rr = t[0];
@@ -792,23 +786,23 @@ __global__ __launch_bounds__(kFinThreads) void finalize_kernel(int op, int nr,
       st->norm = norm;
       st->scale = t[0] > 0.0 ? 1.0 / sqrt(t[0]) : 0.0;
       if (op == kFinResid) {
-        const double stop = fmax(tol, atol / norm_b);
-        const bool cont = (method == kNpsd) ? !(norm < stop) : (norm > stop);
-        st->done = (cont && iter < max_it) ? 0 : 1;
+        const double stop = fmax(in.tol, in.atol / norm_b);
+        const bool cont = (in.method == kNpsd) ? !(norm < stop) : (norm > stop);
+        st->done = (cont && iter < in.max_it) ? 0 : 1;
       }
-      if (hist && iter <= max_it) hist[iter] = norm;
+      if (in.history && iter <= in.max_it) in.history[iter] = norm;
       break;
     }
     case kFinPW:
       st->pw = t[0];
-      st->alpha = rho / t[0];
+      st->alpha = in.rho / t[0];
       break;
     case kFinRZ:
     case kFinRZ2: {  // kFinRZ: t1 = z.(r - r_old); kFinRZ2: t1 = z.r_old
-      const bool flex = (method == kNpcgFlex);
+      const bool flex = (in.method == kNpcgFlex);
       st->rho = t[0];
-      const double num = flex ? (op == kFinRZ ? t[1] : t[0] - t[1]) : t[0];
-      st->beta = (iter == 0) ? 0.0 : num / rho_old;
+      const double num = flex ? (op == kFinRZ ? t[NR > 1 ? 1 : 0] : t[0] - t[NR > 1 ? 1 : 0]) : t[0];
+      st->beta = (iter == 0) ? 0.0 : num / in.rho_old;
       break;
     }
     case kFinDot:
@@ -816,29 +810,30 @@ __global__ __launch_bounds__(kFinThreads) void finalize_kernel(int op, int nr,
       break;
     case kFinDot2:
       aux[0] = t[0];
-      aux[1] = t[1];
+      aux[1] = t[NR > 1 ? 1 : 0];
       break;
     case kFinDot2F32:  // the two sums rounded to FP32 (aux points at two floats)
       reinterpret_cast<float*>(aux)[0] = (float)t[0];
-      reinterpret_cast<float*>(aux)[1] = (float)t[1];
+      reinterpret_cast<float*>(aux)[1] = (float)t[NR > 1 ? 1 : 0];
       break;
     case kFinProj: {
-      const double gN = t[0] / an;
+      const double gN = t[0] / shs[62];
       st->proj[0] = gN;
-      st->proj[1] = aux2 ? (t[1] - gN * cross) / ao : 0.0;
+      st->proj[1] = aux2 ? (t[NR > 1 ? 1 : 0] - gN * in.cross) / shs[63] : 0.0;
       break;
     }
     case kFinNpsd:
       aux[0] = t[0];
-      st->alpha = t[1] / t[0];
-      st->cross = t[2];
+      st->alpha = t[NR > 1 ? 1 : 0] / t[0];
+      st->cross = t[NR > 2 ? 2 : 0];
       break;
   }
 }
 
-static void finalize(int op, int nr, double* partials, unsigned nb, SolveState* st, double* aux,
-                     hipStream_t s, const double* aux2 = nullptr) {
-  finalize_kernel<<<1, kFinThreads, 0, s>>>(op, nr, partials, nb, st, aux, aux2);
+template <int OP, int NR>
+static void finalize(double* partials, unsigned nb, SolveState* st, double* aux, hipStream_t s,
+                     const double* aux2 = nullptr) {
+  finalize_kernel<OP, NR><<<1, kFinThreads, 0, s>>>(partials, nb, st, aux, aux2);
 }
 
 // ---------------------------------------------------------------------------
@@ -899,14 +894,15 @@ int launch_resid_flat(const FlatArgs& a, int init, hipStream_t st) {
 #define MLPCG_RESID(VZ) resid_flat_kernel<VZ, false>
   if (init) MLPCG_FLAT_DISPATCH(MLPCG_RESID_INIT, a);
   else MLPCG_FLAT_DISPATCH(MLPCG_RESID, a);
-  finalize(init ? kFinResidInit : kFinResid, init ? 2 : 1, a.partials, flat_blocks(a), a.st, nullptr, st);
+  if (init) finalize<kFinResidInit, 2>(a.partials, flat_blocks(a), a.st, nullptr, st);
+  else finalize<kFinResid, 1>(a.partials, flat_blocks(a), a.st, nullptr, st);
   return check_launch("resid_flat");
 }
 
 int launch_p_spmv_flat(const FlatArgs& a, hipStream_t st) {
 #define MLPCG_PSPMV(VZ) p_spmv_flat_kernel<VZ>
   MLPCG_FLAT_DISPATCH(MLPCG_PSPMV, a);
-  finalize(kFinPW, 1, a.partials, flat_blocks(a), a.st, nullptr, st);
+  finalize<kFinPW, 1>(a.partials, flat_blocks(a), a.st, nullptr, st);
   return check_launch("p_spmv_flat");
 }
 
@@ -914,7 +910,7 @@ int launch_npsd_dir_flat(const FlatArgs& a, const float* pN, double* alfa_out,
                          hipStream_t st) {
 #define MLPCG_NPSD_DIR(VZ) npsd_dir_flat_kernel<VZ>
   MLPCG_FLAT_DISPATCH(MLPCG_NPSD_DIR, a, pN);
-  finalize(kFinNpsd, 3, a.partials, flat_blocks(a), a.st, alfa_out, st);
+  finalize<kFinNpsd, 3>(a.partials, flat_blocks(a), a.st, alfa_out, st);
   return check_launch("npsd_dir_flat");
 }
 
@@ -922,7 +918,7 @@ int launch_rz_dot(const float* r, const float* z, const float* r_old, long n, So
                   double* partials, hipStream_t st) {
   const unsigned nb = red_blocks(n / kDotRun + 1);
   rz_dot_kernel<<<nb, kThreads, 0, st>>>(r, z, r_old, n, s, partials);
-  finalize(kFinRZ, 2, partials, nb, s, nullptr, st);
+  finalize<kFinRZ, 2>(partials, nb, s, nullptr, st);
   return check_launch("rz_dot");
 }
 
@@ -941,14 +937,15 @@ int launch_gather(const int* idx, const float* grid, float* dst, long n, const i
 int launch_p_spmv_csr(const CsrArgs& a, hipStream_t st) {
   const unsigned nb = red_blocks(a.n);
   p_spmv_csr_kernel<<<nb, kThreads, 0, st>>>(a);
-  finalize(kFinPW, 1, a.partials, nb, a.st, nullptr, st);
+  finalize<kFinPW, 1>(a.partials, nb, a.st, nullptr, st);
   return check_launch("p_spmv_csr");
 }
 
 int launch_resid_csr(const CsrArgs& a, int init, hipStream_t st) {
   const unsigned nb = red_blocks(a.n);
   resid_csr_kernel<<<nb, kThreads, 0, st>>>(a, init);
-  finalize(init ? kFinResidInit : kFinResid, 2, a.partials, nb, a.st, nullptr, st);
+  if (init) finalize<kFinResidInit, 2>(a.partials, nb, a.st, nullptr, st);
+  else finalize<kFinResid, 2>(a.partials, nb, a.st, nullptr, st);
   return check_launch("resid_csr");
 }
 
@@ -956,18 +953,18 @@ int launch_npsd_dir_csr(const CsrArgs& a, const float* pN, double* alfa_out,
                         hipStream_t st) {
   const unsigned nb = red_blocks(a.n);
   npsd_dir_csr_kernel<<<nb, kThreads, 0, st>>>(a, pN);
-  finalize(kFinNpsd, 3, a.partials, nb, a.st, alfa_out, st);
+  finalize<kFinNpsd, 3>(a.partials, nb, a.st, alfa_out, st);
   return check_launch("npsd_dir_csr");
 }
 
 int launch_finalize_rz(double* partials, unsigned nb, SolveState* s, hipStream_t st) {
-  finalize(kFinRZ2, 2, partials, nb, s, nullptr, st);
+  finalize<kFinRZ2, 2>(partials, nb, s, nullptr, st);
   return check_launch("finalize_rz");
 }
 
 int launch_finalize_proj(double* partials, unsigned nb, SolveState* s, const double* alfaN,
                          const double* alfaO, hipStream_t st) {
-  finalize(kFinProj, 2, partials, nb, s, const_cast<double*>(alfaN), st, alfaO);
+  finalize<kFinProj, 2>(partials, nb, s, const_cast<double*>(alfaN), st, alfaO);
   return check_launch("finalize_proj");
 }
 
@@ -975,7 +972,7 @@ int launch_npsd_proj(const float* q, const float* aN, const float* aO, const dou
                      const double* alfaO, long n, SolveState* s, double* partials, hipStream_t st) {
   const unsigned nb = red_blocks(n / kDotRun + 1);
   npsd_proj_kernel<<<nb, kThreads, 0, st>>>(q, aN, aO, n, s, partials);
-  finalize(kFinProj, 2, partials, nb, s, const_cast<double*>(alfaN), st, alfaO);
+  finalize<kFinProj, 2>(partials, nb, s, const_cast<double*>(alfaN), st, alfaO);
   return check_launch("npsd_proj");
 }
 
@@ -1019,7 +1016,7 @@ int launch_loss_resid(int tx, const void* x, const float* b, const uint8_t* code
   else if (tx == kF32) MLPCG_LR(float);
   else MLPCG_REQUIRE(false, "loss_resid: x must be FP32 or BF16 (got %d)", tx);
 #undef MLPCG_LR
-  finalize(kFinDot2, 2, partials, nb, nullptr, out2, st);
+  finalize<kFinDot2, 2>(partials, nb, nullptr, out2, st);
   return check_launch("loss_resid");
 }
 
@@ -1087,7 +1084,8 @@ int launch_comb_grad(int dt, const void* g, const void* x0, const void* x1, cons
     MLPCG_REQUIRE(false, "comb_grad: elements must be FP32 or BF16 (got %d)", dt);
   }
 #undef MLPCG_CG
-  finalize(out_dt == kF32 ? kFinDot2F32 : kFinDot2, 2, partials, nb, nullptr, (double*)out2, st);
+  if (out_dt == kF32) finalize<kFinDot2F32, 2>(partials, nb, nullptr, (double*)out2, st);
+  else finalize<kFinDot2, 2>(partials, nb, nullptr, (double*)out2, st);
   return check_launch("comb_grad");
 }
 
@@ -1095,7 +1093,7 @@ int launch_dot(const float* x, const float* y, long n, double* partials,
                double* out, hipStream_t st) {
   const unsigned nb = red_blocks(n);
   dot_kernel<<<nb, kThreads, 0, st>>>(x, y, n, partials);
-  finalize(kFinDot, 1, partials, nb, nullptr, out, st);
+  finalize<kFinDot, 1>(partials, nb, nullptr, out, st);
   return check_launch("dot");
 }
 

@@ -33,8 +33,13 @@ static size_t dsize(int dt) {
 constexpr long kFusedMinVoxels = 1L << 18;
 
 // FP32 blocks recompute K (split.hpp) on grids above this many voxels.  A 64^3 level's
-// stencils (28 MB) stay in the caches and their apply takes 7.4 us; at 96^3 they no longer do.
+// stencils (28 MB) stay in the caches and their apply takes 7.4 us; at 96^3 they no longer do
+// (stored and recomputed: 64 x 64 x 72 11.9 and 10.3 us, 96^3 20.6 and 13.3 us, 128^3 40 and 18
+// us).  With two or three channels K costs two to three times as much and pays later (96^3 22.6
+// and 30.3 us, 112 x 96 x 128 26 and 34 us, 128^3 40 and 37 us, 256^3 351 and 258 us); mode 2
+// takes it from 2^18 on too.
 constexpr long kSplitMinVoxels = 1L << 18;
+constexpr long kSplitChannelsMinVoxels = 1L << 21;
 
 // plan generation ids: never reused within a process, unlike plan addresses
 static std::atomic<unsigned long> g_next_gen{1};
@@ -135,7 +140,7 @@ int precond_create(Precond** out, int kind, int n, int C, int n1, int n2, int n3
     const bool big = P->V[b.level] >= kFusedMinVoxels || fused_mode == 2;
     b.fused = (half && !b.trans && fused_mode && big && fused_eligible(P->cf, 1, d[0], d[1], d[2])) ? 1 : 0;
     b.split = (dtype == kF32 && !b.trans && fused_mode && P->V[b.level] > kSplitMinVoxels &&
-               split_eligible(C, d[0], d[1], d[2]))
+               (C == 1 || fused_mode == 2 || P->V[b.level] >= kSplitChannelsMinVoxels) && split_eligible(C, d[0], d[1], d[2]))
                   ? 1
                   : 0;
     if (b.split) {

@@ -37,6 +37,12 @@ struct PatchSums {
   double t[C][27];
 };
 
+// the sum over the wave (valid in lane 63) of values that are often zero in all of it: most waves
+// touch no face across i, many none across j
+__device__ __forceinline__ double wave_sum_sparse(double v) {
+  return __builtin_amdgcn_ballot_w64(v != 0.0) == 0 ? 0.0 : wave_sum_dpp(v);
+}
+
 template <typename TI, int C, int VZ>
 __device__ __forceinline__ void patch_accumulate(const TI* __restrict__ img, int n1, int n2, int n3, unsigned first,
                                                  unsigned stride, PatchSums<C>& p) {
@@ -135,7 +141,7 @@ __global__ __launch_bounds__(kThreads) void mean_patch_partial_kernel(const TI* 
   const int w = threadIdx.x >> 6;
 #pragma unroll
   for (int o = 0; o < 27 * C; ++o) {
-    const double s = wave_sum_dpp(p.t[o / 27][o % 27]);
+    const double s = wave_sum_sparse(p.t[o / 27][o % 27]);
     if ((threadIdx.x & 63) == 63) sh[o][w] = s;
   }
   __syncthreads();
@@ -156,8 +162,10 @@ __global__ __launch_bounds__(kPatchFinalThreads) void mean_patch_final_kernel(
   for (int o = wv; o < NV; o += kPatchFinalThreads / 64) {
     double a[kPatchBlocks / 64];
 #pragma unroll
-    for (int u = 0; u < kPatchBlocks / 64; ++u)
-      a[u] = lane + 64 * u < nblk ? partials[(size_t)o * nblk + lane + 64 * u] : 0.0;
+    for (int u = 0; u < kPatchBlocks / 64; ++u)  // (a uniform test: the loads are in flight together)
+      a[u] = 64 * u < nblk ? partials[(size_t)o * nblk + min(lane + 64 * u, nblk - 1)] : 0.0;
+#pragma unroll
+    for (int u = 0; u < kPatchBlocks / 64; ++u) a[u] = lane + 64 * u < nblk ? a[u] : 0.0;
 #pragma unroll
     for (int u = 1; u < kPatchBlocks / 64; ++u) a[0] += a[u];
     const double s = wave_sum_dpp(a[0]);
@@ -184,7 +192,7 @@ __global__ __launch_bounds__(kPatchFinalThreads) void mean_patch_one_kernel(
     patch_accumulate<TI, 1, VZ>(img + (long)s * n1 * n2 * n3, n1, n2, n3, threadIdx.x, kPatchFinalThreads, p);
 #pragma unroll
     for (int o = 0; o < 27; ++o) {
-      const double v = wave_sum_dpp(p.t[0][o]);
+      const double v = wave_sum_sparse(p.t[0][o]);
       if ((threadIdx.x & 63) == 63) sh[27 * s + o][w] = v;
     }
   }

@@ -75,7 +75,7 @@ struct Precond {
 // Per-plan policies.  fused_mode: eligible BF16 blocks recompute their stencils on the
 // matrix cores inside the apply -- 0 never, 1 (default) on grids of at least
 // kFusedMinVoxels voxels, 2 on every eligible grid; FP32 blocks with mode 1 or 2 on grids
-// above kSplitMinVoxels; plus kFuseFoldThird: for three-channel
+// above kSplitMinVoxels (more channels than one with mode 1: kSplitChannelsMinVoxels); plus kFuseFoldThird: for three-channel
 // images whose third channel is the sum of the first two (the [air, fluid, non-solid]
 // images), the fused blocks take two channels with the third channel's weights added to
 // the others' (the caller vouches for the relation).  coarse_tail: the two coarsest SmallSM

@@ -45,8 +45,8 @@ class Preconditioner:
     fused_mode -- BF16 blocks on grids with n1, n2 % 8 == 0 and n3 % 64 == 0 (C <= 3)
       recompute their stencils on the matrix cores inside the apply instead of storing
       them: 0 never, 1 (default) on such grids of at least 2^18 voxels, 2 on every such grid;
-      FP32 blocks of any grid above 2^18 voxels do so with 1 and 2 (FP16 operands split in
-      two, errors as with FP32 stencils);
+      FP32 blocks of any grid above 2^18 voxels do so with 1 and 2, with 1 and several
+      channels from 2^21 on (FP16 operands split in two, errors as with FP32 stencils);
     fold_third -- three-channel images whose third channel is the sum of the first two (the
       [air, fluid, non-solid] images of the reference's models): the fused blocks take two
       channels, the third channel's weights added to the others' (equal in exact arithmetic;

@@ -79,7 +79,8 @@ def test_split_forward_keeps_non_finite_values_local(dev):
 @pytest.mark.parametrize("C,mask,swap,n,shape", [(1, False, False, 2, (64, 64, 68)), (3, True, False, 1, (66, 62, 72)),
                                                  (2, False, True, 1, (64, 72, 64)), (3, False, False, 2, (36, 100, 84))])
 def test_split_plan_matches_stored_stencils(dev, C, mask, swap, n, shape):
-    """Plans whose level 0 is above 2^18 voxels: with the output mask, the input scale and the
+    """Plans whose level 0 is above 2^18 voxels (fused_mode 2 recomputes K there for any channel
+    count): with the output mask, the input scale and the
     pooled epilogue against the stored-stencil plan of the same model (fused_mode 0)."""
     from mlpcg_amd.sm_model_3d import SmallSMModelDn3D
     print(f"split plan {shape} C={C}", flush=True)
@@ -92,7 +93,7 @@ def test_split_plan_matches_stored_stencils(dev, C, mask, swap, n, shape):
     out = (torch.rand(*shape, generator=g) > 0.4).to(torch.uint8)
     out[:, :, 60:] = 0
     out = out.to(dev)
-    a, b = m.make_preconditioner(img), m.make_preconditioner(img, fused_mode=0)
+    a, b = m.make_preconditioner(img, fused_mode=2), m.make_preconditioner(img, fused_mode=0)
     assert a.nbytes < b.nbytes
     for args in ((None, None), (scale, out)):
         za, zb = a.apply(r, *args), b.apply(r, *args)
