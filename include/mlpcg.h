@@ -123,6 +123,11 @@ int mlpcg_sm_linear_inference(const void* image, const void* weight, const void*
 int mlpcg_sm_linear_forward(const void* image, const void* weight, const void* bias, void* z,
                             void* ybar, void* workspace, int C, int n1, int n2, int n3, int dtype,
                             void* stream);
+/* No counterpart in the reference: two SM linears of one image (a level's c0 and c1), which
+ * share the mean patch ybar: the results of two mlpcg_sm_linear_inference calls. */
+int mlpcg_sm_linear_pair(const void* image, const void* weight0, const void* bias0, void* z0, const void* weight1,
+                         const void* bias1, void* z1, void* ybar, void* workspace, int C, int n1, int n2, int n3,
+                         int dtype, void* stream);
 /* No counterpart in the reference: mlpcg_sm_linear_inference for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops, harnesses
  * that forbid hipMalloc).  Same results as mlpcg_sm_linear_inference (same kernels, same

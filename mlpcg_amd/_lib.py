@@ -61,6 +61,7 @@ SIGNATURES = {
     "mlpcg_sm_linear_workspace_size": (sz, [i32, i32, i32, i32, i32]),
     "mlpcg_sm_linear_inference": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, vp]),
     "mlpcg_sm_linear_forward": (i32, [vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, vp]),
+    "mlpcg_sm_linear_pair": (i32, [vp, vp, vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, vp]),
     "mlpcg_sm_linear_backward": (i32, [vp, vp, vp, vp, i32, i32, vp]),
     "mlpcg_sm_linear_noalloc_scratch_bytes": (sz, []),
     "mlpcg_sm_linear_inference_noalloc": (i32, [vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, vp]),
@@ -135,6 +136,10 @@ def ptr(t) -> int | None:
 
 
 def stream_ptr(device=None) -> int:
+    """The current stream of a device, as a handle (without the Stream object that
+    torch.cuda.current_stream builds: 2 us a call)."""
+    if isinstance(device, torch.device) and device.index is not None and torch.cuda.is_initialized():
+        return torch._C._cuda_getCurrentRawStream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 

@@ -277,6 +277,16 @@ int mlpcg_sm_linear_inference(const void* image, const void* weight, const void*
   MLPCG_REQUIRE(aligned16(image), "sm_linear: image must be 16-byte aligned");
   return launch_sm_linear(dtype, image, weight, bias, z, ybar, workspace, C, n1, n2, n3, STREAM(stream));
 }
+int mlpcg_sm_linear_pair(const void* image, const void* weight0, const void* bias0, void* z0, const void* weight1,
+                         const void* bias1, void* z1, void* ybar, void* workspace, int C, int n1, int n2, int n3,
+                         int dtype, void* stream) {
+  if (check_block_args("sm_linear_pair", C, 1, n1, n2, n3, dtype)) return -1;
+  MLPCG_REQUIRE(image && weight0 && bias0 && z0 && weight1 && bias1 && z1 && ybar && workspace,
+                "sm_linear_pair: null pointer");
+  MLPCG_REQUIRE(aligned16(image), "sm_linear_pair: image must be 16-byte aligned");
+  return launch_sm_linear_pair(dtype, image, weight0, bias0, z0, weight1, bias1, z1, ybar, workspace, C, n1, n2, n3,
+                               STREAM(stream));
+}
 size_t mlpcg_sm_linear_noalloc_scratch_bytes(void) { return sm_linear_scratch_bytes(); }
 int mlpcg_sm_linear_inference_noalloc(const void* image, const void* weight, const void* bias, void* z,
                                       void* ybar, int C, int n1, int n2, int n3, int dtype, void* stream) {

@@ -31,9 +31,13 @@ def _acc(dtype):
     return ACC_DTYPE[code_of(dtype)]
 
 
+def _param(t, acc):
+    return t if t.dtype == acc and t.is_contiguous() else t.detach().to(acc).contiguous()
+
+
 def _params(weight, bias, dtype):
     acc = _acc(dtype)
-    return weight.detach().to(acc).contiguous(), bias.detach().to(acc).contiguous()
+    return _param(weight, acc), _param(bias, acc)
 
 
 def workspace(nbytes, device):
@@ -199,6 +203,25 @@ def sm_linear(image, weight, bias):
     check(lib.mlpcg_sm_linear_forward(ptr(image), ptr(w), ptr(b), ptr(z), ptr(ybar), ptr(ws), Cimg,
                                       n1, n2, n3, dt, stream_ptr(image.device)), "sm_linear")
     return z, ybar
+
+
+def sm_linear_pair(image, weight0, bias0, weight1, bias1):
+    """-> (z0, z1): sm_linear(image, weight0, bias0)[0] and sm_linear(image, weight1, bias1)[0]
+    from one mean patch (a level's c0 and c1)."""
+    require_cuda(image)
+    dt = code_of(image.dtype)
+    acc = _acc(image.dtype)
+    w0, b0 = _params(weight0, bias0, image.dtype)
+    w1, b1 = _params(weight1, bias1, image.dtype)
+    Cimg = image.shape[0]
+    n1, n2, n3 = _grid(image)
+    z0 = torch.empty(1, dtype=acc, device=image.device)
+    z1 = torch.empty(1, dtype=acc, device=image.device)
+    ybar = torch.empty(1, Cimg, 3, 3, 3, dtype=acc, device=image.device)
+    ws = workspace(lib.mlpcg_sm_linear_workspace_size(Cimg, n1, n2, n3, dt), image.device)
+    check(lib.mlpcg_sm_linear_pair(ptr(image), ptr(w0), ptr(b0), ptr(z0), ptr(w1), ptr(b1), ptr(z1), ptr(ybar), ptr(ws),
+                                   Cimg, n1, n2, n3, dt, stream_ptr(image.device)), "sm_linear_pair")
+    return z0, z1
 
 
 def sm_linear_backward(g, ybar):

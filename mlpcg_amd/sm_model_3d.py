@@ -188,6 +188,15 @@ class SmallLinearBlock3DNew(BaseModel):
         return SMLinearFunction3D.inference(image, self.weight, self.bias, timer)
 
 
+def _plain_linears(a, b, image):
+    """Whether both modules are SM linears as they come (no subclass or patched eval_forward) on
+    an image that the native call takes as it is."""
+    return (type(a) is SmallLinearBlock3DNew and type(b) is SmallLinearBlock3DNew
+            and "eval_forward" not in a.__dict__ and "eval_forward" not in b.__dict__
+            and image.is_cuda and image.is_contiguous() and a.weight.shape[1] == b.weight.shape[1] == image.shape[0]
+            and a.weight.device == b.weight.device == image.device)
+
+
 ######################
 # Level transfers (F.avg_pool3d / F.interpolate replacements with HIP backward)
 ######################
@@ -329,9 +338,13 @@ class SmallSMModelDn3D(BaseModel):
         x[-1] = self.l.eval_forward(fine_img, x[-1], timer)
         for i in range(self.n, 0, -1):
             x[i] = upsample(x[i], self.mode)
-            if not c0_cached:
+            if not c0_cached and not c1_cached and timer is None and _plain_linears(self.c0[i - 1], self.c1[i - 1], imgs[i - 1]):
+                # one mean patch for both (a timer counts them one by one)
+                a, b2 = self.c0[i - 1], self.c1[i - 1]
+                c0[i - 1], c1[i - 1] = K.sm_linear_pair(imgs[i - 1], a.weight, a.bias, b2.weight, b2.bias)
+            if not c0_cached and c0[i - 1] is None:
                 c0[i - 1] = self.c0[i - 1].eval_forward(imgs[i - 1], timer)
-            if not c1_cached:
+            if not c1_cached and c1[i - 1] is None:
                 c1[i - 1] = self.c1[i - 1].eval_forward(imgs[i - 1], timer)
             if self.swap_ord:
                 x[i - 1] = _comb(c0[i - 1], x[i - 1], c1[i - 1], x[i])
