@@ -89,18 +89,16 @@ static int block_fwd(bool trans, const void* image, const void* x, const void* w
   const size_t V = (size_t)n1 * n2 * n3;
   if (!trans && dtype == kBF16 && V >= kFusedForwardMinVoxels && fused_eligible(C, B, n1, n2, n3)) {
     // BF16 block: K recomputed on the matrix cores (the fused apply of the BF16 plans)
-    // from an FP16 copy of the image (exact for BF16 image values in the FP16 normal
-    // range) and the FP32 weights packed for it; no stencils are stored.  K, x and the
+    // from the image in FP16 (exact for BF16 image values in the FP16 normal range; a
+    // caller's copy, or converted as it is staged: a copy made here took 10 us at 256^3) and
+    // the FP32 weights packed for it; no stencils are stored.  K, x and the
     // sums round as in the stored-stencil apply (K to BF16, FP32 sums).
-    char* ws = (char*)workspace;
-    const void* img16 = image16 ? image16 : ws;
-    void* wbuf = ws + ((C * V * 2 + 255) & ~(size_t)255);
-    const void* wpack = wpack_in ? wpack_in : wbuf;
-    if (!image16 && launch_cast(kBF16, kF16, image, ws, (long)(C * V), STREAM(stream))) return -1;
-    if (!wpack_in && launch_fused_pack(kBF16, weight, bias, C, wbuf, STREAM(stream))) return -1;
+    const void* wpack = wpack_in ? wpack_in : workspace;
+    if (!wpack_in && launch_fused_pack(kBF16, weight, bias, C, workspace, STREAM(stream))) return -1;
     FusedArgs f;
     memset(&f, 0, sizeof(f));
-    f.img = img16;
+    f.img = image16 ? image16 : image;
+    f.img_bf16 = image16 ? 0 : 1;
     f.apack = wpack;
     f.x = x;
     f.y = y;

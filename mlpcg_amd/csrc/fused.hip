@@ -255,7 +255,8 @@ __host__ __device__ constexpr int fused_waves(int C, int FI, int EPI) {
          : C == 3 ? ((EPI & kEpiDot1) ? 1 : 4)
                   : 1;
 }
-template <typename TX, typename TY, typename TP, int C, int FI, int EPI, bool PL = false>
+// TI: the image's type; a BF16 image (block forwards) becomes FP16 as it is staged.
+template <typename TX, typename TY, typename TP, int C, int FI, int EPI, bool PL = false, typename TI = f16>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(fused_waves(C, FI, EPI), 8)))
 void sm_fused_kernel(FusedArgs a) {
   constexpr int kTile = tile_cells(FI);
@@ -334,7 +335,7 @@ void sm_fused_kernel(FusedArgs a) {
   // planes).  The staging code is instantiated once per wave index (a uniform branch), so
   // the row geometry is folded at compile time and a row costs a few scalar instructions.
   const TX* __restrict__ x = (const TX*)a.x;
-  const f16* __restrict__ img = (const f16*)a.img;
+  const TI* __restrict__ img = (const TI*)a.img;
   static_assert((FI + 2) * kPj % 4 == 0 && kRowCells == 66, "staging assumes 4 waves x kRows rows of 66 cells");
   {
     constexpr unsigned kOut = 0x80000000u;  // beyond any plane (planes are under 2^31 bytes)
@@ -357,7 +358,7 @@ void sm_fused_kernel(FusedArgs a) {
       for (int k0 = 0; k0 < kRows; k0 += 13) {
         constexpr int KB = 13;
         bf16 xv[KB][2];
-        f16 iv[KB][C][2];
+        TI iv[KB][C][2];
 #pragma unroll
         for (int kk = 0; kk < KB; ++kk) {
           const int k = k0 + kk;
@@ -376,7 +377,7 @@ void sm_fused_kernel(FusedArgs a) {
             for (int c = 0; c < C; ++c) {
               const auto ir = row_rsrc(img + (c * V + p0 + po), rok ? ipb : 0);
 #pragma unroll
-              for (int u = 0; u < 2; ++u) iv[kk][c][u] = rsrc_load(ir, zi[u], soff * irb, (const f16*)nullptr);
+              for (int u = 0; u < 2; ++u) iv[kk][c][u] = rsrc_load(ir, zi[u], soff * irb, (const TI*)nullptr);
             }
           }
         }
@@ -386,7 +387,7 @@ void sm_fused_kernel(FusedArgs a) {
           if (k0 + kk < kRows) {
             xs[r * kPz + lane] = xv[kk][0];
 #pragma unroll
-            for (int c = 0; c < C; ++c) is[c * kTile + r * kPz + lane] = iv[kk][c][0];
+            for (int c = 0; c < C; ++c) is[c * kTile + r * kPz + lane] = (f16)(float)iv[kk][c][0];
           }
         }
         if (lane < 2) {
@@ -396,7 +397,7 @@ void sm_fused_kernel(FusedArgs a) {
             if (k0 + kk < kRows) {
               xs[r * kPz + 64 + lane] = xv[kk][1];
 #pragma unroll
-              for (int c = 0; c < C; ++c) is[c * kTile + r * kPz + 64 + lane] = iv[kk][c][1];
+              for (int c = 0; c < C; ++c) is[c * kTile + r * kPz + 64 + lane] = (f16)(float)iv[kk][c][1];
             }
           }
         }
@@ -810,15 +811,15 @@ int launch_fused_pack(int tw, const void* W, const void* b, int C, void* wbuf, h
   return check_launch("fused_pack");
 }
 
-template <typename TX, typename TY, int C, int EPI, bool PL = false>
+template <typename TX, typename TY, int C, int EPI, bool PL = false, typename TI = f16>
 static void launch_fused_t(const FusedArgs& a, hipStream_t st) {
   const unsigned nb = fused_blocks(C, a.n1, a.n2, a.n3);
   const int fi = fused_fi(C, a.n1, a.n2, a.n3);
   if constexpr ((C + 1) * tile_cells(8) * 2 <= kMaxFusedLds) {
-    if (fi == 8) return sm_fused_kernel<TX, TY, bf16, C, 8, EPI, PL><<<nb, kThreads, 0, st>>>(a);
+    if (fi == 8) return sm_fused_kernel<TX, TY, bf16, C, 8, EPI, PL, TI><<<nb, kThreads, 0, st>>>(a);
   }
-  if (fi == 4) sm_fused_kernel<TX, TY, bf16, C, 4, EPI, PL><<<nb, kThreads, 0, st>>>(a);
-  else sm_fused_kernel<TX, TY, bf16, C, 2, EPI, PL><<<nb, kThreads, 0, st>>>(a);
+  if (fi == 4) sm_fused_kernel<TX, TY, bf16, C, 4, EPI, PL, TI><<<nb, kThreads, 0, st>>>(a);
+  else sm_fused_kernel<TX, TY, bf16, C, 2, EPI, PL, TI><<<nb, kThreads, 0, st>>>(a);
 }
 
 // The epilogues of a preconditioner application get compile-time kernels: the pre blocks
@@ -831,6 +832,8 @@ static void launch_fused_epi(const FusedArgs& a, hipStream_t st) {
   const int epi = (a.prev ? kEpiPrev : 0) | (a.mask_a ? kEpiMaskA : 0) | (a.mask_b ? kEpiMaskB : 0) |
                   (a.partials ? kEpiDot0 : 0) | (a.partials && a.dot1 ? kEpiDot1 : 0);
   if constexpr (sizeof(TY) == 2) {
+    if constexpr (sizeof(TX) == 2)
+      if (a.img_bf16) return launch_fused_t<TX, TY, C, 0, false, bf16>(a, st);
     if (epi == 0) return a.pool_out ? launch_fused_t<TX, TY, C, 0, true>(a, st) : launch_fused_t<TX, TY, C, 0>(a, st);
     if constexpr (sizeof(TX) == 2)
       if (epi == kEpiPrev) return launch_fused_t<TX, TY, C, kEpiPrev>(a, st);
@@ -869,6 +872,9 @@ int launch_sm_fused(int tw, int tx, int ty, int C, const FusedArgs& args, hipStr
   MLPCG_REQUIRE(!args.partials || args.dot0, "sm_fused: partials need dot0");
   MLPCG_REQUIRE(!args.pool_out || (ty == kBF16 && !args.prev && !args.mask_a && !args.mask_b && !args.partials),
                 "sm_fused: the pooled output needs a BF16 output and no epilogue operands");
+  MLPCG_REQUIRE(!args.img_bf16 || (tx == kBF16 && ty == kBF16 && !args.prev && !args.mask_a && !args.mask_b &&
+                                   !args.partials && !args.pool_out),
+                "sm_fused: a BF16 image needs BF16 vectors and no epilogue operands");
   const FusedArgs& a = args;
 #define MLPCG_FU(TXX, TYY)                                 \
   do {                                                     \

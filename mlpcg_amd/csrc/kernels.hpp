@@ -64,6 +64,7 @@ struct FusedArgs {
   // optional: idle tiles (launch_idle_tiles) of the grid x and mask_b belong to; x must be zero
   // where the fluid is not, and mask_b, if given, the fluid
   const uint8_t* idle;
+  int img_bf16;  // img is BF16 (BF16 vectors, no epilogue operands)
   int n1, n2, n3;
 };
 

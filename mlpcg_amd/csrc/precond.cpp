@@ -224,6 +224,7 @@ int Precond::run_block(int k, int level, const void* x, int tx, void* y, int ty,
   if (blocks[k].fused) {
     FusedArgs f;
     f.idle = idle;
+    f.img_bf16 = 0;
     f.pool_out = pool_out;
     f.dot0 = dot0;
     f.dot1 = dot1;
