@@ -34,8 +34,9 @@ static bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 // apply (as the BF16 plans do); smaller grids stream stored stencils.
 constexpr size_t kFusedForwardMinVoxels = (size_t)1 << 18;
 
-// FP32 block forwards on grids of at least this many voxels recompute K on the matrix cores
-// (split.hpp) instead of storing it.
+// FP32 block forwards, and BF16 ones that the fused apply does not take (ragged grids, batches),
+// on grids of at least this many voxels recompute K on the matrix cores (split.hpp) instead of
+// storing it; so do the input gradients (igrad.hpp).
 constexpr size_t kSplitMinVoxels = (size_t)1 << 14;
 
 }  // namespace mlpcg
@@ -107,10 +108,11 @@ static int block_fwd(bool trans, const void* image, const void* x, const void* w
     f.n3 = n3;
     return launch_sm_fused(kBF16, kBF16, kBF16, C, f, STREAM(stream));
   }
-  if (!trans && dtype == kF32 && V >= kSplitMinVoxels && split_eligible(C, n1, n2, n3)) {
+  if (!trans && (dtype == kF32 || dtype == kBF16) && V >= kSplitMinVoxels && split_eligible(C, n1, n2, n3)) {
     if (launch_split_pack(weight, bias, C, workspace, STREAM(stream))) return -1;
     SplitArgs f;
     memset(&f, 0, sizeof(f));
+    f.is_bf16 = dtype == kBF16;
     f.img = (const float*)image;
     f.pack = workspace;
     f.x = (const float*)x;

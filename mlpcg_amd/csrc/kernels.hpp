@@ -98,6 +98,7 @@ struct SplitArgs {
   double* partials;
   // optional (B = 1, even grid, no epilogue operands): the 2x2x2 means of y, as avgpool2's
   float* pool_out;
+  int is_bf16;  // img, x and y are BF16 (no epilogue operands)
   int B, n1, n2, n3;
 };
 size_t split_pack_bytes(int C);

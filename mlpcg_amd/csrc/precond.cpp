@@ -247,6 +247,7 @@ int Precond::run_block(int k, int level, const void* x, int tx, void* y, int ty,
   }
   if (blocks[k].split) {
     SplitArgs f;
+    f.is_bf16 = 0;
     f.img = (const float*)img[level];
     f.pack = wpack[k];
     f.x = (const float*)x;

@@ -364,13 +364,16 @@ constexpr int kEpiPrev = 1, kEpiMaskA = 2, kEpiMaskB = 4, kEpiDot0 = 8, kEpiDot1
 __host__ __device__ constexpr int split_waves(int C, int BB) { return C == 1 ? (BB == 1 ? 4 : 3) : 2; }
 
 // The apply.  EPI: compile-time epilogue (kEpiRuntime: every operand tested), PL: also write
-// the 2x2x2 means of y; BB: right-hand sides per workgroup (K is shared by them).
-template <int C, int FI, int BB, int EPI, bool PL>
+// the 2x2x2 means of y; BB: right-hand sides per workgroup (K is shared by them).  T: the type of
+// x, image and y; a BF16 image is exact in one FP16 value, and 11 bits of the weights are more
+// than a BF16 result keeps.
+template <typename T, int C, int FI, int BB, int EPI, bool PL>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(split_waves(C, BB), 8)))
 void sm_split_kernel(SplitArgs a) {
   constexpr int kCells = tile_cells(FI);
+  constexpr bool FULL = sizeof(T) == 4;
   __shared__ __attribute__((aligned(16))) float xs[BB][kCells];
-  __shared__ __attribute__((aligned(16))) f16 ih[C * kCells], il[C * kCells];
+  __shared__ __attribute__((aligned(16))) f16 ih[C * kCells], il[FULL ? C * kCells : 8];
   __shared__ unsigned sh[12];
   if (solve_done(a.done)) return;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -381,10 +384,10 @@ void sm_split_kernel(SplitArgs a) {
 
   Raw<FI> rx[BB], ri[C];
 #pragma unroll
-  for (int c = 0; c < C; ++c) load_raw<FI, kPJ>(ri[c], a.img + c * V, t, a.n1, a.n2, a.n3, w, lane);
+  for (int c = 0; c < C; ++c) load_raw<FI, kPJ>(ri[c], (const T*)a.img + c * V, t, a.n1, a.n2, a.n3, w, lane);
 #pragma unroll
   for (int bb = 0; bb < BB; ++bb)
-    if (BB == 1 || b0 + bb < a.B) load_raw<FI, kPJ>(rx[bb], a.x + (long)(b0 + bb) * V, t, a.n1, a.n2, a.n3, w, lane);
+    if (BB == 1 || b0 + bb < a.B) load_raw<FI, kPJ>(rx[bb], (const T*)a.x + (long)(b0 + bb) * V, t, a.n1, a.n2, a.n3, w, lane);
   const PackHeader* hd = (const PackHeader*)a.pack;
   const float scale = a.in_scale ? (float)(*a.in_scale) : 1.f;
   const float c0 = a.prev ? *a.c0 : 0.f, c1 = a.prev ? *a.c1 : 0.f;
@@ -400,8 +403,8 @@ void sm_split_kernel(SplitArgs a) {
   }
   xany = __builtin_amdgcn_ballot_w64(xany != 0) != 0;
   if (lane == 0) sh[8 + w] = xany;
-  const ImageTile it = stage_image<C, FI>(ri, hd->img_limit, w, lane, ih, il, sh);
-  Weights<C> W;
+  const ImageTile it = stage_image<C, FI, kPJ, FULL>(ri, hd->img_limit, w, lane, ih, il, sh);
+  Weights<C, FULL> W;
   W.load(a.pack, lane);
   W.set_bias(((const float*)((const char*)a.pack + kHeaderBytes + pack_w_bytes(C)))[lane & 31] * pow2(it.exp), h);
   // x = 0 everywhere: every finite K gives y = 0
@@ -428,7 +431,7 @@ void sm_split_kernel(SplitArgs a) {
   float pp[PL ? FI * 2 : 1];
   const int rows_i = a.n1 - t.i0, rows_j = a.n2 - t.j0;
   const long plane = (long)a.n2 * a.n3, v00 = ((long)t.i0 * a.n2 + t.j0 + w) * a.n3 + t.z0, j4 = 4L * a.n3;
-  float* __restrict__ y = a.y + b0 * V;
+  T* __restrict__ y = (T*)a.y + b0 * V;
 
   auto chunks = [&](auto lo_c) {
     constexpr bool LO = decltype(lo_c)::value;
@@ -456,7 +459,7 @@ void sm_split_kernel(SplitArgs a) {
       const bool skip = zero || (LB && has_b && __builtin_amdgcn_ballot_w64(zok && kb != 0) == 0);
       if (!skip) {
         f16x K[2];
-        stencils<C, LO, true>(W, ih, il, kCells, wb, cell, K);
+        stencils<C, LO, FULL>(W, ih, il, kCells, wb, cell, K);
 #pragma unroll
         for (int bb = 0; bb < BB; ++bb) {
           float pe = 0.f, po = 0.f;
@@ -485,7 +488,7 @@ void sm_split_kernel(SplitArgs a) {
         if (LA && has_a && ka == 0) v = 0.f;
         if (LP && has_p) v = c0 * pv + c1 * v;
         if (LB && has_b && kb == 0) v = 0.f;
-        if (zok) (y + bb * V + vr)[myz] = v;
+        if (zok) (y + bb * V + vr)[myz] = (T)v;
         if (PL) pp[q] = halves_sum(v, v);
         if (LD0 && has_0) {
           red[0] += (double)v * (double)da;
@@ -495,8 +498,12 @@ void sm_split_kernel(SplitArgs a) {
       }
     }
   };
-  if (it.has_lo && !zero) chunks(std::true_type());
-  else chunks(std::false_type());
+  if constexpr (FULL) {
+    if (it.has_lo && !zero) chunks(std::true_type());
+    else chunks(std::false_type());
+  } else {
+    chunks(std::false_type());
+  }
   if (LD0 && has_0) block_partials<2>(red, a.partials);
   if constexpr (PL) {
     // the means of the stored output in avgpool2_kernel's order (z pair, then rows 2J, 2J + 1
@@ -531,12 +538,12 @@ inline unsigned blocks_at(int FI, int n1, int n2, int n3) {
 }
 inline int planes(int n1, int n2, int n3) { return blocks_at(4, n1, n2, n3) >= kMinBlocks ? 4 : 2; }
 
-template <int C, int BB, int EPI, bool PL>
+template <int C, int BB, int EPI, bool PL, typename T = float>
 void launch(const SplitArgs& a, hipStream_t st) {
   const int fi = planes(a.n1, a.n2, a.n3);
   const dim3 g(blocks_at(fi, a.n1, a.n2, a.n3), (unsigned)((a.B + BB - 1) / BB));
-  if (fi == 4) sm_split_kernel<C, 4, BB, EPI, PL><<<g, kThreads, 0, st>>>(a);
-  else sm_split_kernel<C, 2, BB, EPI, PL><<<g, kThreads, 0, st>>>(a);
+  if (fi == 4) sm_split_kernel<T, C, 4, BB, EPI, PL><<<g, kThreads, 0, st>>>(a);
+  else sm_split_kernel<T, C, 2, BB, EPI, PL><<<g, kThreads, 0, st>>>(a);
 }
 
 // Compile-time epilogues for the launches of a preconditioner application and of block
@@ -545,6 +552,7 @@ template <int C>
 void launch_epi(const SplitArgs& a, hipStream_t st) {
   const int epi = (a.prev ? kEpiPrev : 0) | (a.mask_a ? kEpiMaskA : 0) | (a.mask_b ? kEpiMaskB : 0) |
                   (a.partials ? kEpiDot0 : 0) | (a.partials && a.dot1 ? kEpiDot1 : 0);
+  if (a.is_bf16) return a.B > 1 ? launch<C, 2, 0, false, bf16>(a, st) : launch<C, 1, 0, false, bf16>(a, st);
   if (epi == 0 && a.pool_out) return launch<C, 1, 0, true>(a, st);
   if (epi == 0 && a.B > 1) return launch<C, 2, 0, false>(a, st);
   if (epi == 0) return launch<C, 1, 0, false>(a, st);
@@ -586,6 +594,7 @@ int launch_sm_split(int C, const SplitArgs& a, hipStream_t st) {
                 a.n3, C);
   const bool epi = a.prev || a.mask_a || a.mask_b || a.partials;
   MLPCG_REQUIRE(a.B >= 1 && (a.B == 1 || (!epi && !a.pool_out)), "sm_split: epilogues need B = 1");
+  MLPCG_REQUIRE(!a.is_bf16 || (!epi && !a.pool_out), "sm_split: BF16 blocks have no epilogue");
   MLPCG_REQUIRE((!a.partials || a.dot0) && (!a.dot1 || a.dot0), "sm_split: dot sums need dot0");
   MLPCG_REQUIRE(!a.pool_out || (!epi && a.n1 % 2 == 0 && a.n2 % 2 == 0 && a.n3 % 2 == 0),
                 "sm_split: the pooled output needs an even grid and no epilogue operands");
