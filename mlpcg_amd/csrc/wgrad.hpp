@@ -24,7 +24,7 @@
 // LDS reads, about equally, then by the staging of the tiles (a third of the time), all above
 // the matrix products.  Before (FP32 matrix products gathered from global memory or staged
 // rows, C = 3 on the VALU) -> now: 128^3 FP32 C = 1 88 -> 28 us, two right-hand sides 238 ->
-// 37 us, C = 3 576 -> 98 us; 256^3 C = 1 712 -> 178 us.  Errors against 64 bits (norm-wise):
+// 37 us, C = 3 576 -> 76 us; 256^3 C = 1 712 -> 178 us.  Errors against 64 bits (norm-wise):
 // 0.8 to 1.4e-7 where the FP32 products had 0.8 to 3.3e-7.
 #pragma once
 
@@ -148,8 +148,9 @@ __device__ __forceinline__ void products(float g, const float (&x)[8], float (&G
   for (int j = 0; j < 8; ++j) G[j] = ACC ? __builtin_fmaf(gb[j], x[j], G[j]) : gb[j] * x[j];
 }
 
-// registers for this many waves per SIMD
-__host__ __device__ constexpr int waves(int C, int BB) { return C == 1 ? 4 : 2; }
+// registers for this many waves per SIMD: what keeps the kernels from spilling (C = 3 at two
+// waves: 320 bytes of scratch, 128^3 98 us against 76, 256^3 850 against 488)
+__host__ __device__ constexpr int waves(int C, int BB) { return C == 1 ? (BB == 1 ? 3 : 2) : 1; }
 
 // BB: right-hand sides staged together
 template <typename T, int C, int BB>
