@@ -138,7 +138,8 @@ def ptr(t) -> int | None:
 def stream_ptr(device=None) -> int:
     """The current stream of a device, as a handle (without the Stream object that
     torch.cuda.current_stream builds: 2 us a call)."""
-    if isinstance(device, torch.device) and device.index is not None and torch.cuda.is_initialized():
+    if (isinstance(device, torch.device) and device.type == "cuda" and device.index is not None
+            and torch.cuda.is_initialized()):
         return torch._C._cuda_getCurrentRawStream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 

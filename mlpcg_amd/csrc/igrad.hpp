@@ -69,8 +69,7 @@ template <typename TI, int C, int R, int BB>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ig_waves(C, BB), 8)))
 void igrad_kernel(IgradArgs a) {
   constexpr int PJ = R + 4, FI = kIgPlanes, kCells = tile_cells(FI, PJ);
-  // a BF16 image is exact in one FP16 value, and 11 bits of the weights are more than the
-  // result keeps
+  // a BF16 image is exact in one FP16 value
   constexpr bool FULL = sizeof(TI) == 4;
   __shared__ __attribute__((aligned(16))) f16 ih[C * kCells], il[FULL ? C * kCells : 8];
   __shared__ unsigned sh[8];
@@ -90,7 +89,7 @@ void igrad_kernel(IgradArgs a) {
   const ImageTile it = stage_image<C, FI, PJ, FULL>(ri, hd->img_limit, w, lane, ih, il, sh);
   const int i = i0 + w;
   if (i >= a.n1) return;  // uniform; no barrier follows
-  Weights<C, FULL> W;
+  Weights<C> W;
   W.load(a.pack, lane);
   W.set_bias(((const float*)((const char*)a.pack + kHeaderBytes + pack_w_bytes(C)))[lane & 31] * pow2(it.exp), h);
   const float inv_i = pow2(-it.exp), inv_w = hd->inv_scale;
@@ -152,7 +151,7 @@ void igrad_kernel(IgradArgs a) {
       load_g(j + 1);
       if ((unsigned)j < (unsigned)a.n2) {  // uniform
         f16x K[2];
-        stencils<C, LO, FULL>(W, ih, il, kCells, wb, s * kPitch, K);
+        stencils<C, LO>(W, ih, il, kCells, wb, s * kPitch, K);
         if (ragged) {  // uniform: cells past the grid add nothing, whatever K is there
 #pragma unroll
           for (int k = 0; k < 15; ++k) {
@@ -304,7 +303,7 @@ size_t fused_sgrad_bytes(int n1, int n2, int n3) {
 
 // Time of launch_igrad and the packing, stored K and its transposed gather -> now: FP32 C = 1
 // 256^3 835 -> 215 us, 128^3 98 -> 41 us, two right-hand sides 119 -> 56 us, 64^3 25 -> 19 us;
-// C = 3 256^3 1730 -> 520 us; BF16 256^3 C = 1 280 (nine BF16 column sums) -> 168 us.  Errors
+// C = 3 256^3 1730 -> 520 us; BF16 256^3 C = 1 280 (nine BF16 column sums) -> 181 us, C = 3 409 -> 390 us.  Errors
 // against 64 bits (norm-wise): FP32 0.9 to 1.4e-7 (was 1.1 to 1.5e-7), BF16 1.7e-3, the
 // result's rounding (was 2.1 to 2.5e-3).
 int launch_igrad(int dtype, const void* img, const void* pack, const void* g, void* dx, void* work, size_t bytes, int C,

@@ -274,17 +274,15 @@ __device__ __forceinline__ ImageTile stage_image(const Raw<FI, PJ> (&raw)[C], in
 }
 
 // A lane's packed weights, and the first product of one chunk for one z parity.
-// WL = false: hi alone (11 bits, for results of 8; the bias keeps 22).
-template <int C, bool WL = true>
+template <int C>
 struct Weights {
-  static constexpr int kParts = WL ? 2 : 1;
-  h8 w[2][kParts][2][C];  // [parity][hi, lo][k half][channel]
+  h8 w[2][2][2][C];  // [parity][hi, lo][k half][channel]
   __device__ __forceinline__ void load(const void* pack, int lane) {
     const f16* p = (const f16*)((const char*)pack + kHeaderBytes);
 #pragma unroll
     for (int par = 0; par < 2; ++par)
 #pragma unroll
-      for (int part = 0; part < kParts; ++part)
+      for (int part = 0; part < 2; ++part)
 #pragma unroll
         for (int kc = 0; kc < 2; ++kc)
 #pragma unroll
@@ -297,8 +295,8 @@ struct Weights {
     const f16 hi = (f16)b, lo = (f16)(b - (float)hi), rest = (f16)(b - (float)hi - (float)lo);
 #pragma unroll
     for (int par = 0; par < 2; ++par) {
-      w[par][0][1][0][spare_slot(par)] = h == 0 ? hi : WL ? rest : lo;
-      if constexpr (WL) w[par][1][1][0][spare_slot(par)] = h == 0 ? lo : (f16)0.f;
+      w[par][0][1][0][spare_slot(par)] = h == 0 ? hi : rest;
+      w[par][1][1][0][spare_slot(par)] = h == 0 ? lo : (f16)0.f;
     }
   }
 };
@@ -335,8 +333,8 @@ __device__ __forceinline__ void operands(const f16* arr, const WordBase& wb, int
   b[1][1] = __builtin_bit_cast(h8, u32x4s{o4, both_hi(e[0], e[1]), both_hi(e[2], e[3]), (e4 & 0xffff0000u) | one_lo});
 }
 // scaled K of the lane's columns for both parities, from the tile at `cell`
-template <int C, bool LO, bool WL>
-__device__ __forceinline__ void stencils(const Weights<C, WL>& W, const f16* hi, const f16* lo, int cells,
+template <int C, bool LO>
+__device__ __forceinline__ void stencils(const Weights<C>& W, const f16* hi, const f16* lo, int cells,
                                          const WordBase& wb, int cell, f16x (&K)[2]) {
 #pragma unroll
   for (int c = 0; c < C; ++c) {
@@ -349,8 +347,7 @@ __device__ __forceinline__ void stencils(const Weights<C, WL>& W, const f16* hi,
 #pragma unroll
       for (int kc = 0; kc < 2; ++kc) {
         const f16x in = c == 0 && kc == 0 ? f16x{} : K[par];
-        if constexpr (WL) K[par] = __builtin_amdgcn_mfma_f32_32x32x16_f16(W.w[par][1][kc][c], bh[par][kc], in, 0, 0, 0);
-        else K[par] = in;
+        K[par] = __builtin_amdgcn_mfma_f32_32x32x16_f16(W.w[par][1][kc][c], bh[par][kc], in, 0, 0, 0);
         if (LO) K[par] = __builtin_amdgcn_mfma_f32_32x32x16_f16(W.w[par][0][kc][c], bl[par][kc], K[par], 0, 0, 0);
         K[par] = __builtin_amdgcn_mfma_f32_32x32x16_f16(W.w[par][0][kc][c], bh[par][kc], K[par], 0, 0, 0);
       }
@@ -365,8 +362,7 @@ __host__ __device__ constexpr int split_waves(int C, int BB) { return C == 1 ? (
 
 // The apply.  EPI: compile-time epilogue (kEpiRuntime: every operand tested), PL: also write
 // the 2x2x2 means of y; BB: right-hand sides per workgroup (K is shared by them).  T: the type of
-// x, image and y; a BF16 image is exact in one FP16 value, and 11 bits of the weights are more
-// than a BF16 result keeps.
+// x, image and y; a BF16 image is exact in one FP16 value.
 template <typename T, int C, int FI, int BB, int EPI, bool PL>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(split_waves(C, BB), 8)))
 void sm_split_kernel(SplitArgs a) {
@@ -404,7 +400,7 @@ void sm_split_kernel(SplitArgs a) {
   xany = __builtin_amdgcn_ballot_w64(xany != 0) != 0;
   if (lane == 0) sh[8 + w] = xany;
   const ImageTile it = stage_image<C, FI, kPJ, FULL>(ri, hd->img_limit, w, lane, ih, il, sh);
-  Weights<C, FULL> W;
+  Weights<C> W;
   W.load(a.pack, lane);
   W.set_bias(((const float*)((const char*)a.pack + kHeaderBytes + pack_w_bytes(C)))[lane & 31] * pow2(it.exp), h);
   // x = 0 everywhere: every finite K gives y = 0
@@ -459,7 +455,7 @@ void sm_split_kernel(SplitArgs a) {
       const bool skip = zero || (LB && has_b && __builtin_amdgcn_ballot_w64(zok && kb != 0) == 0);
       if (!skip) {
         f16x K[2];
-        stencils<C, LO, FULL>(W, ih, il, kCells, wb, cell, K);
+        stencils<C, LO>(W, ih, il, kCells, wb, cell, K);
 #pragma unroll
         for (int bb = 0; bb < BB; ++bb) {
           float pe = 0.f, po = 0.f;
@@ -598,9 +594,18 @@ int launch_sm_split(int C, const SplitArgs& a, hipStream_t st) {
   MLPCG_REQUIRE((!a.partials || a.dot0) && (!a.dot1 || a.dot0), "sm_split: dot sums need dot0");
   MLPCG_REQUIRE(!a.pool_out || (!epi && a.n1 % 2 == 0 && a.n2 % 2 == 0 && a.n3 % 2 == 0),
                 "sm_split: the pooled output needs an even grid and no epilogue operands");
-  if (C == 1) split::launch_epi<1>(a, st);
-  else if (C == 2) split::launch_epi<2>(a, st);
-  else split::launch_epi<3>(a, st);
+  // a launch takes 65535 workgroups of two right-hand sides at most
+  constexpr int kMost = 2 * 65535;
+  const size_t V = (size_t)a.n1 * a.n2 * a.n3, es = a.is_bf16 ? 2 : 4;
+  for (int b = 0; b < a.B; b += kMost) {
+    SplitArgs p = a;
+    p.x = (const float*)((const char*)a.x + (size_t)b * V * es);
+    p.y = (float*)((char*)a.y + (size_t)b * V * es);
+    p.B = a.B - b < kMost ? a.B - b : kMost;
+    if (C == 1) split::launch_epi<1>(p, st);
+    else if (C == 2) split::launch_epi<2>(p, st);
+    else split::launch_epi<3>(p, st);
+  }
   return check_launch("sm_split");
 }
 

@@ -59,7 +59,7 @@ def test_input_gradient(dev, dtype, C, B, shape, kind):
         bound = mag * (2.0 ** -21 + 64 * 2.0 ** -24)
         norm = 32 * 2.0 ** -24
     else:
-        # weights rounded to 11 bits, 2^-12, FP32 sums, the result rounded to BF16
+        # room for weights of 11 bits, 2^-12, FP32 sums, the result rounded to BF16
         bound = mag * (2.0 ** -12 + 64 * 2.0 ** -24) + ref.abs() * 2.0 ** -8
         norm = 2.0 ** -8
     tiny = float(mag.max()) * 2.0 ** -40

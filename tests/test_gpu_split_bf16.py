@@ -31,6 +31,6 @@ def test_bf16_block_forward(dev, C, B, shape):
     for p, xs in enumerate(shifts(x.double()[:, 0])):
         ref += ((W[p] @ P).reshape(shape) + b.double()[p]) * xs
         mag += ((W[p].abs() @ P).reshape(shape) + b.double()[p].abs()) * xs.abs()
-    # weights to 11 bits (2^-12), FP32 sums, the result rounded to BF16 (2^-9)
+    # room for weights of 11 bits (2^-12), FP32 sums, the result rounded to BF16 (2^-9)
     assert torch.all((y - ref).abs() <= mag * (2.0 ** -12 + 64 * 2.0 ** -24) + ref.abs() * 2.0 ** -8)
     assert float((y - ref).norm() / ref.norm()) <= 2.0 ** -8
