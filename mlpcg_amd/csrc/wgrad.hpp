@@ -3,14 +3,18 @@
 // with P_q the 27 C image taps and a column of ones (the bias gradient), a 27 x (27C + 1)
 // product over all voxels: gW[p][q] = D[p][q], gb[p] = D[p][27C].
 //
-// a, c and the image are scaled by powers of two (from the tiles' largest finite magnitudes) and G, formed in FP32, and P are split into two FP16 values each (see
-// split_common.hpp); D = G_hi P_hi + G_lo P_hi + G_hi P_lo on v_mfma_f32_32x32x16_f16.  For
-// BF16 data G is exact in its two parts and P in one, so every product is exact; tiles whose
-// image has no low part leave the third product out.  The products with a low part have
-// accumulators of their own: fewer roundings of the large sums (and the matrix cores cut,
-// not round, what is far below their largest addend: adding all three to fresh accumulators
-// per row doubled the error).  A workgroup keeps its smallest factors so far; where a tile
-// needs a smaller one, the sums are rescaled (exact).
+// a, c and the image are scaled by powers of two and G, formed in FP32, and P are split into
+// two FP16 values each (see split_common.hpp); D = G_hi P_hi + G_lo P_hi + G_hi P_lo on
+// v_mfma_f32_32x32x16_f16.  For BF16 data G is exact in its two parts and P in one, so every
+// product is exact; tiles whose image has no low part leave the third product out.  The
+// products with a low part have accumulators of their own: fewer roundings of the large sums
+// (and the matrix cores cut, not round, what is far below their largest addend: adding all
+// three to fresh accumulators per row doubled the error).
+//
+// The factors of a and c (per right-hand side) and of each image channel come from the tile's
+// own largest finite magnitudes, and a tile's products are added, scaled back, to FP32 sums
+// kept beside its accumulators: no tile's factor reaches another's, whether that is empty or
+// its values are far larger.
 //
 // Tile: 4 planes x 8 rows x 64 z; x and the image with a one-cell halo in LDS, any extents.
 // A wave takes rows of 64 voxels, 16 voxels per product: lane (h, m) = (lane / 32, lane % 32)
@@ -42,7 +46,7 @@ constexpr int kIRow = 68, kIPlane = 716;      // image pitches (half words); cel
 constexpr int kXCells = (kI + 2) * kXPlane, kICells = (kI + 2) * kIPlane;
 static_assert(kXRow % 32 == 3 && kXPlane % 32 == 9 && (kIRow / 2) % 32 == 2 && (kIPlane / 2) % 32 == 6, "banks");
 static_assert(kXPlane >= kPJ * kXRow && kIPlane >= kPJ * kIRow, "planes do not overlap");
-constexpr int kTargetG = 6, kTargetP = 4;  // |a|, |c| into [2^6, 2^7), |image| into [2^4, 2^5)
+constexpr int kTargetG = 6, kTargetP = 14;  // |a|, |c| into [2^6, 2^7), |image| into [2^14, 2^15)
 constexpr int kOnes = 40;                  // words of FP16 ones, and of zeros, for the bias column
 constexpr int kRw = 3;                     // staged rows per wave and plane: j = w, w + 4, w + 8 of 10
 static_assert(2 * kRows <= kThreads, "staging");
@@ -161,7 +165,7 @@ void wgrad_kernel(const T* __restrict__ a, const T* __restrict__ cv, int B, cons
   constexpr int kXB = BB * kXCells * 4, kIB = C * kICells * 2, kRed = 4 * 32 * 32 * 4;
   constexpr int kOnesAt = kXB + 2 * kIB, kUsed = kOnesAt + 2 * kOnes * 4;
   __shared__ __attribute__((aligned(16))) char lds[kUsed > kRed ? kUsed : kRed];
-  __shared__ unsigned sh[4][4];
+  __shared__ unsigned sh[4][2 * BB + C + 1];
   float* xs = (float*)lds;      // [BB][kXCells]
   f16* ih = (f16*)(lds + kXB);  // [C][kICells], then the low parts
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -191,24 +195,10 @@ void wgrad_kernel(const T* __restrict__ a, const T* __restrict__ cv, int B, cons
     lo_o[t] = o1 ? kOnesAt / 4 + kOnes : (kXB + kIB) / 4 + word;
     ish[t] = s % 3 == 1 ? 0 : 16;
   }
-  // the products of the high parts, and those with a low part: both in units of the block's
-  // scales so far (the smallest factors of its tiles)
-  f16x acc[NT], acl[NT];
+  // sums over the tiles so far
+  f16x sum[NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) acc[t] = acl[t] = f16x{};
-  int ex = 126, eg = 126, ei = 126;
-  auto rescale = [&](int exg, int eimg) {  // by 2^exg, and 2^eimg but for the column of ones
-    if (exg == 0 && eimg == 0) return;
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-      const int e = exg + (t == kOneTile && one ? 0 : eimg);
-#pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        acc[t][i] = ldexpf(acc[t][i], e);
-        acl[t][i] = ldexpf(acl[t][i], e);
-      }
-    }
-  };
+  for (int t = 0; t < NT; ++t) sum[t] = f16x{};
 
   for (unsigned tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
     const unsigned u = tile / tz;
@@ -230,9 +220,9 @@ void wgrad_kernel(const T* __restrict__ a, const T* __restrict__ cv, int B, cons
       }
     };
     bool has_lo = false;
+    int ei[C];  // exponents of the image's factors
     for (int b0 = 0; b0 < B; b0 += BB) {
       Raw ri[C], rx[BB];
-      float mi = 0.f, mx = 0.f, mg = 0.f;
       if (b0 == 0) {
 #pragma unroll
         for (int c = 0; c < C; ++c) load_tile(ri[c], img + c * V, pos, n1, n2, n3, w, lane);
@@ -247,69 +237,88 @@ void wgrad_kernel(const T* __restrict__ a, const T* __restrict__ cv, int B, cons
 #pragma unroll
         for (int q = 0; q < kI * kJ / 4; ++q)
           rg[bb][q] = ld_as(row_of_a(b0 + bb, q), (unsigned)(pos.z0 + lane) * (unsigned)sizeof(T), 0, a);
-      if (b0 == 0) {
-#pragma unroll
-        for (int c = 0; c < C; ++c) mi = fmaxf(mi, max_of(ri[c]));
-      }
+      // largest magnitudes: c and a of each right-hand side, the image's channels
+      float mf[2 * BB + C];
 #pragma unroll
       for (int bb = 0; bb < BB; ++bb) {
-        mx = fmaxf(mx, max_of(rx[bb]));
+        mf[2 * bb] = max_of(rx[bb]);
+        float m = 0.f;
 #pragma unroll
-        for (int q = 0; q < kI * kJ / 4; ++q) mg = fmaxf(mg, fabsf(rg[bb][q]));
+        for (int q = 0; q < kI * kJ / 4; ++q) m = fmaxf(m, fabsf(rg[bb][q]));
+        mf[2 * bb + 1] = m;
       }
-      unsigned bi = __float_as_uint(mi), bx = __float_as_uint(mx), bg = __float_as_uint(mg);
-      if (__builtin_amdgcn_ballot_w64(max(bi, max(bx, bg)) >= 0x7f800000u)) {  // infinities set no scale
-        bi = bx = bg = 0;
-        if (b0 == 0)
-          for (int c = 0; c < C; ++c) bi = max(bi, finite_max_of(ri[c]));
+#pragma unroll
+      for (int c = 0; c < C; ++c) mf[2 * BB + c] = b0 == 0 ? max_of(ri[c]) : 0.f;
+      unsigned mu[2 * BB + C], all = 0;
+#pragma unroll
+      for (int k = 0; k < 2 * BB + C; ++k) all = max(all, mu[k] = __float_as_uint(mf[k]));
+      if (__builtin_amdgcn_ballot_w64(all >= 0x7f800000u)) {  // infinities set no scale
         for (int bb = 0; bb < BB; ++bb) {
-          bx = max(bx, finite_max_of(rx[bb]));
-          for (int q = 0; q < kI * kJ / 4; ++q) bg = max(bg, finite_bits(rg[bb][q]));
+          mu[2 * bb] = finite_max_of(rx[bb]);
+          mu[2 * bb + 1] = 0;
+          for (int q = 0; q < kI * kJ / 4; ++q) mu[2 * bb + 1] = max(mu[2 * bb + 1], finite_bits(rg[bb][q]));
         }
+        for (int c = 0; c < C; ++c) mu[2 * BB + c] = b0 == 0 ? finite_max_of(ri[c]) : 0u;
       }
-      bi = wave_max(bi);
-      bx = wave_max(bx);
-      bg = wave_max(bg);
+#pragma unroll
+      for (int k = 0; k < 2 * BB + C; ++k) mu[k] = wave_max(mu[k]);
       __syncthreads();  // the previous tile's reads are done
       if (lane == 0) {
-        sh[w][0] = bi;
-        sh[w][1] = bx;
-        sh[w][2] = bg;
+#pragma unroll
+        for (int k = 0; k < 2 * BB + C; ++k) sh[w][k] = mu[k];
       }
       __syncthreads();
       auto over_waves = [&](int k) {
         return (unsigned)__builtin_amdgcn_readfirstlane((int)max(max(sh[0][k], sh[1][k]), max(sh[2][k], sh[3][k])));
       };
-      const int ex_n = min(ex, scale_exp(over_waves(1), kTargetG)), eg_n = min(eg, scale_exp(over_waves(2), kTargetG));
-      const int ei_n = b0 == 0 ? min(ei, scale_exp(over_waves(0), kTargetP)) : ei;
-      rescale(ex_n - ex + eg_n - eg, ei_n - ei);
-      ex = ex_n;
-      eg = eg_n;
-      ei = ei_n;
-      const float sx = pow2(ex), sg = pow2(eg);
+      if (b0 == 0) {
 #pragma unroll
-      for (int bb = 0; bb < BB; ++bb)
-        each(rx[bb], w, lane, [&](int k, int j, int e, float v) {
-          xs[bb * kXCells + k * kXPlane + j * kXRow + e] = v * sx;
+        for (int c = 0; c < C; ++c) ei[c] = scale_exp(over_waves(2 * BB + c), kTargetP);
+      }
+      // G in units of 2^-e, the largest that a right-hand side's own factors give (they add up
+      // in G; one of zeros has no say, and one 2^100 below the other adds nothing)
+      int ex[BB], e = 2 * 126;
+      bool some[BB];
+#pragma unroll
+      for (int bb = 0; bb < BB; ++bb) {
+        const unsigned bx = over_waves(2 * bb), bg = over_waves(2 * bb + 1);
+        ex[bb] = scale_exp(bx, kTargetG);
+        some[bb] = bx != 0u && bg != 0u;
+        if (some[bb]) e = min(e, ex[bb] + scale_exp(bg, kTargetG));
+      }
+      float sg[BB];
+#pragma unroll
+      for (int bb = 0; bb < BB; ++bb) sg[bb] = some[bb] && e - ex[bb] >= -126 ? pow2(e - ex[bb]) : 0.f;
+#pragma unroll
+      for (int bb = 0; bb < BB; ++bb) {
+        const float sx = pow2(ex[bb]);
+        each(rx[bb], w, lane, [&](int k, int j, int z, float v) {
+          xs[bb * kXCells + k * kXPlane + j * kXRow + z] = v * sx;
         });
+      }
       if (b0 == 0) {
         unsigned any = 0;
-        const float si = pow2(ei);
 #pragma unroll
-        for (int c = 0; c < C; ++c)
-          each(ri[c], w, lane, [&](int k, int j, int e, float v) {
+        for (int c = 0; c < C; ++c) {
+          const float si = pow2(ei[c]);
+          each(ri[c], w, lane, [&](int k, int j, int z, float v) {
             const float sv = v * si;
             const f16 hi = (f16)sv, lo = (f16)(sv - (float)hi);
-            f16* d = ih + c * kICells + k * kIPlane + j * kIRow + 1 + e;
+            f16* d = ih + c * kICells + k * kIPlane + j * kIRow + 1 + z;
             d[0] = hi;
             d[C * kICells] = lo;
             any |= __builtin_bit_cast(unsigned short, lo);
           });
+        }
         any = __builtin_amdgcn_ballot_w64((any & 0x7fffu) != 0) != 0;
-        if (lane == 0) sh[w][3] = any;
+        if (lane == 0) sh[w][2 * BB + C] = any;
       }
       __syncthreads();
-      if (b0 == 0) has_lo = over_waves(3) != 0;
+      if (b0 == 0) has_lo = over_waves(2 * BB + C) != 0;
+      // the products of the high parts, and those with a low part
+      f16x acc[NT], acl[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t] = acl[t] = f16x{};
 
       auto rows = [&](auto lo_c) {
         constexpr bool LO = decltype(lo_c)::value;
@@ -361,8 +370,8 @@ void wgrad_kernel(const T* __restrict__ a, const T* __restrict__ cv, int B, cons
             float G[8];
 #pragma unroll
             for (int bb = 0; bb < BB; ++bb) {
-              if (bb == 0) products<false>(gc[bb][s] * sg, cur.x[bb], G);
-              else products<true>(gc[bb][s] * sg, cur.x[bb], G);
+              if (bb == 0) products<false>(gc[bb][s] * sg[bb], cur.x[bb], G);
+              else products<true>(gc[bb][s] * sg[bb], cur.x[bb], G);
             }
             u32x4s gh, gl;
 #pragma unroll
@@ -402,6 +411,14 @@ void wgrad_kernel(const T* __restrict__ a, const T* __restrict__ cv, int B, cons
       };
       if (has_lo) rows(std::true_type());
       else rows(std::false_type());
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        int u = -e;  // the column's scale: of G, and of the image's channel
+#pragma unroll
+        for (int c = 0; c < C; ++c) u -= (32 * t + m) / 27 == c && 32 * t + m < 27 * C ? ei[c] : 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) sum[t][i] += ldexpf(acc[t][i] + acl[t][i], u);
+      }
     }
   }
   // D[8 (i / 4) + 4 h + i % 4][32 t + m] of the wave, the waves added in order
@@ -411,8 +428,7 @@ void wgrad_kernel(const T* __restrict__ a, const T* __restrict__ cv, int B, cons
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 16; ++i)
-      red[(w * 32 + 8 * (i >> 2) + 4 * h + (i & 3)) * 32 + m] =
-          ldexpf(acc[t][i] + acl[t][i], -ex - eg - (t == kOneTile && one ? 0 : ei));
+      red[(w * 32 + 8 * (i >> 2) + 4 * h + (i & 3)) * 32 + m] = sum[t][i];
     __syncthreads();
     for (int e = threadIdx.x; e < 27 * 32; e += kThreads) {
       const int pp = e >> 5, q = 32 * t + (e & 31);
