@@ -465,6 +465,8 @@ int wgrad_blocks(int most, int n1, int n2, int n3) { return wgrad::blocks(most, 
 
 int launch_wgrad(int dtype, const void* a, const void* c, const void* img, float* part, int nblk, int C, int B, int n1,
                  int n2, int n3, hipStream_t st) {
+  MLPCG_REQUIRE((long)n1 * n2 * n3 * (dtype == kF32 ? 4 : 2) < (1L << 31), "weight_grad: grid (%d,%d,%d) too large", n1,
+                n2, n3);
   if (dtype == kF32) wgrad::launch<float>(a, c, img, part, nblk, C, B, n1, n2, n3, st);
   else if (dtype == kF16) wgrad::launch<f16>(a, c, img, part, nblk, C, B, n1, n2, n3, st);
   else if (dtype == kBF16) wgrad::launch<bf16>(a, c, img, part, nblk, C, B, n1, n2, n3, st);
