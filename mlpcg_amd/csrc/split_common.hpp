@@ -21,11 +21,20 @@ __device__ __forceinline__ unsigned finite_bits(float v) {
   const unsigned u = __float_as_uint(v) & 0x7fffffffu;
   return u < 0x7f800000u ? u : 0u;
 }
+__device__ __forceinline__ unsigned magnitude(float v) { return __float_as_uint(v) & 0x7fffffffu; }
+constexpr unsigned kInfinity = 0x7f800000u;
+// the larger one, NaN if one is (v_maximum3_f32)
+__device__ __forceinline__ float max_nan(float a, float b) { return __builtin_elementwise_maximum(a, b); }
+// a magnitude in the order of its size, 0 above all (v_lshl_add_u32)
+__device__ __forceinline__ unsigned small_bits(float v) { return (__float_as_uint(v) << 1) - 1u; }
 // 2^e of the largest finite magnitude (its bits); 0 counts as 1
 __device__ __forceinline__ int exponent_of(unsigned bits) {
   return bits == 0u ? 0 : (int)(bits >> 23) - 127;
 }
 __device__ __forceinline__ float pow2(int e) { return __uint_as_float((unsigned)(e + 127) << 23); }
+// small_bits of 2^-2 before a scaling by 2^e: smaller values have fewer than 23 bits in two FP16
+// values (2^-24 is FP16's smallest step)
+__device__ __forceinline__ unsigned least_bits(int e) { return small_bits(ldexpf(0.25f, -e)); }
 
 __device__ __forceinline__ unsigned wave_max(unsigned v) {
   auto step = [](unsigned x, auto ctrl, auto rows) {

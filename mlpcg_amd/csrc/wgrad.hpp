@@ -14,7 +14,13 @@
 // The factors of a and c (per right-hand side) and of each image channel come from the tile's
 // own largest finite magnitudes, and a tile's products are added, scaled back, to FP32 sums
 // kept beside its accumulators: no tile's factor reaches another's, whether that is empty or
-// its values are far larger.
+// its values are far larger.  FP16's smallest step is then 2^-39 of the largest |a| |c| and of
+// the largest |image| of a tile.  Where that is not enough (no product of the tile's centre taps
+// within 2^-16 of that bound, or three image cells in a row that are all 2^-16 and more below
+// it), and in tiles with infinities or NaN, FP32 products are summed on the VALU, over the cells
+// and taps inside the grid alone (some 20 times slower, for a kind of tile that is rare).  Such
+// tiles wait until the workgroup's others are done: among them, that code's registers and
+// instructions cost every tile 5 %.
 //
 // Tile: 4 planes x 8 rows x 64 z; x and the image with a one-cell halo in LDS, any extents.
 // A wave takes rows of 64 voxels, 16 voxels per product: lane (h, m) = (lane / 32, lane % 32)
@@ -27,9 +33,9 @@
 // Bound by VALU (3 instructions per G: product, difference, two conversions of pairs) and
 // LDS reads, about equally, then by the staging of the tiles (a third of the time), all above
 // the matrix products.  Before (FP32 matrix products gathered from global memory or staged
-// rows, C = 3 on the VALU) -> now: 128^3 FP32 C = 1 88 -> 28 us, two right-hand sides 238 ->
-// 37 us, C = 3 576 -> 76 us; 256^3 C = 1 712 -> 178 us.  Errors against 64 bits (norm-wise):
-// 0.8 to 1.4e-7 where the FP32 products had 0.8 to 3.3e-7.
+// rows, C = 3 on the VALU) -> now: 128^3 FP32 C = 1 88 -> 30 us, two right-hand sides 238 ->
+// 44 us, C = 3 576 -> 75 us; 256^3 C = 1 712 -> 190 us.  Errors against 64 bits (norm-wise):
+// 0.8 to 1.9e-7 where the FP32 products had 0.8 to 5.2e-7.
 #pragma once
 
 #include "kernels.hpp"
@@ -47,6 +53,7 @@ constexpr int kXCells = (kI + 2) * kXPlane, kICells = (kI + 2) * kIPlane;
 static_assert(kXRow % 32 == 3 && kXPlane % 32 == 9 && (kIRow / 2) % 32 == 2 && (kIPlane / 2) % 32 == 6, "banks");
 static_assert(kXPlane >= kPJ * kXRow && kIPlane >= kPJ * kIRow, "planes do not overlap");
 constexpr int kTargetG = 6, kTargetP = 14;  // |a|, |c| into [2^6, 2^7), |image| into [2^14, 2^15)
+constexpr int kQueue = 32;                 // tiles that wait for their FP32 products
 constexpr int kOnes = 40;                  // words of FP16 ones, and of zeros, for the bias column
 constexpr int kRw = 3;                     // staged rows per wave and plane: j = w, w + 4, w + 8 of 10
 static_assert(2 * kRows <= kThreads, "staging");
@@ -62,27 +69,30 @@ struct Pos {
   int i0, j0, z0;
 };
 
+// (a tensor has fewer than 2^31 bytes, so one resource with 32-bit offsets serves all of its rows;
+// a base for each row or plane filled the scalar registers and beyond)
+constexpr unsigned kOut = 0x80000000u;
 template <typename T>
 __device__ __forceinline__ void load_tile(Raw& r, const T* __restrict__ src, const Pos& t, int n1, int n2, int n3,
                                           int w, int lane) {
-  const long plane = (long)n2 * n3;
-  const int pb = (int)(plane * (long)sizeof(T)), rb = n3 * (int)sizeof(T);
-  const unsigned zo = t.z0 + lane < n3 ? (unsigned)(t.z0 + lane) * (unsigned)sizeof(T) : 0x80000000u;
-  int so[kRw], jb[kRw];  // row offsets; plane bytes, or 0 for rows outside the grid
+  const int rb = n3 * (int)sizeof(T), pb = n2 * rb;
+  const unsigned zo = t.z0 + lane < n3 ? (unsigned)(t.z0 + lane) * (unsigned)sizeof(T) : kOut;
+  int so[kRw];
+  unsigned vo[kRw];  // kOut in rows outside the grid
 #pragma unroll
   for (int u = 0; u < kRw; ++u) {
     const int gj = t.j0 + w + 4 * u - 1;
     const bool ok = (unsigned)gj < (unsigned)n2 && w + 4 * u < kPJ;
     so[u] = ok ? gj * rb : 0;
-    jb[u] = ok ? pb : 0;
+    vo[u] = ok ? zo : kOut;
   }
-  const T* p = src + (t.i0 - 1) * plane;
 #pragma unroll
   for (int k = 0; k < kI + 2; ++k) {
-    const bool ok = (unsigned)(t.i0 + k - 1) < (unsigned)n1;
+    const int gi = t.i0 + k - 1;
+    const bool ok = (unsigned)gi < (unsigned)n1;
+    const auto res = rsrc(src, ok ? n1 * pb : 0);
 #pragma unroll
-    for (int u = 0; u < kRw; ++u) r.m[k][u] = ld_as(rsrc(ok ? p : src, ok ? jb[u] : 0), zo, so[u], src);
-    p += plane;
+    for (int u = 0; u < kRw; ++u) r.m[k][u] = ld_as(res, vo[u], ok ? gi * pb + so[u] : 0, src);
   }
   const int hrow = threadIdx.x >> 1, z = (threadIdx.x & 1) ? t.z0 + kZ : t.z0 - 1;
   const int gi = t.i0 + hrow / kPJ - 1, gj = t.j0 + hrow % kPJ - 1;
@@ -102,13 +112,22 @@ __device__ __forceinline__ void each(const Raw& r, int w, int lane, F&& f) {
   const int hrow = threadIdx.x >> 1;
   if (hrow < kRows) f(hrow / kPJ, hrow % kPJ, (int)(threadIdx.x & 1) * (kZ + 1), r.halo);
 }
-// largest magnitude (NaN aside), infinite if one is
-__device__ __forceinline__ float max_of(const Raw& r) {
+// largest magnitude (bits; kInfinity or more with an infinite or NaN cell)
+__device__ __forceinline__ unsigned max_of(const Raw& r) {
   float m = fabsf(r.halo);
 #pragma unroll
   for (int k = 0; k < kI + 2; ++k)
 #pragma unroll
-    for (int u = 0; u < kRw; ++u) m = fmaxf(m, fabsf(r.m[k][u]));
+    for (int u = 0; u < kRw; ++u) m = max_nan(m, fabsf(r.m[k][u]));
+  return magnitude(m);
+}
+// smallest magnitude that is not 0 (small_bits)
+__device__ __forceinline__ unsigned min_of(const Raw& r) {
+  unsigned m = small_bits(r.halo);
+#pragma unroll
+  for (int k = 0; k < kI + 2; ++k)
+#pragma unroll
+    for (int u = 0; u < kRw; ++u) m = min(m, small_bits(r.m[k][u]));
   return m;
 }
 // the same of the finite cells alone
@@ -122,6 +141,20 @@ __device__ __forceinline__ unsigned finite_max_of(const Raw& r) {
 }
 __device__ __forceinline__ int scale_exp(unsigned bits, int target) {
   return max(-126, min(target - exponent_of(bits), 126));
+}
+// Whether three cells in a row of a tile hold values below `least` only (small_bits), not all 0
+// (the z-halo cells, which other lanes hold, by themselves).  If not, sums over a patch are as
+// good as if the smaller values were held like `least`.
+__device__ __forceinline__ bool has_small_rows(const Raw& r, unsigned least) {
+  bool bad = small_bits(r.halo) < least;
+#pragma unroll
+  for (int k = 0; k < kI + 2; ++k)
+#pragma unroll
+    for (int u = 0; u < kRw; ++u) {
+      const float v = fabsf(r.m[k][u]);
+      bad |= small_bits(fmaxf(v, fmaxf(wave_from_prev(v), wave_from_next(v)))) < least;
+    }
+  return bad;
 }
 // lane I of a row of 16 to the whole row
 template <int I>
@@ -154,7 +187,7 @@ __device__ __forceinline__ void products(float g, const float (&x)[8], float (&G
 
 // registers for this many waves per SIMD: what keeps the kernels from spilling (C = 3 at two
 // waves: 320 bytes of scratch, 128^3 98 us against 76, 256^3 850 against 488)
-__host__ __device__ constexpr int waves(int C, int BB) { return C == 1 ? (BB == 1 ? 3 : 2) : 1; }
+__host__ __device__ constexpr int waves(int C, int BB) { return C == 1 ? (BB == 1 ? 3 : 2) : C == 2 && BB == 1 ? 2 : 1; }
 
 // BB: right-hand sides staged together
 template <typename T, int C, int BB>
@@ -165,7 +198,8 @@ void wgrad_kernel(const T* __restrict__ a, const T* __restrict__ cv, int B, cons
   constexpr int kXB = BB * kXCells * 4, kIB = C * kICells * 2, kRed = 4 * 32 * 32 * 4;
   constexpr int kOnesAt = kXB + 2 * kIB, kUsed = kOnesAt + 2 * kOnes * 4;
   __shared__ __attribute__((aligned(16))) char lds[kUsed > kRed ? kUsed : kRed];
-  __shared__ unsigned sh[4][2 * BB + C + 1];
+  __shared__ unsigned sh[4][2 * BB + C + 3], queue[kQueue][2];
+  constexpr int kFlagA = 2 * BB + C, kFlagB = kFlagA + 1, kFlagC = kFlagA + 2;
   float* xs = (float*)lds;      // [BB][kXCells]
   f16* ih = (f16*)(lds + kXB);  // [C][kICells], then the low parts
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -200,224 +234,356 @@ void wgrad_kernel(const T* __restrict__ a, const T* __restrict__ cv, int B, cons
 #pragma unroll
   for (int t = 0; t < NT; ++t) sum[t] = f16x{};
 
-  for (unsigned tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+  auto tile_at = [&](unsigned tile) {
     const unsigned u = tile / tz;
-    const Pos pos{(int)(u / tj) * kI, (int)(u % tj) * kJ, (int)(tile % tz) * kZ};
-    // a row of a (range-checked: rows and cells outside the grid read 0)
-    auto row_of_a = [&](int b, int q) {
-      const int gi = pos.i0 + (q >> 1), gj = pos.j0 + w + 4 * (q & 1);
-      const bool ok = gi < n1 && gj < n2 && b < B;
-      return rsrc(a + (ok ? (long)b * V + ((long)gi * n2 + gj) * n3 : 0L), ok ? n3 * (int)sizeof(T) : 0);
-    };
-    // the lane's a values of a row: voxels 16 s + 8 h + lane % 8
-    const unsigned go = (unsigned)(pos.z0 + 8 * h + (lane & 7)) * (unsigned)sizeof(T);
-    auto load_g = [&](float (&g)[BB][4], int b0, int q) {
+    return Pos{(int)(u / tj) * kI, (int)(u % tj) * kJ, (int)(tile % tz) * kZ};
+  };
+  // a row of a (range-checked: rows and cells outside the grid read 0)
+  auto a_row = [&](const Pos& pos, int b, int i, int j) {
+    const int gi = pos.i0 + i, gj = pos.j0 + j;
+    const bool ok = gi < n1 && gj < n2 && b < B;
+    return rsrc(a + (ok ? (long)b * V + ((long)gi * n2 + gj) * n3 : 0L), ok ? n3 * (int)sizeof(T) : 0);
+  };
+  unsigned tile = blockIdx.x;
+  for (;;) {
+    int queued = 0;
+    for (; tile < tiles && queued < kQueue; tile += gridDim.x) {
+      const Pos pos = tile_at(tile);
+      // the lane's a values of a row: voxels 16 s + 8 h + lane % 8
+      const unsigned go = (unsigned)(pos.z0 + 8 * h + (lane & 7)) * (unsigned)sizeof(T);
+      auto load_g = [&](float (&g)[BB][4], int b0, int q) {
 #pragma unroll
-      for (int bb = 0; bb < BB; ++bb) {
-        const auto r = row_of_a(b0 + bb, q);
-#pragma unroll
-        for (int s = 0; s < 4; ++s) g[bb][s] = ld_as(r, go + 16 * s * (unsigned)sizeof(T), 0, a);
-      }
-    };
-    bool has_lo = false;
-    int ei[C];  // exponents of the image's factors
-    for (int b0 = 0; b0 < B; b0 += BB) {
-      Raw ri[C], rx[BB];
-      if (b0 == 0) {
-#pragma unroll
-        for (int c = 0; c < C; ++c) load_tile(ri[c], img + c * V, pos, n1, n2, n3, w, lane);
-      }
-      // (an absent right-hand side repeats the last: its a reads as 0)
-#pragma unroll
-      for (int bb = 0; bb < BB; ++bb) load_tile(rx[bb], cv + (long)min(b0 + bb, B - 1) * V, pos, n1, n2, n3, w, lane);
-      // a's rows, for the scale only (the products read them again, from L2)
-      float rg[BB][kI * kJ / 4];
-#pragma unroll
-      for (int bb = 0; bb < BB; ++bb)
-#pragma unroll
-        for (int q = 0; q < kI * kJ / 4; ++q)
-          rg[bb][q] = ld_as(row_of_a(b0 + bb, q), (unsigned)(pos.z0 + lane) * (unsigned)sizeof(T), 0, a);
-      // largest magnitudes: c and a of each right-hand side, the image's channels
-      float mf[2 * BB + C];
-#pragma unroll
-      for (int bb = 0; bb < BB; ++bb) {
-        mf[2 * bb] = max_of(rx[bb]);
-        float m = 0.f;
-#pragma unroll
-        for (int q = 0; q < kI * kJ / 4; ++q) m = fmaxf(m, fabsf(rg[bb][q]));
-        mf[2 * bb + 1] = m;
-      }
-#pragma unroll
-      for (int c = 0; c < C; ++c) mf[2 * BB + c] = b0 == 0 ? max_of(ri[c]) : 0.f;
-      unsigned mu[2 * BB + C], all = 0;
-#pragma unroll
-      for (int k = 0; k < 2 * BB + C; ++k) all = max(all, mu[k] = __float_as_uint(mf[k]));
-      if (__builtin_amdgcn_ballot_w64(all >= 0x7f800000u)) {  // infinities set no scale
         for (int bb = 0; bb < BB; ++bb) {
-          mu[2 * bb] = finite_max_of(rx[bb]);
-          mu[2 * bb + 1] = 0;
-          for (int q = 0; q < kI * kJ / 4; ++q) mu[2 * bb + 1] = max(mu[2 * bb + 1], finite_bits(rg[bb][q]));
+          const auto r = a_row(pos, b0 + bb, q >> 1, w + 4 * (q & 1));
+#pragma unroll
+          for (int s = 0; s < 4; ++s) g[bb][s] = ld_as(r, go + 16 * s * (unsigned)sizeof(T), 0, a);
         }
-        for (int c = 0; c < C; ++c) mu[2 * BB + c] = b0 == 0 ? finite_max_of(ri[c]) : 0u;
-      }
-#pragma unroll
-      for (int k = 0; k < 2 * BB + C; ++k) mu[k] = wave_max(mu[k]);
-      __syncthreads();  // the previous tile's reads are done
-      if (lane == 0) {
-#pragma unroll
-        for (int k = 0; k < 2 * BB + C; ++k) sh[w][k] = mu[k];
-      }
-      __syncthreads();
-      auto over_waves = [&](int k) {
-        return (unsigned)__builtin_amdgcn_readfirstlane((int)max(max(sh[0][k], sh[1][k]), max(sh[2][k], sh[3][k])));
       };
-      if (b0 == 0) {
+      bool has_lo = false;
+      int ei[C];  // exponents of the image's factors
+      for (int b0 = 0; b0 < B; b0 += BB) {
+        Raw ri[C], rx[BB];
+        if (b0 == 0) {
 #pragma unroll
-        for (int c = 0; c < C; ++c) ei[c] = scale_exp(over_waves(2 * BB + c), kTargetP);
-      }
-      // G in units of 2^-e, the largest that a right-hand side's own factors give (they add up
-      // in G; one of zeros has no say, and one 2^100 below the other adds nothing)
-      int ex[BB], e = 2 * 126;
-      bool some[BB];
+          for (int c = 0; c < C; ++c) load_tile(ri[c], img + c * V, pos, n1, n2, n3, w, lane);
+        }
+        // (an absent right-hand side repeats the last: its a reads as 0)
 #pragma unroll
-      for (int bb = 0; bb < BB; ++bb) {
-        const unsigned bx = over_waves(2 * bb), bg = over_waves(2 * bb + 1);
-        ex[bb] = scale_exp(bx, kTargetG);
-        some[bb] = bx != 0u && bg != 0u;
-        if (some[bb]) e = min(e, ex[bb] + scale_exp(bg, kTargetG));
-      }
-      float sg[BB];
+        for (int bb = 0; bb < BB; ++bb) load_tile(rx[bb], cv + (long)min(b0 + bb, B - 1) * V, pos, n1, n2, n3, w, lane);
+        // a's rows, for the scale only (the products read them again, from L2): the two whose rows
+        // of x the wave holds too, as x.m[..][u + (w == 0)]
+        float rg[BB][kI * kJ / 4];
+        const int rb = n3 * (int)sizeof(T), pb = n2 * rb;
+        const unsigned zo = pos.z0 + lane < n3 ? (unsigned)(pos.z0 + lane) * (unsigned)sizeof(T) : kOut;
 #pragma unroll
-      for (int bb = 0; bb < BB; ++bb) sg[bb] = some[bb] && e - ex[bb] >= -126 ? pow2(e - ex[bb]) : 0.f;
+        for (int bb = 0; bb < BB; ++bb)
 #pragma unroll
-      for (int bb = 0; bb < BB; ++bb) {
-        const float sx = pow2(ex[bb]);
-        each(rx[bb], w, lane, [&](int k, int j, int z, float v) {
-          xs[bb * kXCells + k * kXPlane + j * kXRow + z] = v * sx;
-        });
-      }
-      if (b0 == 0) {
-        unsigned any = 0;
+          for (int q = 0; q < kI * kJ / 4; ++q) {
+            const int gi = pos.i0 + (q >> 1), gj = pos.j0 + ((w + 3) & 3) + 4 * (q & 1);
+            const bool ok = gi < n1 && gj < n2 && b0 + bb < B;
+            rg[bb][q] = ld_as(rsrc(a + (long)min(b0 + bb, B - 1) * V, ok ? n1 * pb : 0), zo, ok ? gi * pb + gj * rb : 0, a);
+          }
+        // largest magnitudes: c and a of each right-hand side, the image's channels
+        unsigned mu[2 * BB + C], mn[C], all_v = 0, all_i = 0;
+#pragma unroll
+        for (int bb = 0; bb < BB; ++bb) {
+          mu[2 * bb] = max_of(rx[bb]);
+          float m = 0.f;
+#pragma unroll
+          for (int q = 0; q < kI * kJ / 4; ++q) m = max_nan(m, fabsf(rg[bb][q]));
+          mu[2 * bb + 1] = magnitude(m);
+          all_v = max(all_v, max(mu[2 * bb], mu[2 * bb + 1]));
+        }
 #pragma unroll
         for (int c = 0; c < C; ++c) {
-          const float si = pow2(ei[c]);
-          each(ri[c], w, lane, [&](int k, int j, int z, float v) {
-            const float sv = v * si;
-            const f16 hi = (f16)sv, lo = (f16)(sv - (float)hi);
-            f16* d = ih + c * kICells + k * kIPlane + j * kIRow + 1 + z;
-            d[0] = hi;
-            d[C * kICells] = lo;
-            any |= __builtin_bit_cast(unsigned short, lo);
+          mu[2 * BB + c] = 0;
+          if (b0 == 0) {
+            all_i = max(all_i, mu[2 * BB + c] = max_of(ri[c]));
+            mn[c] = min_of(ri[c]);
+          }
+        }
+        // the largest product of a centre tap (below FP32's range it counts as none)
+        float most = 0.f;
+        auto centres = [&](auto first) {
+#pragma unroll
+          for (int bb = 0; bb < BB; ++bb)
+#pragma unroll
+            for (int q = 0; q < kI * kJ / 4; ++q)
+              most = fmaxf(most, fabsf(rg[bb][q] * rx[bb].m[(q >> 1) + 1][(q & 1) + decltype(first)::value]));
+        };
+        if (w == 0) centres(std::integral_constant<int, 1>());
+        else centres(std::integral_constant<int, 0>());
+        const bool bad_v = __builtin_amdgcn_ballot_w64(all_v >= kInfinity) != 0;
+        const bool bad_i = __builtin_amdgcn_ballot_w64(all_i >= kInfinity) != 0;
+        if (bad_v || bad_i) {  // infinities set no scale
+          for (int bb = 0; bb < BB; ++bb) {
+            mu[2 * bb] = finite_max_of(rx[bb]);
+            mu[2 * bb + 1] = 0;
+            for (int q = 0; q < kI * kJ / 4; ++q) mu[2 * bb + 1] = max(mu[2 * bb + 1], finite_bits(rg[bb][q]));
+          }
+          for (int c = 0; c < C; ++c) mu[2 * BB + c] = b0 == 0 ? finite_max_of(ri[c]) : 0u;
+        }
+#pragma unroll
+        for (int k = 0; k < 2 * BB + C; ++k) mu[k] = wave_max(mu[k]);
+        __syncthreads();  // the previous tile's reads are done
+        if (lane == 0) {
+#pragma unroll
+          for (int k = 0; k < 2 * BB + C; ++k) sh[w][k] = mu[k];
+          sh[w][kFlagA] = (bad_v ? 1 : 0) | (bad_i ? 2 : 0);
+        }
+        __syncthreads();
+        auto over_waves = [&](int k) {
+          return (unsigned)__builtin_amdgcn_readfirstlane((int)max(max(sh[0][k], sh[1][k]), max(sh[2][k], sh[3][k])));
+        };
+        auto any_wave = [&](int k) {
+          return (unsigned)__builtin_amdgcn_readfirstlane((int)(sh[0][k] | sh[1][k] | sh[2][k] | sh[3][k]));
+        };
+        const unsigned bad = any_wave(kFlagA);
+        if (b0 == 0) {
+#pragma unroll
+          for (int c = 0; c < C; ++c) ei[c] = scale_exp(over_waves(2 * BB + c), kTargetP);
+        }
+        // G in units of 2^-e, the largest that a right-hand side's own factors give (they add up
+        // in G; one of zeros has no say, and one 2^100 below the other adds nothing)
+        int ex[BB], e = 2 * 126;
+        bool some[BB];
+#pragma unroll
+        for (int bb = 0; bb < BB; ++bb) {
+          const unsigned bx = over_waves(2 * bb), bg = over_waves(2 * bb + 1);
+          ex[bb] = scale_exp(bx, kTargetG);
+          some[bb] = bx != 0u && bg != 0u;
+          if (some[bb]) e = min(e, ex[bb] + scale_exp(bg, kTargetG));
+        }
+        float sg[BB];
+#pragma unroll
+        for (int bb = 0; bb < BB; ++bb) sg[bb] = some[bb] && e - ex[bb] >= -126 ? pow2(e - ex[bb]) : 0.f;
+#pragma unroll
+        for (int bb = 0; bb < BB; ++bb) {
+          const float sx = pow2(ex[bb]);
+          each(rx[bb], w, lane, [&](int k, int j, int z, float v) {
+            xs[bb * kXCells + k * kXPlane + j * kXRow + z] = v * sx;
           });
         }
-        any = __builtin_amdgcn_ballot_w64((any & 0x7fffu) != 0) != 0;
-        if (lane == 0) sh[w][2 * BB + C] = any;
-      }
-      __syncthreads();
-      if (b0 == 0) has_lo = over_waves(2 * BB + C) != 0;
-      // the products of the high parts, and those with a low part
-      f16x acc[NT], acl[NT];
+        unsigned flags = 0;  // 1: low parts, 2: small image values, 4: a product near the bound
+        flags |= __builtin_amdgcn_ballot_w64(most >= ldexpf(0.25f, -e)) != 0 ? 4u : 0u;
+        if (b0 == 0) {
+          unsigned any = 0;
+          bool small = false;
 #pragma unroll
-      for (int t = 0; t < NT; ++t) acc[t] = acl[t] = f16x{};
-
-      auto rows = [&](auto lo_c) {
-        constexpr bool LO = decltype(lo_c)::value;
-        // operands of one product step, read one step ahead of their use
-        struct Step {
-          float x[BB][8];
-          unsigned ph[NT][5];
-        };
-        struct Base {
-          int x, i[NT], l[NT];
-        };
-        auto base = [&](int q) {  // row w + 4 (q % 2) of plane q / 2
-          const int irow = ((q >> 1) * kIPlane + (q & 1) * 4 * kIRow) / 2;
-          Base r;
-          r.x = xo + (q >> 1) * kXPlane + (q & 1) * 4 * kXRow;
-#pragma unroll
-          for (int t = 0; t < NT; ++t) {
-            const int step = t == kOneTile ? on_row * irow : irow;
-            r.i[t] = io[t] + step;
-            r.l[t] = lo_o[t] + step;
+          for (int c = 0; c < C; ++c) {
+            const float si = pow2(ei[c]);
+            small |= mn[c] < least_bits(ei[c]);
+            each(ri[c], w, lane, [&](int k, int j, int z, float v) {
+              const float sv = v * si;
+              const f16 hi = (f16)sv, lo = (f16)(sv - (float)hi);
+              f16* d = ih + c * kICells + k * kIPlane + j * kIRow + 1 + z;
+              d[0] = hi;
+              d[C * kICells] = lo;
+              any |= __builtin_bit_cast(unsigned short, lo);
+            });
           }
-          return r;
-        };
-        auto load = [&](Step& st, const Base& r, int s) {
-#pragma unroll
-          for (int bb = 0; bb < BB; ++bb)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) st.x[bb][j] = ((const float*)lds)[r.x + bb * kXCells + 16 * s + j];
-#pragma unroll
-          for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int k = 0; k < 5; ++k) st.ph[t][k] = ((const unsigned*)lds)[r.i[t] + 8 * s + k];
-        };
-        float gc[BB][4], gn[BB][4];
-        load_g(gc, b0, 0);
-        Base bc = base(0);
-        Step cur;
-        load(cur, bc, 0);
+          flags |= __builtin_amdgcn_ballot_w64((any & 0x7fffu) != 0) != 0 ? 1u : 0u;
+          flags |= __builtin_amdgcn_ballot_w64(small) != 0 ? 2u : 0u;
+        }
+        if (lane == 0) sh[w][kFlagB] = flags;
+        __syncthreads();
+        flags = any_wave(kFlagB);
+        if (b0 == 0) has_lo = (flags & 1) != 0;
+        // (an image that does not do sends all of the tile's right-hand sides to the queue)
+        bool wide = bad != 0;
+        if (b0 == 0 && !wide && (flags & 2)) {
+          bool rows = false;
 #pragma unroll 1
-        for (int q = 0; q < kI * kJ / 4; ++q) {
-          const int qn = q + 1 < kI * kJ / 4 ? q + 1 : q;
-          load_g(gn, b0, qn);
-          const Base bn = base(qn);
+          for (int c = 0; c < C; ++c) {
+            Raw r;  // (read again: kept, the cells would take registers from everyone)
+            load_tile(r, img + c * V, pos, n1, n2, n3, w, lane);
+            int ec = ei[0];
 #pragma unroll
-          for (int s = 0; s < 4; ++s) {
-            Step nxt;
-            if (s < 3) load(nxt, bc, s + 1);
-            else load(nxt, bn, 0);
-            float G[8];
+            for (int k = 1; k < C; ++k) ec = c == k ? ei[k] : ec;
+            rows |= has_small_rows(r, least_bits(ec));
+          }
+          const bool any = __builtin_amdgcn_ballot_w64(rows) != 0;
+          if (lane == 0) sh[w][kFlagC] = any;
+          __syncthreads();
+          wide = any_wave(kFlagC) != 0;
+        }
+        const bool none = e == 2 * 126;  // no right-hand side has both x and g
+        if (none && !wide) continue;
+        if (wide || !(flags & 4)) {
+          if (threadIdx.x == 0) {
+            queue[queued][0] = tile;
+            queue[queued][1] = (unsigned)b0;
+          }
+          ++queued;
+          break;
+        }
+        // the products of the high parts, and those with a low part
+        f16x acc[NT], acl[NT];
 #pragma unroll
-            for (int bb = 0; bb < BB; ++bb) {
-              if (bb == 0) products<false>(gc[bb][s] * sg[bb], cur.x[bb], G);
-              else products<true>(gc[bb][s] * sg[bb], cur.x[bb], G);
-            }
-            u32x4s gh, gl;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-              unsigned hi, lo;
-              split_pair(G[2 * k], G[2 * k + 1], hi, lo);
-              gh[k] = hi;
-              gl[k] = lo;
-            }
-            auto cols = [&](const unsigned (&x)[5], int t) {
-              u32x4s r;
-#pragma unroll
-              for (int k = 0; k < 4; ++k) r[k] = __builtin_amdgcn_alignbit(x[k + 1], x[k], (unsigned)ish[t]);
-              return __builtin_bit_cast(h8, r);
-            };
-            const h8 ah = __builtin_bit_cast(h8, gh), al = __builtin_bit_cast(h8, gl);
+        for (int t = 0; t < NT; ++t) acc[t] = acl[t] = f16x{};
+
+        auto rows = [&](auto lo_c) {
+          constexpr bool LO = decltype(lo_c)::value;
+          // operands of one product step, read one step ahead of their use
+          struct Step {
+            float x[BB][8];
+            unsigned ph[NT][5];
+          };
+          struct Base {
+            int x, i[NT], l[NT];
+          };
+          auto base = [&](int q) {  // row w + 4 (q % 2) of plane q / 2
+            const int irow = ((q >> 1) * kIPlane + (q & 1) * 4 * kIRow) / 2;
+            Base r;
+            r.x = xo + (q >> 1) * kXPlane + (q & 1) * 4 * kXRow;
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-              const h8 ph = cols(cur.ph[t], t);
-              acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, ph, acc[t], 0, 0, 0);
-              acl[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, ph, acl[t], 0, 0, 0);
-              if (LO) {
-                unsigned pl[5];
-#pragma unroll
-                for (int k = 0; k < 5; ++k) pl[k] = ((const unsigned*)lds)[bc.l[t] + 8 * s + k];
-                acl[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, cols(pl, t), acl[t], 0, 0, 0);
-              }
+              const int step = t == kOneTile ? on_row * irow : irow;
+              r.i[t] = io[t] + step;
+              r.l[t] = lo_o[t] + step;
             }
-            cur = nxt;
+            return r;
+          };
+          auto load = [&](Step& st, const Base& r, int s) {
+#pragma unroll
+            for (int bb = 0; bb < BB; ++bb)
+#pragma unroll
+              for (int j = 0; j < 8; ++j) st.x[bb][j] = ((const float*)lds)[r.x + bb * kXCells + 16 * s + j];
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+              for (int k = 0; k < 5; ++k) st.ph[t][k] = ((const unsigned*)lds)[r.i[t] + 8 * s + k];
+          };
+          float gc[BB][4], gn[BB][4];
+          load_g(gc, b0, 0);
+          Base bc = base(0);
+          Step cur;
+          load(cur, bc, 0);
+#pragma unroll 1
+          for (int q = 0; q < kI * kJ / 4; ++q) {
+            const int qn = q + 1 < kI * kJ / 4 ? q + 1 : q;
+            load_g(gn, b0, qn);
+            const Base bn = base(qn);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+              Step nxt;
+              if (s < 3) load(nxt, bc, s + 1);
+              else load(nxt, bn, 0);
+              float G[8];
+#pragma unroll
+              for (int bb = 0; bb < BB; ++bb) {
+                if (bb == 0) products<false>(gc[bb][s] * sg[bb], cur.x[bb], G);
+                else products<true>(gc[bb][s] * sg[bb], cur.x[bb], G);
+              }
+              u32x4s gh, gl;
+#pragma unroll
+              for (int k = 0; k < 4; ++k) {
+                unsigned hi, lo;
+                split_pair(G[2 * k], G[2 * k + 1], hi, lo);
+                gh[k] = hi;
+                gl[k] = lo;
+              }
+              auto cols = [&](const unsigned (&x)[5], int t) {
+                u32x4s r;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) r[k] = __builtin_amdgcn_alignbit(x[k + 1], x[k], (unsigned)ish[t]);
+                return __builtin_bit_cast(h8, r);
+              };
+              const h8 ah = __builtin_bit_cast(h8, gh), al = __builtin_bit_cast(h8, gl);
+#pragma unroll
+              for (int t = 0; t < NT; ++t) {
+                const h8 ph = cols(cur.ph[t], t);
+                acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, ph, acc[t], 0, 0, 0);
+                acl[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, ph, acl[t], 0, 0, 0);
+                if (LO) {
+                  unsigned pl[5];
+#pragma unroll
+                  for (int k = 0; k < 5; ++k) pl[k] = ((const unsigned*)lds)[bc.l[t] + 8 * s + k];
+                  acl[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, cols(pl, t), acl[t], 0, 0, 0);
+                }
+              }
+              cur = nxt;
+            }
+            bc = bn;
+#pragma unroll
+            for (int bb = 0; bb < BB; ++bb)
+#pragma unroll
+              for (int s = 0; s < 4; ++s) gc[bb][s] = gn[bb][s];
           }
-          bc = bn;
+        };
+        if (has_lo) rows(std::true_type());
+        else rows(std::false_type());
 #pragma unroll
-          for (int bb = 0; bb < BB; ++bb)
+        for (int t = 0; t < NT; ++t) {
+          int u = -e;  // the column's scale: of G, and of the image's channel
 #pragma unroll
-            for (int s = 0; s < 4; ++s) gc[bb][s] = gn[bb][s];
+          for (int c = 0; c < C; ++c) u -= (32 * t + m) / 27 == c && 32 * t + m < 27 * C ? ei[c] : 0;
+#pragma unroll
+          for (int i = 0; i < 16; ++i) sum[t][i] += ldexpf(acc[t][i] + acl[t][i], u);
         }
-      };
-      if (has_lo) rows(std::true_type());
-      else rows(std::false_type());
+      }
+    }
+    if (queued == 0) break;
+    // FP32 products of the tiles that wait, from their first right-hand side that has to
+    int hv = h, mv = m;  // opaque: nothing of this is to be worked out before, or kept in registers
+    asm volatile("" : "+v"(hv), "+v"(mv));
+    int col[NT];
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        int u = -e;  // the column's scale: of G, and of the image's channel
+    for (int t = 0; t < NT; ++t) {
+      const int q = min(32 * t + mv, 27 * C - 1), s = q % 27;
+      col[t] = (q / 27) * kICells + (s / 9) * kIPlane + (s / 3 % 3) * kIRow + 1 + s % 3;
+    }
+#pragma unroll 1
+    for (int k = 0; k < queued; ++k) {
+      __syncthreads();
+      const Pos pos = tile_at((unsigned)__builtin_amdgcn_readfirstlane((int)queue[k][0]));
+#pragma unroll 1
+      for (int c = 0; c < C; ++c) {  // the image as it is, in the space of its two parts
+        Raw r;
+        load_tile(r, img + c * V, pos, n1, n2, n3, w, lane);
+        each(r, w, lane, [&](int k, int j, int z, float v) {
+          ((float*)ih)[c * kICells + k * kIPlane + j * kIRow + 1 + z] = v;
+        });
+      }
+#pragma unroll 1
+      for (int b = __builtin_amdgcn_readfirstlane((int)queue[k][1]); b < B; ++b) {
+        Raw r;
+        load_tile(r, cv + (long)b * V, pos, n1, n2, n3, w, lane);
+        __syncthreads();
+        each(r, w, lane, [&](int k, int j, int z, float v) { xs[k * kXPlane + j * kXRow + z] = v; });
+        __syncthreads();
+#pragma unroll 1
+        for (int q = 0; q < kI * kJ / 4; ++q) {
+          const int pi = q >> 1, pj = w + 4 * (q & 1), gi = pos.i0 + pi, gj = pos.j0 + pj;
+          if (gi >= n1 || gj >= n2) continue;
+          const float ga = ld_as(a_row(pos, b, pi, pj), (unsigned)(pos.z0 + lane) * (unsigned)sizeof(T), 0, a);
+          f16x row[NT];
 #pragma unroll
-        for (int c = 0; c < C; ++c) u -= (32 * t + m) / 27 == c && 32 * t + m < 27 * C ? ei[c] : 0;
+          for (int t = 0; t < NT; ++t) row[t] = f16x{};
+#pragma unroll 1
+          for (int z = 0; z < min(kZ, n3 - pos.z0); ++z) {
+            const float av = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ga), z));
+            float pv[NT];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) sum[t][i] += ldexpf(acc[t][i] + acl[t][i], u);
+            for (int t = 0; t < NT; ++t) {
+              const float v = ((const float*)ih)[col[t] + pi * kIPlane + pj * kIRow + z];
+              pv[t] = 32 * t + mv >= 27 * C ? 1.f : v;
+            }
+            asm volatile("" : "+v"(hv));
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              const int p0 = 8 * (i >> 2) + (i & 3), p1 = p0 + 4 < 27 ? p0 + 4 : 26, tap = hv ? p1 : p0;
+              const int d1 = tap / 9 - 1, d2 = tap / 3 % 3 - 1, d3 = tap % 3 - 1;
+              const bool in = (unsigned)(gi + d1) < (unsigned)n1 && (unsigned)(gj + d2) < (unsigned)n2 &&
+                              (unsigned)(pos.z0 + z + d3) < (unsigned)n3;
+              const float G = av * xs[(pi + 1 + d1) * kXPlane + (pj + 1 + d2) * kXRow + z + 1 + d3];
+#pragma unroll
+              for (int t = 0; t < NT; ++t) row[t][i] = fmaf(in ? G : 0.f, pv[t], row[t][i]);
+            }
+          }
+#pragma unroll
+          for (int t = 0; t < NT; ++t) sum[t] += row[t];
+        }
       }
     }
   }
