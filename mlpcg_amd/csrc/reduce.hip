@@ -20,13 +20,15 @@ namespace mlpcg {
 // ---------------------------------------------------------------------------
 // Mean patch.  A voxel u contributes to ybar[s,e] iff u - e is inside the grid, i.e.
 // per axis: e = -1 excludes the last cell, e = 0 none, e = +1 the first.  So the 27 sums
-// follow by inclusion and exclusion from T[a1][a2][a3], a in {all, first, last} per axis:
-// the total and the sums over the faces, edges and corners.  An interior row only adds to
-// T[0][0][.]; the rows of the faces take a branch, so the pass over the image is bound by
-// its loads (adding every run to 27 masked sums was VALU-bound).  All sums are FP64.  Each
+// add up from those over the grid's disjoint parts T[a1][a2][a3], a in {middle, first, last}
+// per axis: its inside, faces, edges and corners (taken away from a total instead, an infinite
+// cell would make NaN of the sums without it, and a large one would cost them their digits).
+// An interior row only adds to T[0][0][.]; the rows of the faces take a branch, so the pass
+// over the image is bound by its loads (adding every run to 27 masked sums was VALU-bound).
+// The only cell of an axis counts as middle.  All sums are FP64.  Each
 // sum of a workgroup leaves its wave by DPP adds: 27 C butterflies over __shfl_xor, an LDS
 // round trip per step, took 20 us on a grid of any size with C = 3.  Whole call, FP32,
-// before -> now: 256^3 C = 1 56 -> 25 us, C = 3 176 -> 56 us; 128^3 C = 3 151 -> 22 us;
+// before -> now: 256^3 C = 1 56 -> 23 us, C = 3 176 -> 48 us; 128^3 C = 3 151 -> 21 us;
 // below that the launches and their host side remain (C = 3, 16^3: 34 -> 20 us).
 // ---------------------------------------------------------------------------
 constexpr int kPatchBlocks = 512;       // workgroups of the partial sums at most (two per CU)
@@ -52,50 +54,56 @@ __device__ __forceinline__ void patch_accumulate(const TI* __restrict__ img, int
     for (int o = 0; o < 27; ++o) p.t[s][o] = 0.0;
   const long V = (long)n1 * n2 * n3;
   const unsigned n3c = (unsigned)(n3 / VZ), nch = (unsigned)n1 * (unsigned)n2 * n3c;
+  typedef typename AccOf<TI>::type A;
+  A next[C][VZ];  // loaded a run ahead
+  auto load = [&](unsigned cid) {
+#pragma unroll
+    for (int s = 0; s < C; ++s) load_vec<VZ>(img + s * V + (long)cid * VZ, next[s]);
+  };
+  if (first < nch) load(first);
   for (unsigned cid = first; cid < nch; cid += stride) {
+    A run[C][VZ];
+#pragma unroll
+    for (int s = 0; s < C; ++s)
+#pragma unroll
+      for (int u = 0; u < VZ; ++u) run[s][u] = next[s][u];
+    load(cid + stride < nch ? cid + stride : nch - 1);
     const unsigned row = cid / n3c, kc = cid - row * n3c;
     const unsigned i = row / (unsigned)n2, j = row - i * (unsigned)n2;
-    const bool zf = kc == 0, zl = kc == n3c - 1;
-    const bool edge = i == 0 || (int)i == n1 - 1 || j == 0 || (int)j == n2 - 1;
+    const bool zf = kc == 0 && n3 > 1, zl = kc == n3c - 1 && n3 > 1;
+    const int a1 = n1 == 1 ? 0 : i == 0 ? 1 : (int)i == n1 - 1 ? 2 : 0;
+    const int a2 = n2 == 1 ? 0 : j == 0 ? 1 : (int)j == n2 - 1 ? 2 : 0;
 #pragma unroll
     for (int s = 0; s < C; ++s) {
-      typedef typename AccOf<TI>::type A;
-      A v[VZ];
-      load_vec<VZ>(img + s * V + (long)cid * VZ, v);
-      double cs = (double)v[0];
+      const A(&v)[VZ] = run[s];
+      // (of one cell that is first or last, the middle keeps nothing)
+      double mid = (double)(zf || (VZ == 1 && zl) ? A(0) : v[0]);
 #pragma unroll
-      for (int u = 1; u < VZ; ++u) cs += (double)v[u];
-      const double t3[3] = {cs, zf ? (double)v[0] : 0.0, zl ? (double)v[VZ - 1] : 0.0};
-      auto add = [&](int a1, int a2) {
+      for (int u = 1; u < VZ; ++u) mid += (double)(u == VZ - 1 && zl ? A(0) : v[u]);
+      const double t3[3] = {mid, (double)(zf ? v[0] : A(0)), (double)(zl ? v[VZ - 1] : A(0))};
+      const int part = 3 * a1 + a2;
+      if (part == 0) {
 #pragma unroll
-        for (int u = 0; u < 3; ++u) p.t[s][9 * a1 + 3 * a2 + u] += t3[u];
-      };
-      add(0, 0);
-      if (edge) {
-        const bool i0 = i == 0, i1 = (int)i == n1 - 1;
-        if (i0) add(1, 0);
-        if (i1) add(2, 0);
-        if (j == 0) {
-          add(0, 1);
-          if (i0) add(1, 1);
-          if (i1) add(2, 1);
-        }
-        if ((int)j == n2 - 1) {
-          add(0, 2);
-          if (i0) add(1, 2);
-          if (i1) add(2, 2);
-        }
+        for (int u = 0; u < 3; ++u) p.t[s][u] += t3[u];
+      }
+      int face = part;  // opaque: as one if and else the two take twice the registers
+      asm volatile("" : "+v"(face));
+      if (face != 0) {
+#pragma unroll
+        for (int a = 1; a < 9; ++a)
+#pragma unroll
+          for (int u = 0; u < 3; ++u) p.t[s][3 * a + u] += face == a ? t3[u] : 0.0;
       }
     }
   }
 }
 
-// ybar = (inclusion-exclusion of the 27 C sums in T) / V, then z0 = w0 . ybar + b0 and, if
+// ybar = (sums over the parts that an offset leaves inside the grid) / V, then z0 = w0 . ybar + b0 and, if
 // w1 is given, z1 = w1 . ybar + b1: c0 and c1 of one level share their mean patch
 // (sm_model_3d.py:236-239 evaluates both on the same image), so one reduction serves both.
 // Run by threads 0 .. 127 of the workgroup that holds T in LDS; red: 4 doubles of LDS.
 template <typename A>
-__device__ __forceinline__ void patch_finish(const double* T, double* red, int NV, double invV,
+__device__ __forceinline__ void patch_finish(const double* T, double* red, int n1, int n2, int n3, int NV, double invV,
                                              const A* __restrict__ w0, const A* __restrict__ b0, A* __restrict__ z0,
                                              const A* __restrict__ w1, const A* __restrict__ b1, A* __restrict__ z1,
                                              A* __restrict__ ybar) {
@@ -104,14 +112,13 @@ __device__ __forceinline__ void patch_finish(const double* T, double* red, int N
   if (o < NV) {
     const double* t = T + (o / 27) * 27;
     const int e = o % 27;
-    // per axis: the sums over all cells, less those over the cell that the offset drops
-    const int d1 = e / 9 == 1 ? 0 : (e / 9 == 0 ? 2 : 1), d2 = (e / 3) % 3 == 1 ? 0 : ((e / 3) % 3 == 0 ? 2 : 1);
-    const int d3 = e % 3 == 1 ? 0 : (e % 3 == 0 ? 2 : 1);
+    // whether part a of an axis of n cells counts for offset d - 1
+    auto has = [](int d, int a, int n) { return d == 1 || (n > 1 && a != (d == 0 ? 2 : 1)); };
     double s = 0.0;
-    for (int m = 0; m < 8; ++m) {
-      if (((m & 1) && !d1) || ((m & 2) && !d2) || ((m & 4) && !d3)) continue;
-      const double v = t[9 * ((m & 1) ? d1 : 0) + 3 * ((m & 2) ? d2 : 0) + ((m & 4) ? d3 : 0)];
-      s += (__popc(m) & 1) ? -v : v;
+#pragma unroll
+    for (int a = 0; a < 27; ++a) {
+      const double v = t[a];
+      if (has(e / 9, a / 9, n1) && has(e / 3 % 3, a / 3 % 3, n2) && has(e % 3, a % 3, n3)) s += v;
     }
     const A yb = (A)(s * invV);
     ybar[o] = yb;
@@ -154,7 +161,7 @@ __global__ __launch_bounds__(kThreads) void mean_patch_partial_kernel(const TI* 
 constexpr int kPatchFinalThreads = 1024;
 template <typename A>
 __global__ __launch_bounds__(kPatchFinalThreads) void mean_patch_final_kernel(
-    const double* __restrict__ partials, int nblk, int NV, double invV, const A* __restrict__ w0,
+    const double* __restrict__ partials, int nblk, int n1, int n2, int n3, int NV, double invV, const A* __restrict__ w0,
     const A* __restrict__ b0, A* __restrict__ z0, const A* __restrict__ w1, const A* __restrict__ b1,
     A* __restrict__ z1, A* __restrict__ ybar) {
   __shared__ double T[27 * 3], red[4];
@@ -172,7 +179,7 @@ __global__ __launch_bounds__(kPatchFinalThreads) void mean_patch_final_kernel(
     if (lane == 63) T[o] = s;
   }
   __syncthreads();
-  patch_finish<A>(T, red, NV, invV, w0, b0, z0, w1, b1, z1, ybar);
+  patch_finish<A>(T, red, n1, n2, n3, NV, invV, w0, b0, z0, w1, b1, z1, ybar);
 }
 
 // Small grids: sums, patch and products in one workgroup (one launch instead of two).
@@ -204,7 +211,7 @@ __global__ __launch_bounds__(kPatchFinalThreads) void mean_patch_one_kernel(
     T[o] = s;
   }
   __syncthreads();
-  patch_finish<A>(T, red, 27 * C, invV, w0, b0, z0, w1, b1, z1, ybar);
+  patch_finish<A>(T, red, n1, n2, n3, 27 * C, invV, w0, b0, z0, w1, b1, z1, ybar);
 }
 
 static int mean_patch_vz(int n3) { return (n3 % 4 == 0) ? 4 : (n3 % 2 == 0 ? 2 : 1); }
@@ -233,9 +240,9 @@ static void launch_mp_t(const void* img, double* part, int nblk, bool one, doubl
           (A*)ybar);                                                                                             \
     } else {                                                                                                     \
       mean_patch_partial_kernel<TI, CC, VZZ><<<nblk, kThreads, 0, st>>>((const TI*)img, n1, n2, n3, part);       \
-      mean_patch_final_kernel<A><<<1, kPatchFinalThreads, 0, st>>>(part, nblk, 27 * C, invV, (const A*)w0,       \
-                                                                   (const A*)b0, (A*)z0, (const A*)w1,           \
-                                                                   (const A*)b1, (A*)z1, (A*)ybar);              \
+      mean_patch_final_kernel<A><<<1, kPatchFinalThreads, 0, st>>>(part, nblk, n1, n2, n3, 27 * C, invV,         \
+                                                                   (const A*)w0, (const A*)b0, (A*)z0,           \
+                                                                   (const A*)w1, (const A*)b1, (A*)z1, (A*)ybar); \
     }                                                                                                            \
     return;                                                                                                      \
   }
