@@ -53,23 +53,34 @@ __device__ __forceinline__ void patch_accumulate(const TI* __restrict__ img, int
 #pragma unroll
     for (int o = 0; o < 27; ++o) p.t[s][o] = 0.0;
   const long V = (long)n1 * n2 * n3;
-  const unsigned n3c = (unsigned)(n3 / VZ), nch = (unsigned)n1 * (unsigned)n2 * n3c;
+  const unsigned n3c = (unsigned)(n3 / VZ);
+  const long nch = (long)n1 * n2 * n3c;
   typedef typename AccOf<TI>::type A;
   A next[C][VZ];  // loaded a run ahead
-  auto load = [&](unsigned cid) {
+  auto load = [&](long cid) {
 #pragma unroll
-    for (int s = 0; s < C; ++s) load_vec<VZ>(img + s * V + (long)cid * VZ, next[s]);
+    for (int s = 0; s < C; ++s) load_vec<VZ>(img + s * V + cid * VZ, next[s]);
   };
   if (first < nch) load(first);
-  for (unsigned cid = first; cid < nch; cid += stride) {
+  for (long cid = first; cid < nch; cid += stride) {
     A run[C][VZ];
 #pragma unroll
     for (int s = 0; s < C; ++s)
 #pragma unroll
       for (int u = 0; u < VZ; ++u) run[s][u] = next[s][u];
     load(cid + stride < nch ? cid + stride : nch - 1);
-    const unsigned row = cid / n3c, kc = cid - row * n3c;
-    const unsigned i = row / (unsigned)n2, j = row - i * (unsigned)n2;
+    unsigned i, j, kc;
+    if (nch <= 0xffffffffL) {  // uniform; 64-bit divisions take a hundred instructions more
+      const unsigned row = (unsigned)cid / n3c;
+      kc = (unsigned)cid - row * n3c;
+      i = row / (unsigned)n2;
+      j = row - i * (unsigned)n2;
+    } else {
+      const long row = cid / n3c;
+      kc = (unsigned)(cid - row * n3c);
+      i = (unsigned)(row / n2);
+      j = (unsigned)(row - (long)i * n2);
+    }
     const bool zf = kc == 0 && n3 > 1, zl = kc == n3c - 1 && n3 > 1;
     const int a1 = n1 == 1 ? 0 : i == 0 ? 1 : (int)i == n1 - 1 ? 2 : 0;
     const int a2 = n2 == 1 ? 0 : j == 0 ? 1 : (int)j == n2 - 1 ? 2 : 0;
