@@ -14,7 +14,8 @@
 //     add to the neighbouring z tiles go to a side array, an entry per row and tile.
 // The lower lanes hold the columns of d1 = -1 and two of d1 = 0, the upper lanes those of
 // d1 = +1 and the third of d1 = 0 (its row j + 1, while the lower lanes finish row j - 1 from
-// theirs: the upper lanes' sums wait two steps).  All sums are FP32 in a fixed order.
+// theirs: the upper lanes' sums wait two steps).  All sums are FP32 in a fixed order.  Tiles
+// and blocks that ask for exact stencils get them as in split.hpp.
 #pragma once
 
 #include <algorithm>
@@ -69,10 +70,10 @@ template <typename TI, int C, int R, int BB>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ig_waves(C, BB), 8)))
 void igrad_kernel(IgradArgs a) {
   constexpr int PJ = R + 4, FI = kIgPlanes, kCells = tile_cells(FI, PJ);
-  // a BF16 image is exact in one FP16 value
   constexpr bool FULL = sizeof(TI) == 4;
-  __shared__ __attribute__((aligned(16))) f16 ih[C * kCells], il[FULL ? C * kCells : 8];
-  __shared__ unsigned sh[8];
+  __shared__ __attribute__((aligned(16))) char im[C * kCells * (FULL ? 4 : 2)];
+  __shared__ unsigned sh[4 * (C + 2)];
+  const f16 *ih = (const f16*)im, *il = ih + C * kCells;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h = lane >> 5, n = lane & 31;
   const unsigned tz = (unsigned)((a.n3 + kZ - 1) / kZ), tj = (unsigned)((a.n2 + R - 1) / R);
@@ -86,13 +87,13 @@ void igrad_kernel(IgradArgs a) {
   for (int c = 0; c < C; ++c)
     load_raw<FI, PJ>(ri[c], (const TI*)a.img + c * V, Tile{i0, j0 - 1, z0}, a.n1, a.n2, a.n3, w, lane);
   const PackHeader* hd = (const PackHeader*)a.pack;
-  const ImageTile it = stage_image<C, FI, PJ, FULL>(ri, hd->img_limit, w, lane, ih, il, sh);
+  const ImageTile<C> it =
+      stage_image<TI, C, FI, PJ>(ri, hd, 0, 0, w, lane, im, sh, (const TI*)a.img, Tile{i0, j0 - 1, z0}, a.n1, a.n2, a.n3);
   const int i = i0 + w;
   if (i >= a.n1) return;  // uniform; no barrier follows
   Weights<C> W;
   W.load(a.pack, lane);
-  W.set_bias(((const float*)((const char*)a.pack + kHeaderBytes + pack_w_bytes(C)))[lane & 31] * pow2(it.exp), h);
-  const float inv_i = pow2(-it.exp), inv_w = hd->inv_scale;
+  W.set_bias(ldexpf(((const float*)((const char*)a.pack + kHeaderBytes + pack_w_bytes(C)))[lane & 31], it.E - kOne), h);
   WordBase wb;
   wb.init<PJ>(h, n, w * PJ);
 
@@ -113,32 +114,36 @@ void igrad_kernel(IgradArgs a) {
       gn[bb][1] = ld_as(r, o1, ok ? j * rb : 0, gp);
     }
   };
-  RowSum m[BB][3], q[BB][2];
-  float d1[BB][2], d2[BB][2];
-#pragma unroll
-  for (int bb = 0; bb < BB; ++bb) {
-#pragma unroll
-    for (int k = 0; k < 3; ++k) m[bb][k] = RowSum{0.f, 0.f, 0.f, 0.f};
-    q[bb][0] = q[bb][1] = RowSum{0.f, 0.f, 0.f, 0.f};
-    d1[bb][0] = d1[bb][1] = d2[bb][0] = d2[bb][1] = 0.f;
-  }
   const int rows = min(R, a.n2 - j0);  // output rows
-  load_g(j0 - 1);
-  // where the lane's pair, its cell of T[0] and its edge sums of row j - 1 go; one row on per step
   const long e8 = (long)tz * 8;
-  float *pm[BB], *pq[BB];
-  float* pe[BB];
-#pragma unroll
-  for (int bb = 0; bb < BB; ++bb) {
-    float* T = a.T + (long)(b0 + bb) * 3 * V + i * plane + (long)(j0 - 2) * a.n3 + z0 + 2 * n;
-    pm[bb] = T + (h ? 2 * V : 0);
-    pq[bb] = T + V + h;
-    // [row][z tile][main, mid of the lower / upper lanes][right, left]
-    pe[bb] = a.edge + (((long)(b0 + bb) * a.n1 + i) * a.n2 + j0 - 2) * e8 + zt * 8 + 2 * h + (n == 0 ? 1 : 0);
-  }
 
-  auto march = [&](auto lo_c) {
-    constexpr bool LO = decltype(lo_c)::value;
+  // Returns whether a sum is infinite or NaN.  (K scaled by 2^E overflows where g is some 2^90 or
+  // more: the wave then marches again with exact stencils.)
+  auto march = [&](auto mode) -> bool {
+    constexpr int M = decltype(mode)::value;  // 0: hi alone, 1: hi and lo, 2: exact stencils
+    const int back = M == 2 ? 0 : -it.E;
+    float most = 0.f;
+    RowSum m[BB][3], q[BB][2];
+    float d1[BB][2], d2[BB][2];
+#pragma unroll
+    for (int bb = 0; bb < BB; ++bb) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) m[bb][k] = RowSum{0.f, 0.f, 0.f, 0.f};
+      q[bb][0] = q[bb][1] = RowSum{0.f, 0.f, 0.f, 0.f};
+      d1[bb][0] = d1[bb][1] = d2[bb][0] = d2[bb][1] = 0.f;
+    }
+    load_g(j0 - 1);
+    // where the lane's pair, its cell of T[0] and its edge sums of row j - 1 go; one row on per step
+    float *pm[BB], *pq[BB];
+    float* pe[BB];
+#pragma unroll
+    for (int bb = 0; bb < BB; ++bb) {
+      float* T = a.T + (long)(b0 + bb) * 3 * V + i * plane + (long)(j0 - 2) * a.n3 + z0 + 2 * n;
+      pm[bb] = T + (h ? 2 * V : 0);
+      pq[bb] = T + V + h;
+      // [row][z tile][main, mid of the lower / upper lanes][right, left]
+      pe[bb] = a.edge + (((long)(b0 + bb) * a.n1 + i) * a.n2 + j0 - 2) * e8 + zt * 8 + 2 * h + (n == 0 ? 1 : 0);
+    }
 #pragma unroll 1
     for (int s = 0; s < rows + 2; ++s) {
       const int j = j0 - 1 + s;
@@ -151,7 +156,16 @@ void igrad_kernel(IgradArgs a) {
       load_g(j + 1);
       if ((unsigned)j < (unsigned)a.n2) {  // uniform
         f16x K[2];
-        stencils<C, LO>(W, ih, il, kCells, wb, s * kPitch, K);
+        if constexpr (M == 2)
+          exact_stencils<C, PJ>(a.pack, kCells, (w * PJ + s) * kPitch + 2 * n, h, K, [&](int c, int e) {
+            if (it.exact) return (float)((const TI*)im)[e];  // uniform
+            int fc = it.f[0];
+#pragma unroll
+            for (int k = 1; k < C; ++k) fc = c == k ? it.f[k] : fc;
+            return ldexpf((float)ih[e] + (FULL ? (float)il[e] : 0.f), -fc);
+          });
+        else
+          stencils<C, M == 1, C != 3 || M == 1>(W, ih, il, kCells, wb, s * kPitch, K);
         if (ragged) {  // uniform: cells past the grid add nothing, whatever K is there
 #pragma unroll
           for (int k = 0; k < 15; ++k) {
@@ -174,10 +188,15 @@ void igrad_kernel(IgradArgs a) {
 #pragma unroll
       for (int bb = 0; bb < BB; ++bb) {
         if (BB > 1 && b0 + bb >= a.B) break;
-        const float fx = inv_i, fw = inv_w;
         RowSum r = m[bb][0], p = q[bb][0];
-        r = RowSum{r.e * fx * fw, r.o * fx * fw, r.ex * fx * fw, r.ox * fx * fw};
-        p = RowSum{p.e * fx * fw, p.o * fx * fw, p.ex * fx * fw, p.ox * fx * fw};
+        r = RowSum{ldexpf(r.e, back), ldexpf(r.o, back), ldexpf(r.ex, back), ldexpf(r.ox, back)};
+        p = RowSum{ldexpf(p.e, back), ldexpf(p.o, back), ldexpf(p.ex, back), ldexpf(p.ox, back)};
+        if (M != 2) {
+          most = max_nan(most, max_nan(fabsf(r.e), fabsf(r.o)));
+          most = max_nan(most, max_nan(fabsf(r.ex), fabsf(r.ox)));
+          most = max_nan(most, max_nan(fabsf(p.e), fabsf(p.o)));
+          most = max_nan(most, max_nan(fabsf(p.ex), fabsf(p.ox)));
+        }
         // (all lanes take part in the shifts; the first or last of a half drops what it received)
         const float rx = wave_from_prev(r.ex), ry = wave_from_next(r.ox);
         const float px = wave_from_prev(p.ex), py = wave_from_next(p.ox);
@@ -207,11 +226,11 @@ void igrad_kernel(IgradArgs a) {
         d1[bb][1] = qo;
       }
     }
+    return __builtin_amdgcn_ballot_w64(magnitude(most) >= kInfinity) != 0;
   };
-  if constexpr (FULL) {
-    if (it.has_lo) return march(std::true_type());
-  }
-  march(std::false_type());
+  bool exact = it.exact;
+  if (!exact) exact = FULL && it.has_lo ? march(std::integral_constant<int, FULL ? 1 : 0>()) : march(std::integral_constant<int, 0>());
+  if (exact) march(std::integral_constant<int, 2>());
 }
 
 // dx(i, j, k) = T[-1](i + 1) + T[0](i) + T[+1](i - 1), plus the z tiles' edge sums
@@ -302,10 +321,10 @@ size_t fused_sgrad_bytes(int n1, int n2, int n3) {
 }
 
 // Time of launch_igrad and the packing, stored K and its transposed gather -> now: FP32 C = 1
-// 256^3 835 -> 215 us, 128^3 98 -> 41 us, two right-hand sides 119 -> 56 us, 64^3 25 -> 19 us;
-// C = 3 256^3 1730 -> 520 us; BF16 256^3 C = 1 280 (nine BF16 column sums) -> 181 us, C = 3 409 -> 390 us.  Errors
-// against 64 bits (norm-wise): FP32 0.9 to 1.4e-7 (was 1.1 to 1.5e-7), BF16 1.7e-3, the
-// result's rounding (was 2.1 to 2.5e-3).
+// 256^3 835 -> 216 us, 128^3 98 -> 39 us, two right-hand sides 119 -> 55 us, 64^3 25 -> 18 us;
+// C = 3 256^3 1730 -> 468 us; BF16 256^3 C = 1 280 (nine BF16 column sums) -> 180 us, C = 3 409 ->
+// 360 us.  Errors against 64 bits (norm-wise): FP32 0.9 to 1.3e-7 (was 1.0 to 1.9e-7), BF16
+// 1.7e-3, the result's rounding (was 2.1 to 2.5e-3).
 int launch_igrad(int dtype, const void* img, const void* pack, const void* g, void* dx, void* work, size_t bytes, int C,
                  int B, int n1, int n2, int n3, hipStream_t st) {
   MLPCG_REQUIRE(split_eligible(C, n1, n2, n3), "igrad: grid (%d,%d,%d) / C=%d not supported", n1, n2, n3, C);

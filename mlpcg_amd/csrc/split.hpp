@@ -6,18 +6,24 @@
 // 116 bytes per voxel of the stored-stencil apply): it is recomputed from the image tile in
 // LDS.  W and the image are scaled by powers of two and split as v = hi + lo into two FP16
 // values each, which keeps 22 bits and more, and
-//   W . img = W_hi img_hi + W_lo img_hi + W_hi img_lo          (FP16 products, FP32 sums)
-// on v_mfma_f32_32x32x16_f16.  The dropped W_lo img_lo is below 2^-22 of its term, the matrix
-// cores round once where an FP32 chain rounds 28 times; measured against 64 bits the block's
-// error is below that of the FP32 chain (see launch_sm_split).  K meets x in FP32 FMAs.
+//   W . img = W_lo img_hi + W_hi img_lo + W_hi img_hi          (FP16 products, FP32 sums)
+// on v_mfma_f32_32x32x16_f16, the small products first.  The dropped W_lo img_lo is below 2^-22
+// of its term, the matrix cores round a few times where an FP32 chain rounds 28 times; measured
+// against 64 bits the block's error is below that of the FP32 chain (see launch_sm_split).  K
+// meets x in FP32 FMAs.
 //
-// Scaling.  A workgroup takes the largest finite |img| of its tile and scales it into
-// [2^4, 2^5) (exact: a power of two), W likewise over the whole weight when it is packed, so
-// images and weights of any magnitude keep their bits: what falls below FP16's denormal
-// 2^-24 is below 2^-28 of the largest value.  The bias, scaled by both factors, joins as
-// three FP16 parts (33 bits) on spare K slots whose image value is 1 (as an accumulator it
-// took 16 registers and a wave per SIMD); where it is large against W img it limits the
-// image's factor (the bits lost are far below the bias's own).  y is scaled back once.
+// Scaling.  A channel of W is scaled to a largest value in [2^14, 2^15) when it is packed, a
+// channel of a workgroup's image tile likewise, less what makes all products share one unit
+// 2^-E: the channel whose W times image is largest decides, and the bias, which joins scaled by
+// 2^E as three FP16 parts (33 bits) on spare K slots whose image value is 2^15 (as an
+// accumulator it took 16 registers and a wave per SIMD).  y is scaled back once.  FP16's smallest
+// step 2^-24 is then 2^-39 of the largest value: what is within 2^-16 of that keeps its bits.
+//
+// Exact stencils.  Where more is asked for, K comes from FP32 FMAs over the image as it is (some
+// ten times slower): blocks with infinite or NaN weights or whose weights along a line of three
+// taps are all, but not all 0, below 2^-16 of their channel's largest; tiles with an infinite or
+// NaN image value, with three image cells in a row like that (of what the tile's scaling
+// leaves), or with |x| from 2^80 on, which the unscaled K alone can take without overflow.
 //
 // Tile and lanes.  A workgroup of 4 waves covers FI planes x 8 rows x 64 z; the tile with a
 // one-cell halo is staged in LDS (x in FP32, the image as two FP16 arrays), zero outside the
@@ -46,8 +52,9 @@ namespace split {
 
 constexpr int kZ = 64, kJ = 8, kPJ = kJ + 2;
 constexpr int kPitch = 68;      // cells per staged row (66 used; even, for 8-byte x reads)
-constexpr int kTarget = 4;      // largest |W| and |img| are scaled into [2^4, 2^5)
-constexpr int kBiasTarget = 8;  // and the largest scaled bias stays below 2^9
+constexpr int kTarget = 14;  // largest |W| and |img| of a channel are scaled into [2^14, 2^15)
+constexpr int kOne = 15;     // exponent of the image value of the bias's slots
+constexpr float kHuge = 1.2089258e24f;  // 2^80
 
 
 // column i (0..4) of lane half h; the fifth of the upper half is a dummy (zero weights).  The
@@ -56,16 +63,18 @@ __host__ __device__ constexpr int col_of(int h, int i) { return h == 0 ? i : (i 
 __host__ __device__ constexpr bool col_real(int h, int i) { return h == 0 || i < 4; }
 
 struct PackHeader {
-  float inv_scale;  // 1 / (the weights' factor)
-  int img_limit;    // largest exponent of the image's factor (from the bias)
+  int w_exp[3];     // exponents of the channels' factors (kNone: no weight but 0)
+  int bias_limit;   // largest E that the bias leaves
   int finite;       // no weight or bias is infinite or NaN
-  int pad;
+  int exact;        // two FP16 values do not hold the weights
 };
-// header, then W [parity][hi, lo][k half][channel][lane][8] (FP16), then the scaled bias of
-// the 32 rows of D (FP32)
+constexpr int kNone = 1000;
+// header, then W [parity][hi, lo][k half][channel][lane][8] (FP16), the bias of the 32 rows of D,
+// and W as it is, in the order of a lane's results: [27 C taps, bias][lane half][16] (FP32)
 constexpr size_t kHeaderBytes = 64;
 constexpr size_t pack_w_bytes(int C) { return (size_t)2 * 2 * 2 * C * 64 * 8 * sizeof(f16); }
-constexpr size_t pack_bytes(int C) { return kHeaderBytes + pack_w_bytes(C) + 32 * sizeof(float); }
+constexpr size_t pack_exact_at(int C) { return kHeaderBytes + pack_w_bytes(C) + 32 * sizeof(float); }
+constexpr size_t pack_bytes(int C) { return pack_exact_at(C) + (size_t)(27 * C + 1) * 32 * sizeof(float); }
 
 // Tap (of 27) of K slot j of lane half h in k half kc for z parity par; -1: spare.
 __host__ __device__ constexpr int slot_tap(int par, int h, int kc, int j) {
@@ -86,63 +95,84 @@ __host__ __device__ constexpr int reg_tap(int h, int i) {
 // One workgroup per 512 packed values; every workgroup scans the weights for their scale.
 __global__ __launch_bounds__(kThreads) void split_pack_kernel(const float* __restrict__ W, const float* __restrict__ b,
                                                               int C, char* __restrict__ out) {
-  __shared__ unsigned sh[3][4];
-  unsigned mw = 0, mb = 0, bad = 0;
+  __shared__ unsigned sh[5][4];
+  unsigned mw[3] = {0, 0, 0}, mb = 0, bad = 0, line[3];
+  int lc[3];
 #pragma unroll
-  for (int k = 0; k < 9; ++k) {  // C <= 3; clamped, so that all loads are in flight together
-    const float v = W[min(k * kThreads + (int)threadIdx.x, 27 * 27 * C - 1)];
-    const unsigned u = finite_bits(v);
-    mw = mw > u ? mw : u;
-    bad |= (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u;
+  for (int k = 0; k < 3; ++k) {  // lines of three taps (C <= 3; clamped, so that all loads are in flight together)
+    const int t = min(k * kThreads + (int)threadIdx.x, 243 * C - 1);
+    lc[k] = t / 9 % C;
+    float m = 0.f;
+#pragma unroll
+    for (int u = 0; u < 3; ++u) m = max_nan(m, fabsf(W[3 * t + u]));
+    bad |= magnitude(m) >= kInfinity;
+    line[k] = magnitude(m);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) mw[c] = c == lc[k] ? max(mw[c], finite_bits(m)) : mw[c];
   }
   if (threadIdx.x < 27) {
     mb = finite_bits(b[threadIdx.x]);
-    bad |= (__float_as_uint(b[threadIdx.x]) & 0x7f800000u) == 0x7f800000u;
+    bad |= magnitude(b[threadIdx.x]) >= kInfinity;
   }
-  mw = wave_max(mw);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) mw[c] = wave_max(mw[c]);
   mb = wave_max(mb);
   bad = wave_max(bad);
   if ((threadIdx.x & 63) == 0) {
-    sh[0][threadIdx.x >> 6] = mw;
-    sh[1][threadIdx.x >> 6] = mb;
-    sh[2][threadIdx.x >> 6] = bad;
+    for (int c = 0; c < 3; ++c) sh[c][threadIdx.x >> 6] = mw[c];
+    sh[3][threadIdx.x >> 6] = mb;
+    sh[4][threadIdx.x >> 6] = bad;
   }
   __syncthreads();
-  for (int k = 0; k < 4; ++k) {
-    mw = mw > sh[0][k] ? mw : sh[0][k];
-    mb = mb > sh[1][k] ? mb : sh[1][k];
-    bad |= sh[2][k];
+  int ew[3];
+  for (int c = 0; c < 3; ++c) {
+    const unsigned m = max(max(sh[c][0], sh[c][1]), max(sh[c][2], sh[c][3]));
+    ew[c] = m == 0u ? kNone : min(kTarget - exponent_of(m), 126);
   }
-  const int ew = min(kTarget - exponent_of(mw), 100);
-  const float s = pow2(ew);
+  mb = max(max(sh[3][0], sh[3][1]), max(sh[3][2], sh[3][3]));
+  bad = sh[4][0] | sh[4][1] | sh[4][2] | sh[4][3];
   const int nw = (int)(pack_w_bytes(C) / sizeof(f16));
   f16* __restrict__ wp = (f16*)(out + kHeaderBytes);
   float* __restrict__ bp = (float*)(out + kHeaderBytes + pack_w_bytes(C));
-  #pragma unroll
+#pragma unroll
   for (int k = 0; k < 2; ++k) {
     const int e = blockIdx.x * 512 + k * kThreads + threadIdx.x;  // nw is a multiple of 512
     const int j = e % 8, lane = (e / 8) % 64, c = (e / 512) % C, kc = (e / (512 * C)) % 2;
     const int part = (e / (1024 * C)) % 2, par = e / (2048 * C);
     const int m = lane & 31;  // row of D: register i of lane half h
     const int p = reg_tap((m >> 2) & 1, 4 * (m >> 3) + (m & 3)), q = slot_tap(par, lane >> 5, kc, j);
+    const int es = c == 0 ? ew[0] : c == 1 ? ew[1] : ew[2];
     float v = 0.f;
-    if (p >= 0 && q >= 0) {
-      const float w = W[((long)p * C + c) * 27 + q] * s;
+    if (p >= 0 && q >= 0 && es != kNone) {
+      const float w = W[((long)p * C + c) * 27 + q] * pow2(es);
       const f16 hi = (f16)w;
       v = part == 0 ? (float)hi : w - (float)hi;
     }
     wp[e] = (f16)v;
   }
-  if (blockIdx.x == 0 && threadIdx.x < 32) {
-    const int m = threadIdx.x, p = reg_tap((m >> 2) & 1, 4 * (m >> 3) + (m & 3));
-    bp[threadIdx.x] = p >= 0 ? b[p] * s : 0.f;
+  float* __restrict__ xp = (float*)(out + pack_exact_at(C));
+  for (int e = blockIdx.x * kThreads + threadIdx.x; e < (27 * C + 1) * 32; e += gridDim.x * kThreads) {
+    const int p = reg_tap((e >> 4) & 1, e & 15), q = e >> 5;
+    xp[e] = p < 0 ? 0.f : q == 27 * C ? b[p] : W[((long)p * C + q / 27) * 27 + q % 27];
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
+  if (blockIdx.x != 0) return;
+  unsigned small = 0;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const int es = lc[k] == 0 ? ew[0] : lc[k] == 1 ? ew[1] : ew[2];
+    if (es != kNone) small |= (line[k] << 1) - 1u < least_bits(es);
+  }
+  small = __syncthreads_or((int)small);
+  if (threadIdx.x < 32) {
+    const int m = threadIdx.x, p = reg_tap((m >> 2) & 1, 4 * (m >> 3) + (m & 3));
+    bp[threadIdx.x] = p >= 0 ? b[p] : 0.f;
+  }
+  if (threadIdx.x == 0) {
     PackHeader h;
-    h.inv_scale = pow2(-ew);
-    h.img_limit = mb == 0u ? 126 : kBiasTarget - (exponent_of(mb) + ew);
+    for (int c = 0; c < 3; ++c) h.w_exp[c] = ew[c];
+    h.bias_limit = mb == 0u ? kNone : kOne + kTarget - exponent_of(mb);
     h.finite = bad ? 0 : 1;
-    h.pad = 0;
+    h.exact = bad || small ? 1 : 0;
     *(PackHeader*)out = h;
   }
 }
@@ -177,29 +207,44 @@ __device__ __forceinline__ Tile tile_at(int n2, int n3) {
   return Tile{(int)(u / tj) * FI, (int)(u % tj) * kJ, (int)((t + u) % tz) * kZ};
 }
 
-// Raw cells of a staged tile as FP32: rows w, w + 4, ... of the wave, cell z0 + lane of each,
-// and one z-halo cell of the whole tile per thread (rows' cells z0 - 1 and z0 + 64).
+// Raw cells of a staged tile as FP32.  A wave holds rows w, w + 4, ... of every plane, cell
+// z0 + lane of each; where PJ is no multiple of 4, its rows start at (w + 2) % 4 in odd planes, so
+// that each wave has the last two rows' share in every other plane.  And one z-halo cell of the
+// whole tile per thread (rows' cells z0 - 1 and z0 + 64).
 template <int FI, int PJ = kPJ>
 struct Raw {
-  static constexpr int kRows = (tile_rows(FI, PJ) + 3) / 4;
+  static constexpr int kPlanes = FI + 2, kGroups = PJ / 4, kExtra = PJ % 4 ? kPlanes / 2 : 0;
+  static_assert(PJ % 4 == 0 || (PJ % 4 == 2 && kPlanes % 2 == 0), "rows of a tile over four waves");
   static_assert(2 * tile_rows(FI, PJ) <= kThreads, "one halo cell per thread");
-  float m[kRows];
+  float m[kPlanes][kGroups];
+  float x[kExtra ? kExtra : 1];  // row 4 kGroups + w % 2 of plane 2 s + w / 2
   float halo;
+  // the wave's first row in planes of parity k
+  static __device__ __forceinline__ int row0(int k, int w) { return kExtra ? (w + 2 * (k & 1)) & 3 : w; }
 };
 
+// (One resource per plane, whose offsets fit 32 bits, and row offsets shared by the planes of a
+// parity: a resource per row took most of the scalar registers and half of the kernel's
+// instructions.)
 template <int FI, int PJ, typename T>
 __device__ __forceinline__ void load_raw(Raw<FI, PJ>& r, const T* __restrict__ src, const Tile& t, int n1, int n2,
                                          int n3, int w, int lane) {
+  typedef Raw<FI, PJ> R;
+  constexpr unsigned kOut = 0x80000000u;
   const long plane = (long)n2 * n3;
   const int pb = (int)(plane * (int)sizeof(T)), rb = n3 * (int)sizeof(T);
-  const unsigned zo = t.z0 + lane < n3 ? (unsigned)(t.z0 + lane) * (unsigned)sizeof(T) : 0x80000000u;
+  const unsigned zo = t.z0 + lane < n3 ? (unsigned)(t.z0 + lane) * (unsigned)sizeof(T) : kOut;
+  auto load = [&](int k, int row) {
+    const int gi = t.i0 + k - 1, gj = t.j0 + row - 1;
+    const bool oi = (unsigned)gi < (unsigned)n1, oj = (unsigned)gj < (unsigned)n2;
+    return ld_as(rsrc(src + (oi ? gi : 0) * plane, oi ? pb : 0), oj ? zo : kOut, oi && oj ? gj * rb : 0, src);
+  };
 #pragma unroll
-  for (int k = 0; k < Raw<FI, PJ>::kRows; ++k) {
-    const int row = w + 4 * k;
-    const int gi = t.i0 + row / PJ - 1, gj = t.j0 + row % PJ - 1;
-    const bool ok = row < tile_rows(FI, PJ) && (unsigned)gi < (unsigned)n1 && (unsigned)gj < (unsigned)n2;
-    r.m[k] = ld_as(rsrc(src + (ok ? gi : 0) * plane, ok ? pb : 0), zo, (ok ? gj : 0) * rb, src);
-  }
+  for (int k = 0; k < R::kPlanes; ++k)
+#pragma unroll
+    for (int u = 0; u < R::kGroups; ++u) r.m[k][u] = load(k, R::row0(k, w) + 4 * u);
+#pragma unroll
+  for (int s = 0; s < R::kExtra; ++s) r.x[s] = load(2 * s + (w >> 1), 4 * R::kGroups + (w & 1));
   const int hrow = threadIdx.x >> 1, z = (threadIdx.x & 1) ? t.z0 + kZ : t.z0 - 1;
   const int gi = t.i0 + hrow / PJ - 1, gj = t.j0 + hrow % PJ - 1;
   const bool ok = hrow < tile_rows(FI, PJ) && (unsigned)gi < (unsigned)n1 && (unsigned)gj < (unsigned)n2 &&
@@ -209,67 +254,165 @@ __device__ __forceinline__ void load_raw(Raw<FI, PJ>& r, const T* __restrict__ s
 
 template <int FI, int PJ, typename F>
 __device__ __forceinline__ void each_cell(const Raw<FI, PJ>& r, int w, int lane, F&& f) {
+  typedef Raw<FI, PJ> R;
 #pragma unroll
-  for (int k = 0; k < Raw<FI, PJ>::kRows; ++k)
-    if (w + 4 * k < tile_rows(FI, PJ)) f((w + 4 * k) * kPitch + 1 + lane, r.m[k]);
+  for (int k = 0; k < R::kPlanes; ++k)
+#pragma unroll
+    for (int u = 0; u < R::kGroups; ++u) f(R::row0(k, w) * kPitch + 1 + lane + (k * PJ + 4 * u) * kPitch, r.m[k][u]);
+#pragma unroll
+  for (int s = 0; s < R::kExtra; ++s)
+    f(((w >> 1) * PJ + (w & 1)) * kPitch + 1 + lane + (2 * s * PJ + 4 * R::kGroups) * kPitch, r.x[s]);
   if ((int)(threadIdx.x >> 1) < tile_rows(FI, PJ)) f((threadIdx.x >> 1) * kPitch + (threadIdx.x & 1) * (kZ + 1), r.halo);
 }
 
-// The image tile of C channels as two FP16 arrays hi, lo [C][cells].  Returns (uniform) the
-// exponent of the tile's factor; flags: any non-finite cell, any nonzero lo (LO = false: the
-// image is of a type that hi holds, lo is left out).  Ends in a barrier; sh: 8 words of LDS.
-struct ImageTile {
-  int exp;
-  bool nonfinite, has_lo;
-};
-template <int C, int FI, int PJ = kPJ, bool LO = true>
-__device__ __forceinline__ ImageTile stage_image(const Raw<FI, PJ> (&raw)[C], int limit, int w, int lane, f16* hi, f16* lo,
-                                                 unsigned* sh) {
-  unsigned m = 0, bad = 0;
+// Whether three cells in a row of a tile, halo included, hold values below `least` only
+// (small_bits), not all 0.  src: as for load_raw.
+template <int FI, int PJ, typename T>
+__device__ __forceinline__ bool has_small_rows(const Raw<FI, PJ>& r, const T* __restrict__ src, const Tile& t, int n1,
+                                               int n2, int n3, unsigned least) {
+  typedef Raw<FI, PJ> R;
+  bool bad = false;
+  auto row = [&](float cell) {
+    const float v = fabsf(cell);
+    bad |= small_bits(fmaxf(v, fmaxf(wave_from_prev(v), wave_from_next(v)))) < least;
+  };
 #pragma unroll
-  for (int c = 0; c < C; ++c)
+  for (int k = 0; k < R::kPlanes; ++k)
+#pragma unroll
+    for (int u = 0; u < R::kGroups; ++u) row(r.m[k][u]);
+#pragma unroll
+  for (int s = 0; s < R::kExtra; ++s) row(r.x[s]);
+  if (r.halo != 0.f) {  // (then its row is in the grid) with the two cells next to it
+    const int hrow = threadIdx.x >> 1, z = (threadIdx.x & 1) ? t.z0 + kZ - 1 : t.z0;
+    const T* p = src + ((long)(t.i0 + hrow / PJ - 1) * n2 + t.j0 + hrow % PJ - 1) * n3;
+    float v = fmaxf(fabsf(r.halo), fabsf((float)p[z]));
+    const int z2 = (threadIdx.x & 1) ? z - 1 : z + 1;
+    if (z2 < n3) v = fmaxf(v, fabsf((float)p[z2]));
+    bad |= small_bits(v) < least;
+  }
+  return bad;
+}
+
+// The image tile of C channels as two FP16 arrays hi, lo [C][cells], the channels scaled by 2^f,
+// or, for exact stencils, as it is, [C][cells] in the same space (T: its type; a BF16 image has
+// no lo, it is exact in one FP16 value down to 2^-17).  Ends in a barrier; sh: 4 (C + 2) words of
+// LDS; flags: of the wave (uniform), or-ed over the workgroup's; img, t: where raw is from.
+template <int C>
+struct ImageTile {
+  int E, f[C];     // K is scaled by 2^E
+  unsigned flags;  // as passed
+  bool nonfinite, exact, has_lo;
+};
+template <typename T, int C, int FI, int PJ>
+__device__ __forceinline__ ImageTile<C> stage_image(const Raw<FI, PJ> (&raw)[C], const PackHeader* hd, unsigned flags,
+                                                    unsigned exact_flags, int w, int lane, char* im, unsigned* sh,
+                                                    const T* __restrict__ img, const Tile& t, int n1, int n2, int n3) {
+  constexpr bool LO = sizeof(T) == 4;
+  constexpr int kCells = tile_cells(FI, PJ), kS = C + 2;
+  f16 *hi = (f16*)im, *lo = hi + C * kCells;
+  unsigned mx[C], mn[C], most = 0;
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    float m = 0.f;
+    mn[c] = ~0u;
     each_cell<FI, PJ>(raw[c], w, lane, [&](int, float v) {
-      const unsigned u = __float_as_uint(v) & 0x7fffffffu;
-      const bool fin = u < 0x7f800000u;
-      m = max(m, fin ? u : 0u);
-      bad |= fin ? 0u : 1u;
+      m = max_nan(m, fabsf(v));
+      mn[c] = min(mn[c], small_bits(v));
     });
-  m = wave_max(m);
-  bad = __builtin_amdgcn_ballot_w64(bad != 0) != 0;
+    mx[c] = magnitude(m);
+    most = max(most, mx[c]);
+  }
+  const bool bad = __builtin_amdgcn_ballot_w64(most >= kInfinity) != 0;
+  if (bad) {
+    for (int c = 0; c < C; ++c) {
+      mx[c] = 0;
+      each_cell<FI, PJ>(raw[c], w, lane, [&](int, float v) { mx[c] = max(mx[c], finite_bits(v)); });
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < C; ++c) mx[c] = wave_max(mx[c]);
   if (lane == 0) {
-    sh[w] = m;
-    sh[4 + w] = bad;
+#pragma unroll
+    for (int c = 0; c < C; ++c) sh[kS * w + c] = mx[c];
+    sh[kS * w + C] = (bad ? 1u : 0u) | flags << 1;
   }
   __syncthreads();
-  m = max(max(sh[0], sh[1]), max(sh[2], sh[3]));
-  bad = sh[4] | sh[5] | sh[6] | sh[7];
-  ImageTile it;
-  it.exp = __builtin_amdgcn_readfirstlane(max(-126, min(min(kTarget - exponent_of(m), limit), 126)));
-  it.nonfinite = __builtin_amdgcn_readfirstlane((int)bad) != 0;
-  const float s = pow2(it.exp);
-  unsigned any = 0;
+  const unsigned all = (unsigned)__builtin_amdgcn_readfirstlane(
+      (int)(sh[C] | sh[kS + C] | sh[2 * kS + C] | sh[3 * kS + C]));
+  ImageTile<C> it;
+  it.nonfinite = (all & 1) != 0;
+  it.flags = all >> 1;
+  it.E = hd->bias_limit;
+  int own[C];
 #pragma unroll
-  for (int c = 0; c < C; ++c)
-    each_cell<FI, PJ>(raw[c], w, lane, [&](int e, float v) {
-      const float sv = v * s;
-      const f16 h = (f16)sv;
-      hi[c * tile_cells(FI, PJ) + e] = h;
-      if (LO) {
-        const f16 l = (f16)(sv - (float)h);
-        lo[c * tile_cells(FI, PJ) + e] = l;
-        any |= __builtin_bit_cast(unsigned short, l) & 0x7fffu;
-      }
-    });
-  if (!LO) {
-    it.has_lo = false;
+  for (int c = 0; c < C; ++c) {
+    const unsigned m = max(max(sh[c], sh[kS + c]), max(sh[2 * kS + c], sh[3 * kS + c]));
+    own[c] = min(kTarget - exponent_of(m), 126);
+    if (m != 0u && hd->w_exp[c] != kNone) it.E = min(it.E, hd->w_exp[c] + own[c]);
+  }
+  it.E = __builtin_amdgcn_readfirstlane(it.E == kNone ? 0 : it.E);
+  bool small = false;
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    // (below -126 only where the rows are small, or there is no weight)
+    it.f[c] = __builtin_amdgcn_readfirstlane(max(hd->w_exp[c] == kNone ? own[c] : min(it.E - hd->w_exp[c], 126), -126));
+    small |= mn[c] < least_bits(it.f[c] + (LO ? 0 : 15));
+  }
+  it.exact = __builtin_amdgcn_readfirstlane(hd->exact) != 0 || it.nonfinite || (it.flags & exact_flags) != 0;
+  it.has_lo = false;
+  auto store_raw = [&](const Raw<FI, PJ>& r, int c) {
+    each_cell<FI, PJ>(r, w, lane, [&](int e, float v) { ((T*)im)[c * kCells + e] = (T)v; });
+  };
+  if (it.exact) {
+#pragma unroll
+    for (int c = 0; c < C; ++c) store_raw(raw[c], c);
     __syncthreads();
     return it;
   }
-  any = __builtin_amdgcn_ballot_w64(any != 0) != 0;
-  __syncthreads();  // the flags above were read by everyone
-  if (lane == 0) sh[w] = any;
+  unsigned any = 0;
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    const float s = pow2(it.f[c]);
+    each_cell<FI, PJ>(raw[c], w, lane, [&](int e, float v) {
+      const float sv = v * s;
+      const f16 h = (f16)sv;
+      hi[c * kCells + e] = h;
+      if (LO) {
+        const f16 l = (f16)(sv - (float)h);
+        lo[c * kCells + e] = l;
+        any |= __builtin_bit_cast(unsigned short, l) & 0x7fffu;
+      }
+    });
+  }
+  const bool has = LO && __builtin_amdgcn_ballot_w64(any != 0) != 0, few = __builtin_amdgcn_ballot_w64(small) != 0;
+  if (lane == 0) sh[kS * w + C + 1] = (has ? 1u : 0u) | (few ? 2u : 0u);
   __syncthreads();
-  it.has_lo = __builtin_amdgcn_readfirstlane((int)(sh[0] | sh[1] | sh[2] | sh[3])) != 0;
+  const unsigned got = (unsigned)__builtin_amdgcn_readfirstlane(
+      (int)(sh[C + 1] | sh[kS + C + 1] | sh[2 * kS + C + 1] | sh[3 * kS + C + 1]));
+  it.has_lo = (got & 1) != 0;
+  if (got & 2) {  // rare: are small values alone in their rows?
+    const long V = (long)n1 * n2 * n3;
+    bool rows = false;
+#pragma unroll 1
+    for (int c = 0; c < C; ++c) {
+      Raw<FI, PJ> r;  // (read again: kept, the cells would take registers from everyone)
+      load_raw<FI, PJ>(r, img + c * V, t, n1, n2, n3, w, lane);
+      int fc = it.f[0];
+#pragma unroll
+      for (int k = 1; k < C; ++k) fc = c == k ? it.f[k] : fc;
+      rows |= has_small_rows<FI, PJ>(r, img + c * V, t, n1, n2, n3, least_bits(fc + (LO ? 0 : 15)));
+    }
+    it.exact = __syncthreads_or((int)rows) != 0;
+    if (it.exact) {
+#pragma unroll 1
+      for (int c = 0; c < C; ++c) {
+        Raw<FI, PJ> r;
+        load_raw<FI, PJ>(r, img + c * V, t, n1, n2, n3, w, lane);
+        store_raw(r, c);
+      }
+      __syncthreads();
+    }
+  }
   return it;
 }
 
@@ -289,7 +432,7 @@ struct Weights {
           for (int c = 0; c < C; ++c)
             w[par][part][kc][c] = *(const h8*)(p + ((((par * 2 + part) * 2 + kc) * C + c) * 64 + lane) * 8);
   }
-  // the bias of the lane's row of D, scaled: hi and lo on the spare slot of the lower lane
+  // the bias of the lane's row of D, scaled by 2^(E - kOne): hi and lo on the spare slot of the lower lane
   // half, the rest on that of the upper one
   __device__ __forceinline__ void set_bias(float b, int h) {
     const f16 hi = (f16)b, lo = (f16)(b - (float)hi), rest = (f16)(b - (float)hi - (float)lo);
@@ -318,10 +461,10 @@ struct WordBase {
   }
 };
 // The lane's words of one FP16 array at a chunk as the B operands of the two k halves, per z
-// parity; the spare half word (a cell outside the patch) becomes 1 for the bias, or 0.
+// parity; the spare half word (a cell outside the patch) becomes 2^kOne for the bias, or 0.
 template <bool ONE>
 __device__ __forceinline__ void operands(const f16* arr, const WordBase& wb, int cell, h8 (&b)[2][2]) {
-  constexpr unsigned one_hi = ONE ? 0x3c000000u : 0u, one_lo = ONE ? 0x3c00u : 0u;
+  constexpr unsigned one_hi = ONE ? 0x78000000u : 0u, one_lo = ONE ? 0x7800u : 0u;  // 2^kOne
   const char* p = (const char*)arr + 2 * cell;
   auto word = [&](unsigned off) { return *(const unsigned*)(p + off); };
   const u32x4s e = {word(wb.b0[0]), word(wb.b0[1]), word(wb.b0[2]), word(wb.b0[3])};
@@ -332,26 +475,73 @@ __device__ __forceinline__ void operands(const f16* arr, const WordBase& wb, int
   b[1][0] = __builtin_bit_cast(h8, o);
   b[1][1] = __builtin_bit_cast(h8, u32x4s{o4, both_hi(e[0], e[1]), both_hi(e[2], e[3]), (e4 & 0xffff0000u) | one_lo});
 }
-// scaled K of the lane's columns for both parities, from the tile at `cell`
-template <int C, bool LO>
+// scaled K of the lane's columns for both parities, from the tile at `cell`; the products with a
+// low part before the others, whose sums they would otherwise be rounded into (FIRST: of all
+// channels, whose image words then wait in 16 registers each; else channel by channel)
+template <int C, bool LO, bool FIRST = true>
 __device__ __forceinline__ void stencils(const Weights<C>& W, const f16* hi, const f16* lo, int cells,
                                          const WordBase& wb, int cell, f16x (&K)[2]) {
+  h8 bh[C][2][2];
+  auto high = [&](int c) {
+#pragma unroll
+    for (int kc = 0; kc < 2; ++kc)
+#pragma unroll
+      for (int par = 0; par < 2; ++par)
+        K[par] = __builtin_amdgcn_mfma_f32_32x32x16_f16(W.w[par][0][kc][c], bh[c][par][kc], K[par], 0, 0, 0);
+  };
 #pragma unroll
   for (int c = 0; c < C; ++c) {
-    h8 bh[2][2], bl[2][2];
-    if (c == 0) operands<true>(hi, wb, cell, bh);
-    else operands<false>(hi + c * cells, wb, cell, bh);
+    h8 bl[2][2];
+    if (c == 0) operands<true>(hi, wb, cell, bh[c]);
+    else operands<false>(hi + c * cells, wb, cell, bh[c]);
     if (LO) operands<false>(lo + c * cells, wb, cell, bl);
 #pragma unroll
-    for (int par = 0; par < 2; ++par) {
+    for (int kc = 0; kc < 2; ++kc) {
 #pragma unroll
-      for (int kc = 0; kc < 2; ++kc) {
+      for (int par = 0; par < 2; ++par) {
         const f16x in = c == 0 && kc == 0 ? f16x{} : K[par];
-        K[par] = __builtin_amdgcn_mfma_f32_32x32x16_f16(W.w[par][1][kc][c], bh[par][kc], in, 0, 0, 0);
+        K[par] = __builtin_amdgcn_mfma_f32_32x32x16_f16(W.w[par][1][kc][c], bh[c][par][kc], in, 0, 0, 0);
         if (LO) K[par] = __builtin_amdgcn_mfma_f32_32x32x16_f16(W.w[par][0][kc][c], bl[par][kc], K[par], 0, 0, 0);
-        K[par] = __builtin_amdgcn_mfma_f32_32x32x16_f16(W.w[par][0][kc][c], bh[par][kc], K[par], 0, 0, 0);
       }
     }
+    if (!FIRST) high(c);
+  }
+  if (FIRST) {
+#pragma unroll
+    for (int c = 0; c < C; ++c) high(c);
+  }
+}
+
+// The same, not scaled, by FP32 FMAs over the image `at` of a tile cell; cell: that of tap 0 of
+// the lane's even voxel.
+template <int C, int PJ, typename At>
+__device__ __forceinline__ void exact_stencils(const void* pack, int cells, int cell, int h, f16x (&K)[2], At&& at) {
+  const float* w = (const float*)((const char*)pack + pack_exact_at(C)) + 16 * h;
+#pragma unroll
+  for (int i = 0; i < 15; ++i) K[0][i] = K[1][i] = w[27 * C * 32 + i];
+  K[0][15] = K[1][15] = 0.f;
+#pragma unroll 1
+  for (int c = 0; c < C; ++c) {
+#pragma unroll 1
+    for (int k = 0; k < 9; ++k) {
+      const int e = c * cells + cell + (k / 3 * PJ + k % 3) * kPitch;
+      const float f[4] = {at(c, e), at(c, e + 1), at(c, e + 2), at(c, e + 3)};
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+#pragma unroll
+        for (int i = 0; i < 15; ++i) {
+          K[0][i] = fmaf(w[i], f[d], K[0][i]);
+          K[1][i] = fmaf(w[i], f[d + 1], K[1][i]);
+        }
+        w += 32;
+      }
+    }
+  }
+  // (the upper lanes' fifth column is a dummy, and 0 times an infinity would stay)
+#pragma unroll
+  for (int i = 12; i < 15; ++i) {
+    K[0][i] = h ? 0.f : K[0][i];
+    K[1][i] = h ? 0.f : K[1][i];
   }
 }
 
@@ -369,8 +559,9 @@ void sm_split_kernel(SplitArgs a) {
   constexpr int kCells = tile_cells(FI);
   constexpr bool FULL = sizeof(T) == 4;
   __shared__ __attribute__((aligned(16))) float xs[BB][kCells];
-  __shared__ __attribute__((aligned(16))) f16 ih[C * kCells], il[FULL ? C * kCells : 8];
-  __shared__ unsigned sh[12];
+  __shared__ __attribute__((aligned(16))) char im[C * kCells * (FULL ? 4 : 2)];
+  __shared__ unsigned sh[4 * (C + 2)];
+  const f16 *ih = (const f16*)im, *il = ih + C * kCells;
   if (solve_done(a.done)) return;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int h = lane >> 5, n = lane & 31;
@@ -388,25 +579,25 @@ void sm_split_kernel(SplitArgs a) {
   const float scale = a.in_scale ? (float)(*a.in_scale) : 1.f;
   const float c0 = a.prev ? *a.c0 : 0.f, c1 = a.prev ? *a.c1 : 0.f;
 
-  unsigned xany = 0;
+  float xm = 0.f;
 #pragma unroll
   for (int bb = 0; bb < BB; ++bb) {
     if (BB > 1 && b0 + bb >= a.B) break;
     each_cell<FI, kPJ>(rx[bb], w, lane, [&](int e, float v) {
       xs[bb][e] = v;
-      xany |= __float_as_uint(v) & 0x7fffffffu;
+      xm = max_nan(xm, fabsf(v));
     });
   }
-  xany = __builtin_amdgcn_ballot_w64(xany != 0) != 0;
-  if (lane == 0) sh[8 + w] = xany;
-  const ImageTile it = stage_image<C, FI, kPJ, FULL>(ri, hd->img_limit, w, lane, ih, il, sh);
+  constexpr unsigned kSome = 1, kLarge = 2;  // x is not 0 everywhere; too large for a scaled K
+  const unsigned xf = (__builtin_amdgcn_ballot_w64(xm != 0.f) ? kSome : 0u) | (__builtin_amdgcn_ballot_w64(!(xm < kHuge)) ? kLarge : 0u);
+  const ImageTile<C> it =
+      stage_image<T, C, FI, kPJ>(ri, hd, xf, kLarge, w, lane, im, sh, (const T*)a.img, t, a.n1, a.n2, a.n3);
   Weights<C> W;
   W.load(a.pack, lane);
-  W.set_bias(((const float*)((const char*)a.pack + kHeaderBytes + pack_w_bytes(C)))[lane & 31] * pow2(it.exp), h);
+  W.set_bias(ldexpf(((const float*)((const char*)a.pack + kHeaderBytes + pack_w_bytes(C)))[lane & 31], it.E - kOne), h);
   // x = 0 everywhere: every finite K gives y = 0
-  const bool zero = !__builtin_amdgcn_readfirstlane((int)(sh[8] | sh[9] | sh[10] | sh[11])) && !it.nonfinite &&
-                    __builtin_amdgcn_readfirstlane(hd->finite);
-  const float inv_i = pow2(-it.exp), inv_w = hd->inv_scale * scale;
+  const bool zero = !(it.flags & kSome) && !it.nonfinite && __builtin_amdgcn_readfirstlane(hd->finite);
+  const int back = it.exact ? 0 : -it.E;
 
   WordBase wb;
   wb.init(h, n, w);
@@ -429,8 +620,8 @@ void sm_split_kernel(SplitArgs a) {
   const long plane = (long)a.n2 * a.n3, v00 = ((long)t.i0 * a.n2 + t.j0 + w) * a.n3 + t.z0, j4 = 4L * a.n3;
   T* __restrict__ y = (T*)a.y + b0 * V;
 
-  auto chunks = [&](auto lo_c) {
-    constexpr bool LO = decltype(lo_c)::value;
+  auto chunks = [&](auto mode) {
+    constexpr int M = decltype(mode)::value;  // 0: hi alone, 1: hi and lo, 2: exact stencils
 #pragma unroll
     for (int q = 0; q < FI * 2; ++q) {
       const int ii = q >> 1, jj = w + 4 * (q & 1);
@@ -455,7 +646,10 @@ void sm_split_kernel(SplitArgs a) {
       const bool skip = zero || (LB && has_b && __builtin_amdgcn_ballot_w64(zok && kb != 0) == 0);
       if (!skip) {
         f16x K[2];
-        stencils<C, LO>(W, ih, il, kCells, wb, cell, K);
+        if constexpr (M == 2)
+          exact_stencils<C, kPJ>(a.pack, kCells, cell + w * kPitch + 2 * n, h, K, [&](int, int e) { return (float)((const T*)im)[e]; });
+        else
+          stencils<C, M == 1>(W, ih, il, kCells, wb, cell, K);
 #pragma unroll
         for (int bb = 0; bb < BB; ++bb) {
           float pe = 0.f, po = 0.f;
@@ -474,7 +668,7 @@ void sm_split_kernel(SplitArgs a) {
               po = fmaf(K[1][3 * i + k], f[k + 1], po);
             }
           }
-          val[bb] = halves_sum(pe, po) * inv_i * inv_w;
+          val[bb] = ldexpf(halves_sum(pe, po), back) * scale;
         }
       }
 #pragma unroll
@@ -494,12 +688,9 @@ void sm_split_kernel(SplitArgs a) {
       }
     }
   };
-  if constexpr (FULL) {
-    if (it.has_lo && !zero) chunks(std::true_type());
-    else chunks(std::false_type());
-  } else {
-    chunks(std::false_type());
-  }
+  if (it.exact) chunks(std::integral_constant<int, 2>());
+  else if (FULL && it.has_lo && !zero) chunks(std::integral_constant<int, FULL ? 1 : 0>());
+  else chunks(std::integral_constant<int, 0>());
   if (LD0 && has_0) block_partials<2>(red, a.partials);
   if constexpr (PL) {
     // the means of the stored output in avgpool2_kernel's order (z pair, then rows 2J, 2J + 1
@@ -579,11 +770,11 @@ int launch_split_pack(const void* W, const void* b, int C, void* pack, hipStream
 }
 
 // Error against 64 bits (norm-wise, the modules' weights, random and flag images): C = 1
-// 1.06e-7 and 0.97e-7 where the FP32 chain of the stored stencils has 1.17e-7 and 1.07e-7;
-// C = 3 1.56e-7 and 1.11e-7 against 1.89e-7 and 1.38e-7.
+// 1.08e-7 and 0.95e-7 where the FP32 chain of the stored stencils has 1.18e-7 and 1.10e-7;
+// C = 3 1.25e-7 and 0.99e-7 against 1.77e-7 and 1.38e-7.
 // Time of a block forward (packing included), stored stencils -> now: 256^3 C = 1 843 ->
-// 111 us, C = 3 1483 -> 258 us; 128^3 C = 1 90 -> 25 us, two right-hand sides 97 -> 34 us,
-// C = 3 185 -> 46 us; 97 x 75 x 131 C = 3, two right-hand sides 103 -> 44 us; at 32^3 both
+// 100 us, C = 3 1483 -> 244 us; 128^3 C = 1 90 -> 22 us, two right-hand sides 97 -> 30 us,
+// C = 3 185 -> 39 us; 97 x 75 x 131 C = 3, two right-hand sides 103 -> 38 us; at 32^3 both
 // take the 19 us of two launches.
 int launch_sm_split(int C, const SplitArgs& a, hipStream_t st) {
   MLPCG_REQUIRE(split_eligible(C, a.n1, a.n2, a.n3), "sm_split: grid (%d,%d,%d) / C=%d not supported", a.n1, a.n2,

@@ -142,11 +142,13 @@ __device__ __forceinline__ unsigned finite_max_of(const Raw& r) {
 __device__ __forceinline__ int scale_exp(unsigned bits, int target) {
   return max(-126, min(target - exponent_of(bits), 126));
 }
-// Whether three cells in a row of a tile hold values below `least` only (small_bits), not all 0
-// (the z-halo cells, which other lanes hold, by themselves).  If not, sums over a patch are as
-// good as if the smaller values were held like `least`.
-__device__ __forceinline__ bool has_small_rows(const Raw& r, unsigned least) {
-  bool bad = small_bits(r.halo) < least;
+// Whether three cells in a row of a tile, halo included, hold values below `least` only
+// (small_bits), not all 0.  If not, sums over a patch are as good as if the smaller values were
+// held like `least`.  src: as for load_tile.
+template <typename T>
+__device__ __forceinline__ bool has_small_rows(const Raw& r, const T* __restrict__ src, const Pos& t, int n1, int n2,
+                                               int n3, unsigned least) {
+  bool bad = false;
 #pragma unroll
   for (int k = 0; k < kI + 2; ++k)
 #pragma unroll
@@ -154,6 +156,14 @@ __device__ __forceinline__ bool has_small_rows(const Raw& r, unsigned least) {
       const float v = fabsf(r.m[k][u]);
       bad |= small_bits(fmaxf(v, fmaxf(wave_from_prev(v), wave_from_next(v)))) < least;
     }
+  if (r.halo != 0.f) {  // (then its row is in the grid) with the two cells next to it
+    const int hrow = threadIdx.x >> 1, z = (threadIdx.x & 1) ? t.z0 + kZ - 1 : t.z0;
+    const T* p = src + ((long)(t.i0 + hrow / kPJ - 1) * n2 + t.j0 + hrow % kPJ - 1) * n3;
+    float v = fmaxf(fabsf(r.halo), fabsf((float)p[z]));
+    const int z2 = (threadIdx.x & 1) ? z - 1 : z + 1;
+    if (z2 < n3) v = fmaxf(v, fabsf((float)p[z2]));
+    bad |= small_bits(v) < least;
+  }
   return bad;
 }
 // lane I of a row of 16 to the whole row
@@ -400,7 +410,7 @@ void wgrad_kernel(const T* __restrict__ a, const T* __restrict__ cv, int B, cons
             int ec = ei[0];
 #pragma unroll
             for (int k = 1; k < C; ++k) ec = c == k ? ei[k] : ec;
-            rows |= has_small_rows(r, least_bits(ec));
+            rows |= has_small_rows(r, img + c * V, pos, n1, n2, n3, least_bits(ec));
           }
           const bool any = __builtin_amdgcn_ballot_w64(rows) != 0;
           if (lane == 0) sh[w][kFlagC] = any;
