@@ -477,14 +477,17 @@ __device__ __forceinline__ void operands(const f16* arr, const WordBase& wb, int
 }
 // scaled K of the lane's columns for both parities, from the tile at `cell`; the products with a
 // low part before the others, whose sums they would otherwise be rounded into (FIRST: of all
-// channels, whose image words then wait in 16 registers each; else channel by channel)
+// channels, whose image words then wait in 16 registers each; else channel by channel), then the
+// half with the bias.  Norm-wise error over 24 blocks of random weights, C = 1 and 3, images of
+// flags: half by half 9.9e-8 and 1.05e-7, so 9.4e-8 and 9.4e-8; a plan at 256^3 2.20e-7, bias last
+// 2.27e-7, bias first 2.08e-7.
 template <int C, bool LO, bool FIRST = true>
 __device__ __forceinline__ void stencils(const Weights<C>& W, const f16* hi, const f16* lo, int cells,
                                          const WordBase& wb, int cell, f16x (&K)[2]) {
   h8 bh[C][2][2];
   auto high = [&](int c) {
 #pragma unroll
-    for (int kc = 0; kc < 2; ++kc)
+    for (int kc = 1; kc >= 0; --kc)
 #pragma unroll
       for (int par = 0; par < 2; ++par)
         K[par] = __builtin_amdgcn_mfma_f32_32x32x16_f16(W.w[par][0][kc][c], bh[c][par][kc], K[par], 0, 0, 0);
