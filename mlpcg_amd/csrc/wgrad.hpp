@@ -15,12 +15,14 @@
 // own largest finite magnitudes, and a tile's products are added, scaled back, to FP32 sums
 // kept beside its accumulators: no tile's factor reaches another's, whether that is empty or
 // its values are far larger.  FP16's smallest step is then 2^-39 of the largest |a| |c| and of
-// the largest |image| of a tile.  Where that is not enough (no product of the tile's centre taps
-// within 2^-16 of that bound, or three image cells in a row that are all 2^-16 and more below
-// it), and in tiles with infinities or NaN, FP32 products are summed on the VALU, over the cells
-// and taps inside the grid alone (some 20 times slower, for a kind of tile that is rare).  Such
-// tiles wait until the workgroup's others are done: among them, that code's registers and
-// instructions cost every tile 5 %.
+// the largest |image| of a tile.  Where no product of the tile's centre taps comes within 2^-16 of
+// the former, all products are looked at and the largest sets the scale of G.  (What is 2^-39
+// below a tile's largest G is lost: where x falls off into the air by such factors, the image is
+// 0, and the sums' errors stay below the FP32 products'.)  Tiles with three
+// image cells in a row that are all 2^-16 and more below the latter, with infinities or with NaN
+// are summed in FP32 on the VALU, over the cells and taps inside the grid alone (some 10 times
+// slower, for a kind of tile that is rare).  They wait until the workgroup's others are done:
+// among them, that code's registers and instructions cost every tile 5 %.
 //
 // Tile: 4 planes x 8 rows x 64 z; x and the image with a one-cell halo in LDS, any extents.
 // A wave takes rows of 64 voxels, 16 voxels per product: lane (h, m) = (lane / 32, lane % 32)
@@ -208,8 +210,9 @@ void wgrad_kernel(const T* __restrict__ a, const T* __restrict__ cv, int B, cons
   constexpr int kXB = BB * kXCells * 4, kIB = C * kICells * 2, kRed = 4 * 32 * 32 * 4;
   constexpr int kOnesAt = kXB + 2 * kIB, kUsed = kOnesAt + 2 * kOnes * 4;
   __shared__ __attribute__((aligned(16))) char lds[kUsed > kRed ? kUsed : kRed];
-  __shared__ unsigned sh[4][2 * BB + C + 3], queue[kQueue][2];
-  constexpr int kFlagA = 2 * BB + C, kFlagB = kFlagA + 1, kFlagC = kFlagA + 2;
+  __shared__ unsigned sh[4][2 * BB + C + 5], queue[kQueue][2];
+  constexpr int kFlagA = 2 * BB + C, kFlagB = kFlagA + 1, kFlagC = kFlagA + 2, kFlagD = kFlagA + 3,
+                kFlagE = kFlagA + 4;
   float* xs = (float*)lds;      // [BB][kXCells]
   f16* ih = (f16*)(lds + kXB);  // [C][kICells], then the low parts
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -419,7 +422,46 @@ void wgrad_kernel(const T* __restrict__ a, const T* __restrict__ cv, int B, cons
         }
         const bool none = e == 2 * 126;  // no right-hand side has both x and g
         if (none && !wide) continue;
-        if (wide || !(flags & 4)) {
+        if (!wide && !(flags & 4)) {
+          // no centre tap comes near the bound (x may be large beside a solid, where g lies in it):
+          // G's own largest value sets its scale
+          float top = 0.f;
+          unsigned pairs = 0;
+#pragma unroll 1
+          for (int q = 0; q < kI * kJ / 4; ++q) {
+            const int pi = q >> 1, pj = w + 4 * (q & 1);
+#pragma unroll
+            for (int bb = 0; bb < BB; ++bb) {
+              const float g = ld_as(a_row(pos, b0 + bb, pi, pj), (unsigned)(pos.z0 + lane) * (unsigned)sizeof(T), 0, a);
+#pragma unroll 1
+              for (int d = 0; d < 9; ++d) {
+                const float* x = xs + bb * kXCells + (pi + d / 3) * kXPlane + (pj + d % 3) * kXRow + lane;
+                const float m = fmaxf(fabsf(x[0]), fmaxf(fabsf(x[1]), fabsf(x[2])));
+                top = fmaxf(top, fabsf(g * sg[bb]) * m);
+                pairs |= g != 0.f && m != 0.f;
+              }
+            }
+          }
+          const unsigned m = wave_max(__float_as_uint(top));
+          const bool some_g = __builtin_amdgcn_ballot_w64(pairs != 0) != 0;
+          if (lane == 0) {
+            sh[w][kFlagD] = m;
+            sh[w][kFlagE] = some_g;
+          }
+          __syncthreads();
+          const unsigned most_g = over_waves(kFlagD);
+          if (any_wave(kFlagE) == 0) continue;
+          const int up = 2 * kTargetG + 1 - exponent_of(most_g);
+          wide = most_g == 0u;
+#pragma unroll
+          for (int bb = 0; bb < BB; ++bb) {
+            if (!some[bb]) continue;
+            wide |= e + up - ex[bb] > 126;
+            sg[bb] = e + up - ex[bb] >= -126 ? pow2(min(e + up - ex[bb], 126)) : 0.f;
+          }
+          e += up;
+        }
+        if (wide) {
           if (threadIdx.x == 0) {
             queue[queued][0] = tile;
             queue[queued][1] = (unsigned)b0;
@@ -537,7 +579,12 @@ void wgrad_kernel(const T* __restrict__ a, const T* __restrict__ cv, int B, cons
     // FP32 products of the tiles that wait, from their first right-hand side that has to
     int hv = h, mv = m;  // opaque: nothing of this is to be worked out before, or kept in registers
     asm volatile("" : "+v"(hv), "+v"(mv));
-    int col[NT];
+    int col[NT], off[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int p0 = 8 * (i >> 2) + (i & 3), p1 = p0 + 4 < 27 ? p0 + 4 : 26, tap = hv ? p1 : p0;
+      off[i] = (tap / 9) * kXPlane + (tap / 3 % 3) * kXRow + tap % 3;
+    }
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const int q = min(32 * t + mv, 27 * C - 1), s = q % 27;
@@ -573,20 +620,29 @@ void wgrad_kernel(const T* __restrict__ a, const T* __restrict__ cv, int B, cons
 #pragma unroll 1
           for (int z = 0; z < min(kZ, n3 - pos.z0); ++z) {
             const float av = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ga), z));
+            const int at = pi * kXPlane + pj * kXRow + z;
             float pv[NT];
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
               const float v = ((const float*)ih)[col[t] + pi * kIPlane + pj * kIRow + z];
               pv[t] = 32 * t + mv >= 27 * C ? 1.f : v;
             }
-            asm volatile("" : "+v"(hv));
+            if (magnitude(av) < kInfinity) {  // (beyond the grid x is 0)
+#pragma unroll
+              for (int i = 0; i < 16; ++i) {
+                const float G = av * xs[off[i] + at];
+#pragma unroll
+                for (int t = 0; t < NT; ++t) row[t][i] = fmaf(G, pv[t], row[t][i]);
+              }
+              continue;
+            }
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
+              asm volatile("" : "+v"(hv));
               const int p0 = 8 * (i >> 2) + (i & 3), p1 = p0 + 4 < 27 ? p0 + 4 : 26, tap = hv ? p1 : p0;
-              const int d1 = tap / 9 - 1, d2 = tap / 3 % 3 - 1, d3 = tap % 3 - 1;
-              const bool in = (unsigned)(gi + d1) < (unsigned)n1 && (unsigned)(gj + d2) < (unsigned)n2 &&
-                              (unsigned)(pos.z0 + z + d3) < (unsigned)n3;
-              const float G = av * xs[(pi + 1 + d1) * kXPlane + (pj + 1 + d2) * kXRow + z + 1 + d3];
+              const bool in = (unsigned)(gi + tap / 9 - 1) < (unsigned)n1 && (unsigned)(gj + tap / 3 % 3 - 1) < (unsigned)n2 &&
+                              (unsigned)(pos.z0 + z + tap % 3 - 1) < (unsigned)n3;
+              const float G = av * xs[off[i] + at];
 #pragma unroll
               for (int t = 0; t < NT; ++t) row[t][i] = fmaf(in ? G : 0.f, pv[t], row[t][i]);
             }

@@ -96,3 +96,19 @@ def test_unlike_magnitudes_within_a_tile(dev, kind, C, B, shape, dtype):
     for c in range(C + 1):
         q = slice(27 * c, 27 * (c + 1)) if c < C else slice(27 * C, 27 * C + 1)
         assert float(err[:, q].norm() / D[:, q].norm()) <= 32 * 2.0 ** -24, c
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("C,B,d", [(1, 1, 0), (3, 2, 1), (2, 3, 2)])
+def test_tiles_that_see_x_in_their_halo_alone(dev, C, B, d, dtype):
+    """No centre tap of a 4 x 8 x 64 tile has a product, its neighbours' cells do."""
+    shape = (10, 17, 134)
+    print(f"weight gradient x in the halo {dtype} C={C} B={B} axis {d}", flush=True)
+    gen = torch.Generator().manual_seed(10)
+    img, x, g = torch.rand(C, *shape, generator=gen), torch.zeros(B, 1, *shape), torch.randn(B, 1, *shape, generator=gen)
+    edge = (4, 8, 64)[d]
+    x.narrow(2 + d, edge, 1).copy_(torch.randn(B, 1, *shape, generator=gen).narrow(2 + d, edge, 1))
+    img, x, g = (t.to(dtype) for t in (img, x, g))
+    got, (D, A) = _got(dev, img, x, g), _exact(img, x, g)
+    assert torch.all((got - D).abs() <= _bound(A))
+    assert float((got - D).norm() / D.norm()) <= 32 * 2.0 ** -24
