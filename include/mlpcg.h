@@ -59,8 +59,8 @@ int mlpcg_version(void);
  * y[b,v] = sum_p K_p(v) x[b, v+d_p],  K_p(v) = bias[p] + sum_{s,e} weight[p,s,e] image[s, v+e].
  * workspace: mlpcg_sm_block_workspace_size() bytes (stencil weights + gradient partials; for
  * BF16 also an FP16 image copy and packed weights).  BF16 blocks on grids of >= 2^18 voxels
- * with n1, n2 % 8 == 0, n3 % 64 == 0 (B = 1) run on the matrix cores: image values must lie
- * in the FP16 normal range there. */
+ * with n1, n2 % 8 == 0, n3 % 64 == 0 (B = 1) have their forward take the image in FP16: its
+ * values must lie in the FP16 normal range there. */
 size_t mlpcg_sm_block_workspace_size(int C, int B, int n1, int n2, int n3, int dtype);
 /* sm_block_3d.cpp:31  smblock3d.inference(image, x, weights, bias) -> [y] */
 int mlpcg_sm_block_inference(const void* image, const void* x, const void* weight, const void* bias,
@@ -83,8 +83,9 @@ int mlpcg_sm_block_backward(const void* grad_out, const void* image, const void*
  * the image (C x V, equal to the BF16 image converted), and wpack, the weights and bias
  * packed by mlpcg_fused_pack (mlpcg_fused_pack_bytes(C) bytes; they must be the packing
  * of weight and bias).  NULL = made in the workspace per call, as by the plain entry
- * points; results are bit-identical.  Grids the matrix-core path does not take ignore
- * both. */
+ * points; results are bit-identical.  The forward of grids that path does not take ignores
+ * both, and so does the backward: it reads the BF16 image itself and packs the weights in
+ * two parts, 4 us a call. */
 int mlpcg_sm_block_forward_ex(const void* image, const void* image16, const void* wpack, const void* x,
                               const void* weight, const void* bias, void* y, void* workspace, int C, int B, int n1,
                               int n2, int n3, int dtype, void* stream);

@@ -153,7 +153,7 @@ static int block_bwd(bool trans, const void* g, const void* image, const void* x
   // saved from the forward pass): for the block y = sum_p K_p(v) x(v + d_p) it is the scatter of
   // K_p(v) g(v), on the matrix cores with K neither stored nor streamed (igrad.hpp; the packed
   // weights lie before its sums in the K area), or on small grids and in FP16 and FP64 the
-  // transposed gather from stored K.  256^3 C = 1: FP32 835 -> 215 us, BF16 280 -> 181 us.  For
+  // transposed gather from stored K.  256^3 C = 1: FP32 835 -> 216 us, BF16 280 -> 180 us.  For
   // the transpose block it is the block apply itself, from K stored by the first product of the
   // fused apply on BF16 grids which that takes (matrix cores, an FP16 image copy).
   if (!trans && (dtype == kF32 || dtype == kBF16) && V >= kSplitMinVoxels && split_eligible(C, n1, n2, n3)) {

@@ -30,8 +30,8 @@ constexpr int kIgPlanes = 4;  // planes per tile, one per wave
 // Output rows per tile, R: the march computes R + 2 rows of K for R of dx, so long marches cost
 // less (256^3), but a small grid needs more workgroups than they leave (64^3: 64 of 16 rows).
 __host__ __device__ constexpr int ig_rows(int C) { return C == 1 ? 16 : 8; }
-// registers for this many waves per SIMD (C = 3 without its 68 bytes of scratch leaves one wave:
-// 128^3 82 us against 61)
+// registers for this many waves per SIMD (C = 3 without its 52 to 84 bytes of scratch leaves one
+// wave: 128^3 82 us against 63)
 __host__ __device__ constexpr int ig_waves(int C, int BB) { return C == 1 && BB == 1 ? 3 : 2; }
 
 constexpr unsigned kIgBlocks = 512;

@@ -34,9 +34,9 @@ constexpr long kFusedMinVoxels = 1L << 18;
 
 // FP32 blocks recompute K (split.hpp) on grids above this many voxels.  A 64^3 level's
 // stencils (28 MB) stay in the caches and their apply takes 7.4 us; at 96^3 they no longer do
-// (stored and recomputed: 64 x 64 x 72 11.9 and 10.3 us, 96^3 20.6 and 13.3 us, 128^3 40 and 18
-// us).  With two or three channels K costs two to three times as much and pays later (96^3 22.6
-// and 30.3 us, 112 x 96 x 128 26 and 34 us, 128^3 40 and 37 us, 256^3 351 and 258 us); mode 2
+// (stored and recomputed: 64 x 64 x 72 6.5 and 7.2 us, 96^3 20.8 and 11.8 us, 128^3 39 and 15
+// us).  With two or three channels K costs two to three times as much and pays later (96^3 22
+// and 26 us, 112 x 96 x 128 26 and 30 us, 128^3 40 and 35 us, 256^3 329 and 259 us); mode 2
 // takes it from 2^18 on too.
 constexpr long kSplitMinVoxels = 1L << 18;
 constexpr long kSplitChannelsMinVoxels = 1L << 21;

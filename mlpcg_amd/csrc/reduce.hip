@@ -808,8 +808,8 @@ int launch_weight_grad(int dtype, const void* a, const void* c, const void* img,
   int nb = nblk;
   if (dtype == kBF16 && B == 1 && n3 % wgb::kSeg == 0) {
     // whole 64-cell segments of one BF16 right-hand side: columns of J segments, about one
-    // column per wave, with ring staging (256^3 C = 1 142 us against 175 us of the tiles
-    // below, C = 3 242 against 590 us)
+    // column per wave, with ring staging (256^3 C = 1 134 to 157 us from box to box, C = 3 240
+    // to 250, against 190 and 480 us of the tiles below with FP32 data)
     const long segs = (long)n1 * n2 * (n3 / wgb::kSeg);
     const long per_wave = (segs + 4L * nblk - 1) / (4L * nblk);
     const int J = (int)(per_wave < 4 ? 4 : (per_wave > 64 ? 64 : per_wave));
